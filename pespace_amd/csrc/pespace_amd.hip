@@ -64,89 +64,129 @@ __device__ inline Cplx mode_factor(int id) {
 
 #ifndef PES_LNL_FWD_UNIT
 // ---- k_setup ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_setup(const double* __restrict__ params, int P, ModeList modes, double f_ref,
-                        double* __restrict__ setup, double* __restrict__ pconst, int* __restrict__ work_counter) {
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p == 0)  // work queues of the fused kernel launches that follow on this stream
-    for (int i = 0; i < N_WORK_COUNTERS; ++i) work_counter[i] = 0;
+// SETUP_ROWS rows per block.  The first wave computes the PhenomD/HM coefficients, four lanes per
+// row, each carrying one of the four parameter derivatives (a lane carrying all four held them in
+// 8.5 KB of scratch; with and without the gradient, so that both round alike).  The other two
+// waves compute the extrinsic constants meanwhile, a lane per (row, mode) and one for the
+// polarization vectors.  Bound by the latency of one lane's chain: 16 us for one row of one mode,
+// 24 us for 4096 of six modes (one lane per row: 52 and 126)
+constexpr int SETUP_ROWS = 16;
+struct RowParams {
+  double th[PES_N_PARAMS];
+  bool valid;
+};
+__device__ inline RowParams load_params(const double* __restrict__ params, int p) {
+  RowParams r;
+  r.valid = true;
+  for (int i = 0; i < PES_N_PARAMS; ++i) {
+    r.th[i] = params[(size_t)p * PES_N_PARAMS + i];
+    r.valid = r.valid && finite_d(r.th[i]);
+  }
+  r.valid = r.valid && r.th[0] > 0.0 && r.th[1] > 0.0 && r.th[1] <= 1.0 && fabs(r.th[2]) < 1.0 &&
+            fabs(r.th[3]) < 1.0 && r.th[4] > 0.0;
+  if (!r.valid) {  // harmless stand-in values; the row's lnL is set to -inf by k_reduce
+    constexpr double safe[PES_N_PARAMS] = {1.0e6, 1.0, 0.0, 0.0, 1.0e4, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int i = 0; i < PES_N_PARAMS; ++i) r.th[i] = safe[i];
+  }
+  return r;
+}
+
+__global__ __launch_bounds__(192) void k_setup(const double* __restrict__ params, int P, ModeList modes, double f_ref,
+                                               double* __restrict__ setup, double* __restrict__ pconst,
+                                               int* __restrict__ work_counter) {
+  if (blockIdx.x == 0) {
+    // work queues of the fused kernel launches that follow on this stream
+    for (int i = threadIdx.x; i < N_WORK_COUNTERS; i += blockDim.x) work_counter[i] = 0;
+  }
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (wave == 0) {
+    const int k = lane & 3;  // this lane's derivative
+    const int p = blockIdx.x * SETUP_ROWS + (lane >> 2);
+    if (p >= P) return;
+    const RowParams r = load_params(params, p);
+    typedef Dual<double, 1> D;
+    D in[4];
+    for (int i = 0; i < 4; ++i) {
+      in[i] = lift<D>(r.th[i]);
+      in[i].d[0] = i == k ? 1.0 : 0.0;
+    }
+    Phenom<D> ph;
+    phenom_setup(ph, in[0], in[1], in[2], in[3], f_ref);
+    double* su = setup + (size_t)p * N_SETUP * 5;
+#pragma unroll
+    for (int i = 0; i < N_SETUP; ++i) {
+      if (k == 0) su[i * 5] = ph.c[i].v;
+      su[i * 5 + 1 + k] = ph.c[i].d[0];
+    }
+    if (k != 0) return;
+    double* pc = pconst + (size_t)p * PC_STRIDE;
+    const double msec = value_of(ph.c[SU_MSEC]);
+    double fcut = 0.0;
+    for (int mi = 0; mi < modes.n; ++mi) {
+      const double cut = ph.mode_cut(modes.id[mi]) / msec;
+      pc[PC_MODE + mi * PC_MODE_STRIDE + MF_CUT] = cut;
+      fcut = fmax(fcut, cut);
+    }
+    pc[PC_FCUT] = fcut;
+    pc[PC_VALID] = r.valid ? 1.0 : 0.0;
+    pc[PC_OFFANY] = 0.0;  // set by k_duty_off
+    return;
+  }
+  const int idx = threadIdx.x - 64, mi = idx & 7, p = blockIdx.x * SETUP_ROWS + (idx >> 3);
   if (p >= P) return;
-  const double* th = params + (size_t)p * PES_N_PARAMS;
-  double Mc = th[0], q = th[1], c1 = th[2], c2 = th[3], dL = th[4], phi = th[5], iota = th[6];
-  double lam = th[7], bet = th[8], psi = th[9], tc = th[10];
-  bool valid = true;
-  for (int i = 0; i < PES_N_PARAMS; ++i) valid = valid && finite_d(th[i]);
-  valid = valid && Mc > 0.0 && q > 0.0 && q <= 1.0 && fabs(c1) < 1.0 && fabs(c2) < 1.0 && dL > 0.0;
+  const RowParams r = load_params(params, p);
   double* pc = pconst + (size_t)p * PC_STRIDE;
-  if (!valid) {  // harmless stand-in values; the row's lnL is set to -inf by k_reduce
-    Mc = 1.0e6; q = 1.0; c1 = 0.0; c2 = 0.0; dL = 1.0e4; phi = 0.0; iota = 0.0; lam = 0.0; bet = 0.0; psi = 0.0;
-    tc = 0.0;
+  const double dL = r.th[4], phi = r.th[5], iota = r.th[6], lam = r.th[7], bet = r.th[8], psi = r.th[9];
+  if (mi == 7) {  // at most six modes: the row's polarization basis and scalars
+    pc[PC_TC] = r.th[10];
+    pc[PC_DL] = dL;
+    pc[PC_INVDL] = 1.0 / dL;
+    double sl, cl, sb, cb, sp, cp;
+    sincos(lam, &sl, &cl);
+    sincos(bet, &sb, &cb);
+    sincos(psi, &sp, &cp);
+    // antenna.py:70-83, 112-114 and their lambda / beta derivatives
+    const double pv[3] = {sl * cp - cl * sb * sp, -cl * cp - sl * sb * sp, cb * sp};
+    const double qv[3] = {-sl * sp - cl * sb * cp, cl * sp - sl * sb * cp, cb * cp};
+    const double kv[3] = {-cb * cl, -cb * sl, -sb};
+    const double dlp[3] = {cl * cp + sl * sb * sp, sl * cp - cl * sb * sp, 0.0};
+    const double dbp[3] = {-cl * cb * sp, -sl * cb * sp, -sb * sp};
+    const double dlq[3] = {-cl * sp + sl * sb * cp, -sl * sp - cl * sb * cp, 0.0};
+    const double dbq[3] = {-cl * cb * cp, -sl * cb * cp, -sb * cp};
+    const double dlk[3] = {cb * sl, -cb * cl, 0.0};
+    const double dbk[3] = {sb * cl, sb * sl, -cb};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      pc[PC_P + i] = pv[i]; pc[PC_Q + i] = qv[i]; pc[PC_K + i] = kv[i];
+      pc[PC_DLP + i] = dlp[i]; pc[PC_DLQ + i] = dlq[i]; pc[PC_DBP + i] = dbp[i];
+      pc[PC_DBQ + i] = dbq[i]; pc[PC_DLK + i] = dlk[i]; pc[PC_DBK + i] = dbk[i];
+    }
+    return;
   }
-  typedef Dual<double, 4> D4;
-  D4 dMc = lift<D4>(Mc), dq = lift<D4>(q), dc1 = lift<D4>(c1), dc2 = lift<D4>(c2);
-  dMc.d[0] = 1.0; dq.d[1] = 1.0; dc1.d[2] = 1.0; dc2.d[3] = 1.0;
-  Phenom<D4> ph;
-  phenom_setup(ph, dMc, dq, dc1, dc2, f_ref);
-  double* su = setup + (size_t)p * N_SETUP * 5;
-  for (int i = 0; i < N_SETUP; ++i) {
-    su[i * 5 + 0] = ph.c[i].v;
-    for (int k = 0; k < 4; ++k) su[i * 5 + 1 + k] = ph.c[i].d[k];
-  }
-  pc[PC_TC] = tc;
-  pc[PC_DL] = dL;
-  pc[PC_INVDL] = 1.0 / dL;
-  pc[PC_VALID] = valid ? 1.0 : 0.0;
-  pc[PC_OFFANY] = 0.0;  // set by k_duty_off
-  double sl, cl, sb, cb, sp, cp;
-  sincos(lam, &sl, &cl);
-  sincos(bet, &sb, &cb);
-  sincos(psi, &sp, &cp);
-  // antenna.py:70-83, 112-114 and their lambda / beta derivatives
-  double pv[3] = {sl * cp - cl * sb * sp, -cl * cp - sl * sb * sp, cb * sp};
-  double qv[3] = {-sl * sp - cl * sb * cp, cl * sp - sl * sb * cp, cb * cp};
-  double kv[3] = {-cb * cl, -cb * sl, -sb};
-  double dlp[3] = {cl * cp + sl * sb * sp, sl * cp - cl * sb * sp, 0.0};
-  double dbp[3] = {-cl * cb * sp, -sl * cb * sp, -sb * sp};
-  double dlq[3] = {-cl * sp + sl * sb * cp, -sl * sp - cl * sb * cp, 0.0};
-  double dbq[3] = {-cl * cb * cp, -sl * cb * cp, -sb * cp};
-  double dlk[3] = {cb * sl, -cb * cl, 0.0};
-  double dbk[3] = {sb * cl, sb * sl, -cb};
-  for (int i = 0; i < 3; ++i) {
-    pc[PC_P + i] = pv[i]; pc[PC_Q + i] = qv[i]; pc[PC_K + i] = kv[i];
-    pc[PC_DLP + i] = dlp[i]; pc[PC_DLQ + i] = dlq[i]; pc[PC_DBP + i] = dbp[i];
-    pc[PC_DBQ + i] = dbq[i]; pc[PC_DLK + i] = dlk[i]; pc[PC_DBK + i] = dbk[i];
-  }
-  double dist = dL * 1.0e6 * PC_SI;
-  double msec = ph.c[SU_MSEC].v;
-  double az = 0.5 * PI - phi;  // lalsimulation azimuth convention
+  if (mi >= modes.n) return;
+  const double dist = dL * 1.0e6 * PC_SI;
+  const double az = 0.5 * PI - phi;  // lalsimulation azimuth convention
   typedef Dual<double, 1> D1;
   D1 di = lift<D1>(iota);
   di.d[0] = 1.0;
-  double fcut = 0.0;
-  for (int mi = 0; mi < modes.n; ++mi) {
-    int id = modes.id[mi];
-    int l = kModeL[id], m = kModeM[id];
-    D1 y = sw_y(l, m, di);
-    D1 ym = sw_y(l, -m, di);
-    double sgn = (l % 2) ? -1.0 : 1.0;
-    double se, ce;
-    sincos(-(double)m * az, &se, &ce);
-    Cplx e = {ce, se};
-    Cplx u = mode_factor(id);
-    Cplx eu = cmul(e, u);
-    double kp = 0.5 * (y.v + sgn * ym.v), dkp = 0.5 * (y.d[0] + sgn * ym.d[0]);
-    double kc = 0.5 * (sgn * ym.v - y.v), dkc = 0.5 * (sgn * ym.d[0] - y.d[0]);  // times i
-    double* mf = pc + PC_MODE + mi * PC_MODE_STRIDE;
-    Cplx Fp = cscale(eu, kp / dist);
-    // the cross factor is stored doubled: the link term's n.e_x.n = 2 (n.p)(n.q) keeps its 2 there
-    Cplx Fc = cmul({0.0, 2.0 * kc / dist}, eu);
-    Cplx dFp = cscale(eu, dkp / dist);
-    Cplx dFc = cmul({0.0, 2.0 * dkc / dist}, eu);
-    mf[MF_FPR] = Fp.re; mf[MF_FPI] = Fp.im; mf[MF_FCR] = Fc.re; mf[MF_FCI] = Fc.im;
-    mf[MF_CUT] = ph.mode_cut(id) / msec;
-    fcut = fmax(fcut, mf[MF_CUT]);
-    mf[MF_DFPR] = dFp.re; mf[MF_DFPI] = dFp.im; mf[MF_DFCR] = dFc.re; mf[MF_DFCI] = dFc.im;
-  }
-  pc[PC_FCUT] = fcut;
+  const int id = modes.id[mi];
+  const int l = kModeL[id], m = kModeM[id];
+  const D1 y = sw_y(l, m, di);
+  const D1 ym = sw_y(l, -m, di);
+  const double sgn = (l % 2) ? -1.0 : 1.0;
+  double se, ce;
+  sincos(-(double)m * az, &se, &ce);
+  const Cplx eu = cmul({ce, se}, mode_factor(id));
+  const double kp = 0.5 * (y.v + sgn * ym.v), dkp = 0.5 * (y.d[0] + sgn * ym.d[0]);
+  const double kc = 0.5 * (sgn * ym.v - y.v), dkc = 0.5 * (sgn * ym.d[0] - y.d[0]);  // times i
+  double* mf = pc + PC_MODE + mi * PC_MODE_STRIDE;
+  const Cplx Fp = cscale(eu, kp / dist);
+  // the cross factor is stored doubled: the link term's n.e_x.n = 2 (n.p)(n.q) keeps its 2 there
+  const Cplx Fc = cmul({0.0, 2.0 * kc / dist}, eu);
+  const Cplx dFp = cscale(eu, dkp / dist);
+  const Cplx dFc = cmul({0.0, 2.0 * dkc / dist}, eu);
+  mf[MF_FPR] = Fp.re; mf[MF_FPI] = Fp.im; mf[MF_FCR] = Fc.re; mf[MF_FCI] = Fc.im;
+  mf[MF_DFPR] = dFp.re; mf[MF_DFPI] = dFp.im; mf[MF_DFCR] = dFc.re; mf[MF_DFCI] = dFc.im;
 }
 
 // ---- k_nodes ---------------------------------------------------------------------------
@@ -1498,8 +1538,8 @@ static int check_batch_args(const pes_context* ctx, const double* d_params, int 
 // k_setup (which also zeroes the work counters) and k_nodes for P >= 1 rows
 static int launch_setup_nodes(const pes_context* ctx, const BatchScratch& sc, const double* d_params, int P, bool grad,
                               hipStream_t st) {
-  hipLaunchKernelGGL(k_setup, dim3((P + 63) / 64), dim3(64), 0, st, d_params, P, ctx->modes, ctx->f_ref, sc.setup,
-                     sc.pconst, sc.work_counter);
+  hipLaunchKernelGGL(k_setup, dim3((P + SETUP_ROWS - 1) / SETUP_ROWS), dim3(192), 0, st, d_params, P, ctx->modes,
+                     ctx->f_ref, sc.setup, sc.pconst, sc.work_counter);
   HIP_TRY(hipGetLastError());
   const int NNS = ctx->n_nodes + 1;
   dim3 g((NNS + 127) / 128, P * ctx->modes.n);

@@ -333,31 +333,27 @@ PES_HD S radiated_energy(const S& eta, const S& d, const S& chi1, const S& chi2)
          (1.0 + (-0.6714403054720589 - 1.4756929437702908 * eta + 7.304676214885011 * e2) * s);
 }
 
-// Gaussian elimination with partial pivoting (by value) on a 5x5 system.
+// Monomial coefficients x[0..4] of the quartic with value and slope (v1, d1) at f1, value v2 at f2
+// and (v3, d3) at f3: divided differences on f1, f1, f2, f3, f3, then the Newton form expanded.  No
+// elimination: a pivoting solve indexes its matrix at run time, which puts it in scratch memory
+// (k_setup, one row: half of its time)
 template <class S>
-PES_HD void solve5(S a[5][5], S b[5], S x[5]) {
-  for (int k = 0; k < 5; ++k) {
-    int piv = k;
-    double best = fabs(value_of(a[k][k]));
-    for (int r = k + 1; r < 5; ++r) {
-      double v = fabs(value_of(a[r][k]));
-      if (v > best) { best = v; piv = r; }
-    }
-    if (piv != k) {
-      for (int cc = 0; cc < 5; ++cc) { S t = a[k][cc]; a[k][cc] = a[piv][cc]; a[piv][cc] = t; }
-      S t = b[k]; b[k] = b[piv]; b[piv] = t;
-    }
-    for (int r = k + 1; r < 5; ++r) {
-      S fct = a[r][k] / a[k][k];
-      for (int cc = k; cc < 5; ++cc) a[r][cc] = a[r][cc] - fct * a[k][cc];
-      b[r] = b[r] - fct * b[k];
-    }
-  }
-  for (int k = 4; k >= 0; --k) {
-    S acc = b[k];
-    for (int cc = k + 1; cc < 5; ++cc) acc = acc - a[k][cc] * x[cc];
-    x[k] = acc / a[k][k];
-  }
+PES_HD void hermite_quartic(const S& f1, const S& v1, const S& d1, const S& f2, const S& v2, const S& f3, const S& v3,
+                            const S& d3, S x[5]) {
+  const S h12 = f2 - f1, h13 = f3 - f1, h23 = f3 - f2;
+  const S a12 = (v2 - v1) / h12, a23 = (v3 - v2) / h23;
+  const S b1 = (a12 - d1) / h12, b2 = (a23 - a12) / h13, b3 = (d3 - a23) / h23;
+  const S c1 = (b2 - b1) / h13, c2 = (b3 - b2) / h13;
+  const S e = (c2 - c1) / h13;
+  // v1 + (f - f1)(d1 + (f - f1)(b1 + (f - f2)(c1 + (f - f3) e)))
+  S p0 = c1 - f3 * e, p1 = e;                          // c1 + (f - f3) e
+  S q0 = b1 - f2 * p0, q1 = p0 - f2 * p1, q2 = p1;     // b1 + (f - f2) p
+  S r0 = d1 - f1 * q0, r1 = q0 - f1 * q1, r2 = q1 - f1 * q2, r3 = q2;
+  x[0] = v1 - f1 * r0;
+  x[1] = r0 - f1 * r1;
+  x[2] = r1 - f1 * r2;
+  x[3] = r2 - f1 * r3;
+  x[4] = r3;
 }
 
 // Build all setup coefficients from (Mc [Msun], q = m2/m1 <= 1, chi1, chi2) and f_ref [Hz].
@@ -381,6 +377,7 @@ PES_HD void phenom_setup(Phenom<S>& P, const S& Mc, const S& q, const S& chi1_in
   S chis = 0.5 * (chi1 + chi2), chia = 0.5 * (chi1 - chi2);
   S chipn = chis * (1.0 - 76.0 * eta / 113.0) + delta * chia;
   S* c = P.c;
+#pragma unroll
   for (int i = 0; i < N_SETUP; ++i) c[i] = lift<S>(0.0);
   c[SU_MSEC] = M * MTSUN_SI;
   c[SU_AMPSCALE] = (M * MRSUN_SI) * (M * MTSUN_SI);
@@ -501,6 +498,7 @@ PES_HD void phenom_setup(Phenom<S>& P, const S& Mc, const S& q, const S& chi1_in
     S f2 = 0.5 * (f1 + f3);
     // promote coefficients to SF is avoided: evaluate ansatz and derivative by hand
     Phenom<SF> Q;
+#pragma unroll
     for (int i = 0; i < N_SETUP; ++i) {
       Q.c[i].v = c[i];
       Q.c[i].d[0] = lift<S>(0.0);
@@ -513,20 +511,8 @@ PES_HD void phenom_setup(Phenom<S>& P, const S& Mc, const S& q, const S& chi1_in
     x3.v = f3;
     x3.d[0] = lift<S>(1.0);
     SF mrd = Q.amp_mrd(x3);
-    S A[5][5], b[5], x[5];
-    S f1s = lift<S>(f1);
-    S pw1[5], pw2[5], pw3[5];
-    pw1[0] = lift<S>(1.0); pw2[0] = lift<S>(1.0); pw3[0] = lift<S>(1.0);
-    for (int k = 1; k < 5; ++k) { pw1[k] = pw1[k - 1] * f1s; pw2[k] = pw2[k - 1] * f2; pw3[k] = pw3[k - 1] * f3; }
-    for (int k = 0; k < 5; ++k) {
-      A[0][k] = pw1[k];
-      A[1][k] = k == 0 ? lift<S>(0.0) : (double)k * pw1[k - 1];
-      A[2][k] = pw2[k];
-      A[3][k] = pw3[k];
-      A[4][k] = k == 0 ? lift<S>(0.0) : (double)k * pw3[k - 1];
-    }
-    b[0] = ins.v; b[1] = ins.d[0]; b[2] = v2; b[3] = mrd.v; b[4] = mrd.d[0];
-    solve5(A, b, x);
+    S x[5];
+    hermite_quartic(lift<S>(f1), ins.v, ins.d[0], f2, v2, f3, mrd.v, mrd.d[0], x);
     c[SU_D0] = x[0]; c[SU_D1] = x[1]; c[SU_D2] = x[2]; c[SU_D3] = x[3]; c[SU_D4] = x[4];
   }
   // phase C1 connection
@@ -535,6 +521,7 @@ PES_HD void phenom_setup(Phenom<S>& P, const S& Mc, const S& q, const S& chi1_in
     Phenom<SF> Q;
     c[SU_C1INT] = c[SU_C2INT] = c[SU_C1MRD] = c[SU_C2MRD] = lift<S>(0.0);
     c[SU_T0] = c[SU_PHIREF0] = c[SU_MFREF] = lift<S>(0.0);
+#pragma unroll
     for (int i = 0; i < N_SETUP; ++i) {
       Q.c[i].v = c[i];
       Q.c[i].d[0] = lift<S>(0.0);
