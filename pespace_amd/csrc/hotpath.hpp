@@ -747,7 +747,9 @@ __device__ inline void stage_nodes_dma(const double* __restrict__ nodes, const d
 // finished the previous row, the last reader of the buffer the copy for the next row goes to.
 // Without STAGED each lane reads its node rows from global memory (tiles whose node range is
 // wider, e.g. the lowest frequencies of short data).
-template <int PREC, bool GRAD, int KIND, bool STAGED>
+// PAN: the context has panels and dbits marks the rows of a tile with panels that come here (null: a
+// tile without panels)
+template <int PREC, bool GRAD, int KIND, bool STAGED, bool PAN>
 __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, int p0, int p1,
                                  const double* __restrict__ bin_f, const int* __restrict__ bin_j,
                                  const double* __restrict__ bin_s, const double* __restrict__ bin_rec,
@@ -755,7 +757,8 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
                                  const double* __restrict__ nodes, const double* __restrict__ nodes_grad, int NNS,
                                  double du, const ModeList& modes, int lane, int wave, double* acc, int j0,
                                  int nj, double* stage_n, double* stage_g, int& buf,
-                                 const unsigned long long* __restrict__ off_bits, int n_tiles, double* lane_lds) {
+                                 const unsigned long long* __restrict__ off_bits, int n_tiles, double* lane_lds,
+                                 const unsigned long long* __restrict__ dbits) {
   constexpr int NOUT = GRAD ? 1 + PES_N_PARAMS : 1;
   const int bi = tile * TILE + threadIdx.x;
   // a duty-cycled detector's tile whose window is zero for every mode of row p throughout
@@ -769,6 +772,16 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
       return ((off_bits[w] >> (tile & 63)) & 1ull) != 0;
     } else {
       return false;
+    }
+  };
+  // a tile with panels: only the rows that k_panel_class left to this kernel
+  auto row_mine = [&](int p) -> bool {
+    if constexpr (PAN) {
+      if (!dbits) return true;
+      const size_t w = (size_t)__builtin_amdgcn_readfirstlane(p) * ((n_tiles + 63) >> 6) + (tile >> 6);
+      return ((dbits[w] >> (tile & 63)) & 1ull) != 0;
+    } else {
+      return true;
     }
   };
   BinPre b;
@@ -792,12 +805,13 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
   constexpr int SN = MAX_MODES * NJ_STAGE * 4, SG = MAX_MODES * NJ_STAGE * 16;  // doubles per buffer
   if constexpr (STAGED) {  // copy for the first evaluated row
     int q = p0;
-    while (q < p1 && !(row_live(pconst, q, f0) && !tile_off(q))) ++q;
+    while (q < p1 && !(row_mine(q) && row_live(pconst, q, f0) && !tile_off(q))) ++q;
     if (q < p1)
       stage_nodes_dma<GRAD>(nodes, nodes_grad, (size_t)q * modes.n * NNS + j0, NNS, modes.n, nj, stage_n + buf * SN,
                             stage_g + buf * SG, lane, wave);
   }
   for (int p = p0; p < p1; ++p) {
+    if (!row_mine(p)) continue;
     const double* pc = pconst + (size_t)p * PC_STRIDE;
     if (f0 > pc[PC_FCUT] || tile_off(p)) {
       if (threadIdx.x == 0) acc[(p - p0) * NOUT] -= tile_dd[tile];
@@ -834,7 +848,7 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
       size_t nstride, gstride;
       if constexpr (STAGED) {
         int qn = p + 1;  // next evaluated row
-        while (qn < p1 && !(row_live(pconst, qn, f0) && !tile_off(qn))) ++qn;
+        while (qn < p1 && !(row_mine(qn) && row_live(pconst, qn, f0) && !tile_off(qn))) ++qn;
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's copies for row p are in LDS
         __syncthreads();                     // ... and every wave's; all waves are past row p - 1
         if constexpr (kRecEarly) load_rec();
@@ -949,7 +963,7 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
 }
 
 // ------------------------------- kernels ---------------------------------------------------
-// Persistent fused kernel.  Work item = (group of tiles_per_group tiles, chunk of
+// Persistent fused kernel.  Work item = (group of tiles, chunk of
 // chunk_rows<GRAD>() rows);
 // lane <-> bin.  A tile whose first frequency lies above every mode's cut of a row has a
 // zero response for that row: its lnL contribution is the precomputed -sum w |d|^2 of the
@@ -962,19 +976,23 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
 // holds that one variant's code (a kernel holding both orbit kinds spilled 106 instead of 59-74
 // VGPRs).  items (duty-cycled ranges only; null otherwise): the work items of the range that the
 // plain instantiation takes (1) and those the duty one takes (0).
-template <int PREC, bool GRAD, int KD>
+// PAN: the context has panels: this kernel takes the tiles and rows that they leave, and adds to
+// the panel kernel's sums
+template <int PREC, bool GRAD, int KD, bool PAN>
 __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* __restrict__ dets, int n_det, int n_tiles,
                                               const double* __restrict__ bin_f, const int* __restrict__ bin_j,
                                               const double* __restrict__ bin_s, const double* __restrict__ bin_rec,
                                               const double* __restrict__ tile_f0, const double* __restrict__ tile_dd,
-                                              int tiles_per_group, const double* __restrict__ pconst,
+                                              const int* __restrict__ grp, int n_grp, const double* __restrict__ pconst,
                                               const double* __restrict__ nodes,
                                               const double* __restrict__ nodes_grad, int NNS, double du,
                                               ModeList modes, int P, int rows, const int* __restrict__ tile_jr,
-                                              int tile_begin, int tile_end, int group_offset,
+                                              int tile_begin, int group_offset,
                                               int* __restrict__ work_counter, double* __restrict__ partial,
                                               const unsigned long long* __restrict__ off_bits,
-                                              const unsigned char* __restrict__ items) {
+                                              const unsigned char* __restrict__ items,
+                                              const int* __restrict__ tile_pan, BinWork bw, int range, int list_base,
+                                              const unsigned long long* __restrict__ dbits, int fine) {
   constexpr int NOUT = GRAD ? 1 + PES_N_PARAMS : 1;
   constexpr int CH = chunk_rows<GRAD>();  // 4x the rows without the gradient: 1.3% faster
   __shared__ double acc[TILE / 64][CH][NOUT];
@@ -991,13 +1009,14 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
   // there, 0.2% slower with the gradient
   const int lane = threadIdx.x & 63;
   const int wave = GRAD ? (int)(threadIdx.x >> 6) : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // rows (1 <= rows <= CH) per work item, chosen by the host.  This launch covers the tiles
-  // [tile_begin, tile_end) in groups of tiles_per_group, whose partial sums go to groups
-  // group_offset + 0, 1, ...: one launch (and counter) per tile range of one orbit kind and duty
-  // flag, two for a duty-cycled range
+  // rows (1 <= rows <= CH) per work item, chosen by the host.  This launch covers the n_grp groups
+  // of a tile range (group gl: tiles grp[gl] .. grp[gl + 1] - 1; grp null: the one tile
+  // tile_begin + gl), whose partial sums go to groups group_offset + 0, 1, ...: one launch (and
+  // counter) per tile range of one orbit kind and duty flag, two for a duty-cycled range
   const int n_chunks = (P + rows - 1) / rows;
-  const int n_groups_r = (tile_end - tile_begin + tiles_per_group - 1) / tiles_per_group;
-  const int n_work = n_chunks * n_groups_r;
+  // with panels only the groups of the batch's list have work left here
+  const int n_work = n_chunks * (PAN ? bw.state[1 + range] : n_grp);
+  const int epoch = PAN ? bw.state[0] : 0;
   constexpr bool DUTY = kDuty<KD>;
   // the duty pass of a range whose items all run in the plain one: k_duty_items counted none at
   // work_counter[MAX_TILE_RANGES] (every block leaves before its first barrier)
@@ -1010,7 +1029,8 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
     __syncthreads();
     const int w = next_work;
     if (w >= n_work) break;
-    const int gl = w / n_chunks, c = w % n_chunks;
+    const int gi = w / n_chunks, c = w % n_chunks;
+    const int gl = PAN ? bw.list[list_base + gi] : gi;
     const int g = group_offset + gl;
     // a duty-cycled range runs twice: items on the window's plateau (items[] = 1, k_duty_items)
     // here in the plain instantiation, the others in the duty one; each writes only its own
@@ -1020,13 +1040,18 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
       continue;
     }
     const int p0 = c * rows, p1 = min(P, p0 + rows);
+    const int t_first = grp ? grp[gl] : tile_begin + gl, t_end = grp ? grp[gl + 1] : t_first + 1;
     for (int i = threadIdx.x; i < (TILE / 64) * CH * NOUT; i += TILE) (&acc[0][0][0])[i] = 0.0;
     double chunk_cut = 0.0;
     for (int p = p0; p < p1; ++p) chunk_cut = fmax(chunk_cut, pconst[(size_t)p * PC_STRIDE + PC_FCUT]);
     __syncthreads();
-    const int t_first = tile_begin + gl * tiles_per_group;
-    const int t_end = min(tile_end, t_first + tiles_per_group);
     for (int tile = t_first; tile < t_end; ++tile) {
+      const unsigned long long* db = nullptr;
+      if constexpr (PAN) {
+        // a tile with panels: the panel kernel has it, apart from the rows marked in dbits
+        db = tile_pan[2 * tile + 1] > 0 ? dbits : nullptr;
+        if (db && (bw.tile_any[tile] != epoch || tile_f0[tile] > chunk_cut)) continue;
+      }
       const double f0 = tile_f0[tile];
       if (f0 > chunk_cut) {  // no row of the chunk has a mode up here
         if (threadIdx.x == 0) {
@@ -1039,21 +1064,27 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
       const int j0 = tile_jr[2 * tile], nj = tile_jr[2 * tile + 1];
 #define PES_TILE_ARGS                                                                                         \
   det, tile, f0, p0, p1, bin_f, bin_j, bin_s, bin_rec, tile_dd, pconst, nodes, nodes_grad, NNS, du, \
-      modes, lane, wave, &acc[0][0][0], j0, nj, stage_n, &stage_g[0], buf, off_bits, n_tiles, &lane_lds[0]
+      modes, lane, wave, &acc[0][0][0], j0, nj, stage_n, &stage_g[0], buf, off_bits, n_tiles, &lane_lds[0], db
       // the host's tile ranges give this launch detectors of one orbit kind (KD bit 0), all
       // duty-cycled or none (bit 1)
       if (nj <= NJ_STAGE)
-        tile_rows<PREC, GRAD, KD, true>(PES_TILE_ARGS);
+        tile_rows<PREC, GRAD, KD, true, PAN>(PES_TILE_ARGS);
       else
-        tile_rows<PREC, GRAD, KD, false>(PES_TILE_ARGS);
+        tile_rows<PREC, GRAD, KD, false, PAN>(PES_TILE_ARGS);
 #undef PES_TILE_ARGS
     }
     __syncthreads();
     for (int i = threadIdx.x; i < (p1 - p0) * NOUT; i += TILE) {
       const int pl = i / NOUT, o = i % NOUT;
+      if (fine) {  // one tile per item: the waves' sums (k_group_sums adds them as below)
+        for (int k = 0; k < TILE / 64; ++k)
+          partial[(((size_t)g * (TILE / 64) + k) * NOUT + o) * P + p0 + pl] = acc[k][pl][o];
+        continue;
+      }
       double s = 0.0;
       for (int k = 0; k < TILE / 64; ++k) s += acc[k][pl][o];
-      partial[((size_t)g * NOUT + o) * P + p0 + pl] = s;
+      double* ps = partial + ((size_t)g * NOUT + o) * P + p0 + pl;
+      *ps = PAN ? *ps + s : s;
     }
     __syncthreads();
   }

@@ -23,7 +23,8 @@ constexpr int MAX_TILE_RANGES = 16;  // runs of detectors by duty flag per conte
 // fused-kernel launches per batch: one per range, and a second for a duty-cycled range (its work
 // items on the window's plateau run in the plain instantiation), each with its own work counter;
 // a third set counts a duty-cycled range's items that need the window (k_duty_items)
-constexpr int N_WORK_COUNTERS = 3 * MAX_TILE_RANGES;
+// and a fourth serves the panel kernel's launches
+constexpr int N_WORK_COUNTERS = 4 * MAX_TILE_RANGES;
 
 // ---- per-row constant block ------------------------------------------------------------
 enum PConst {

@@ -5,9 +5,11 @@
 //               the extrinsic constants (polarization basis, harmonic factors)
 //   k_nodes     one thread per (row, mode, node): A, dA/du, Psi, dPsi/du on the
 //               log-spaced interpolation nodes (u = ln f)
-//   k_lnl_*     persistent fused kernel: lane <-> frequency bin, loop over the rows
-//               of a chunk; cubic-Hermite node -> bin interpolation, t_c shift,
-//               orbit, six single links, TDI, residual, FP64 reduction
+//   k_panel_class, k_lnl_panel  (long grids) lnL and gradient from short polynomials of the
+//               response's smooth part (panel.hpp)
+//   k_lnl_*     persistent fused kernel, every bin of the tiles that have no panels: lane <->
+//               frequency bin, loop over the rows of a chunk; cubic-Hermite node -> bin
+//               interpolation, t_c shift, orbit, six single links, TDI, residual, FP64 reduction
 //   k_reduce    fixed-order sum of the per-(bin group, row) partials
 #include <hip/hip_runtime.h>
 
@@ -93,10 +95,16 @@ __device__ inline RowParams load_params(const double* __restrict__ params, int p
 
 __global__ __launch_bounds__(192) void k_setup(const double* __restrict__ params, int P, ModeList modes, double f_ref,
                                                double* __restrict__ setup, double* __restrict__ pconst,
-                                               int* __restrict__ work_counter) {
+                                               int* __restrict__ work_counter, int* __restrict__ bin_state) {
   if (blockIdx.x == 0) {
     // work queues of the fused kernel launches that follow on this stream
     for (int i = threadIdx.x; i < N_WORK_COUNTERS; i += blockDim.x) work_counter[i] = 0;
+    if (bin_state && threadIdx.x <= MAX_TILE_RANGES) {  // BinWork: the batch's number, empty lists
+      if (threadIdx.x == 0)
+        ++bin_state[0];
+      else
+        bin_state[threadIdx.x] = 0;
+    }
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (wave == 0) {
@@ -288,33 +296,87 @@ struct BinData {
 };
 
 #include "hotpath.hpp"
+#ifndef PES_LNL_FWD_UNIT
+#include "panel.hpp"
+#endif
 
 #ifndef PES_LNL_FWD_UNIT
-// One block per (64 rows, output): each of the 4 waves sums every 4th bin group in order, then
-// the four wave sums are added in a fixed order, so results do not depend on scheduling.
-constexpr int REDUCE_WAVES = 4;  // the final sum below adds exactly four wave sums
-__global__ __launch_bounds__(64 * REDUCE_WAVES) void k_reduce(const double* __restrict__ partial, int n_groups, int P,
-                                                           int nout, const double* __restrict__ pconst,
-                                                           double* __restrict__ lnl, double* __restrict__ grad) {
-  __shared__ double part[REDUCE_WAVES][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int p = blockIdx.x * 64 + lane;
+// Sum of the group partials of every (row, output): 64 chains (every 64th group, in order), then a
+// tree over the chains: an order that depends on neither the batch nor the scheduling.  RB rows per
+// block (fewer rows, more threads per row: one row of short data 5.8 -> 1.8 us), 256 threads.
+constexpr int REDUCE_CHAINS = 64;
+template <int RB>
+__global__ __launch_bounds__(256) void k_reduce(const double* __restrict__ partial, int n_groups, int P, int nout,
+                                                const double* __restrict__ pconst, double* __restrict__ lnl,
+                                                double* __restrict__ grad) {
+  constexpr int SLOTS = 256 / RB, PER = REDUCE_CHAINS / SLOTS;
+  __shared__ double part[REDUCE_CHAINS][RB];
+  const int r = threadIdx.x % RB, slot = threadIdx.x / RB;
+  const int p = blockIdx.x * RB + r;
   const int o = blockIdx.y;
-  double s = 0.0;
-  if (p < P) {
+#pragma unroll
+  for (int c = 0; c < PER; ++c) {
+    const int k = slot + c * SLOTS;
+    double s = 0.0;
+    if (p < P) {
 #pragma unroll 8
-    for (int g = w; g < n_groups; g += REDUCE_WAVES) s += partial[((size_t)g * nout + o) * P + p];
+      for (int g = k; g < n_groups; g += REDUCE_CHAINS) s += partial[((size_t)g * nout + o) * P + p];
+    }
+    part[k][r] = s;
   }
-  part[w][lane] = s;
   __syncthreads();
-  if (w == 0 && p < P) {
-    const double t = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+#pragma unroll
+  for (int h = REDUCE_CHAINS / 2; h > 0; h >>= 1) {
+    for (int k = slot; k < h; k += SLOTS) part[k][r] += part[k + h][r];
+    __syncthreads();
+  }
+  if (slot == 0 && p < P) {
+    const double t = part[0][r];
     const bool valid = pconst[(size_t)p * PC_STRIDE + PC_VALID] != 0.0;
     if (o == 0)
       lnl[p] = valid ? t : -INFINITY;
     else if (grad)
       grad[(size_t)p * PES_N_PARAMS + (o - 1)] = valid ? t : 0.0;
   }
+}
+
+// Small batches run one tile (panel kernel: one panel) per work item, so that they fill the chip;
+// their sums (fine_pan: per panel; fine_bin: per tile of the four waves of the bin-by-bin kernel) are put
+// together here in the order in which an item of a whole group adds them, so that a row's
+// result does not depend on its batch.  One thread per (group, output, row).
+__global__ __launch_bounds__(256) void k_group_sums(const int* __restrict__ grp, int n_groups, int P, int nout,
+                                                    const double* __restrict__ fine_pan,
+                                                    const double* __restrict__ fine_bin,
+                                                    const int* __restrict__ tile_pan, BinWork bw,
+                                                    double* __restrict__ partial) {
+  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (size_t)n_groups * nout * P) return;
+  const int p = (int)(idx % P), o = (int)(idx / P % nout), g = (int)(idx / ((size_t)P * nout));
+  const int t0 = grp[g], t1 = grp[g + 1];
+  double a = 0.0, d[TILE / 64];
+  bool any = !fine_pan;
+#pragma unroll
+  for (int w = 0; w < TILE / 64; ++w) d[w] = 0.0;
+  for (int t = t0; t < t1; ++t) {
+    if (fine_pan) {
+      const int q0 = tile_pan[2 * t], q1 = q0 + tile_pan[2 * t + 1];
+      double s = 0.0;
+      for (int q = q0; q < q1; ++q) s += fine_pan[((size_t)q * nout + o) * P + p];
+      a += s;
+    }
+    if (!fine_pan || bw.tile_any[t] == bw.state[0]) {
+      any = true;
+#pragma unroll
+      for (int w = 0; w < TILE / 64; ++w) d[w] += fine_bin[(((size_t)t * (TILE / 64) + w) * nout + o) * P + p];
+    }
+  }
+  if (any) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < TILE / 64; ++w) s += d[w];
+    a = fine_pan ? a + s : s;
+  }
+  partial[((size_t)g * nout + o) * P + p] = a;
 }
 
 // ---- work accounting for the profiler: per row, the number of (bin, mode) pairs below the
@@ -431,11 +493,12 @@ __global__ __launch_bounds__(64) void k_duty_items(const DetectorDev* __restrict
                                                    const double* __restrict__ tile_f0, const int* __restrict__ tile_jr,
                                                    const double* __restrict__ pconst, const double* __restrict__ nodes,
                                                    int NNS, double u0, double du, ModeList modes, int P, int rows,
-                                                   int n_chunks, int tile_begin, int tile_end, int tiles_per_group,
+                                                   int n_chunks, int tile_begin, const int* __restrict__ grp,
                                                    int group_offset, int enable, unsigned char* __restrict__ items,
-                                                   int* __restrict__ n_duty_items) {
+                                                   int* __restrict__ n_duty_items, int words,
+                                                   const unsigned long long* __restrict__ dbits) {
   const int gl = blockIdx.x / n_chunks, c = blockIdx.x % n_chunks;
-  const int t_first = tile_begin + gl * tiles_per_group, t_end = min(tile_end, t_first + tiles_per_group);
+  const int t_first = grp ? grp[gl] : tile_begin + gl, t_end = grp ? grp[gl + 1] : t_first + 1;
   const int p0 = c * rows, p1 = min(P, p0 + rows);
   const int nt = t_end - t_first, np = p1 - p0;
   int ok = enable;
@@ -444,6 +507,7 @@ __global__ __launch_bounds__(64) void k_duty_items(const DetectorDev* __restrict
     const double* pc = pconst + (size_t)p * PC_STRIDE;
     const double f0 = tile_f0[tile];
     if (pc[PC_VALID] == 0.0 || f0 > pc[PC_FCUT]) continue;
+    if (dbits && ((dbits[(size_t)p * words + (tile >> 6)] >> (tile & 63)) & 1ull) == 0) continue;  // in panels
     const DetectorDev& det = dets[tile_detector(dets, n_det, tile)];
     const int j0 = tile_jr[2 * tile], j1 = j0 + tile_jr[2 * tile + 1];
     const double tc = pc[PC_TC];
@@ -999,14 +1063,15 @@ __global__ void k_whittle_final(const double* __restrict__ work, int nb, double 
 #define PES_LNL_PARAMS                                                                                       \
   const DetectorDev *dets, int n_det, int n_tiles, const double *bin_f, const int *bin_j, const double *bin_s, \
       const double *bin_rec, const double *tile_f0,                                                       \
-      const double *tile_dd, int tiles_per_group, const double *pconst, const double *nodes,                 \
+      const double *tile_dd, const int *grp, int n_grp, const double *pconst, const double *nodes,           \
       const double *nodes_grad, int NNS, double du, ModeList modes, int P, int rows, const int *tile_jr,     \
-      int tile_begin, int tile_end, int group_offset, int *work_counter, double *partial,                    \
-      const unsigned long long *off_bits, const unsigned char *items
+      int tile_begin, int group_offset, int *work_counter, double *partial,                                  \
+      const unsigned long long *off_bits, const unsigned char *items, const int *tile_pan,                   \
+      BinWork bw, int range, int list_base, const unsigned long long *dbits, int fine
 #define PES_LNL_NAMES                                                                                     \
-  dets, n_det, n_tiles, bin_f, bin_j, bin_s, bin_rec, tile_f0, tile_dd, tiles_per_group, pconst, \
-      nodes, nodes_grad, NNS, du, modes, P, rows, tile_jr, tile_begin, tile_end, group_offset, work_counter, partial, \
-      off_bits, items
+  dets, n_det, n_tiles, bin_f, bin_j, bin_s, bin_rec, tile_f0, tile_dd, grp, n_grp, pconst,  \
+      nodes, nodes_grad, NNS, du, modes, P, rows, tile_jr, tile_begin, group_offset, work_counter, partial, \
+      off_bits, items, tile_pan, bw, range, list_base, dbits, fine
 
 }  // namespace
 
@@ -1022,12 +1087,19 @@ hipError_t launch_lnl_fwd(int precision, int kd, int grid, hipStream_t st, PES_L
 hipError_t pes::launch_lnl_fwd(int precision, int kd, int grid, hipStream_t st, PES_LNL_PARAMS) {
   // lnL alone is the FP64 forward in every precision mode (the modes differ in the adjoint only)
   (void)precision;
+#define PES_LNL_FWD(KD)                                                                                     \
+  if (dbits)                                                                                                \
+    hipLaunchKernelGGL((k_lnl<0, false, KD, true>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES);          \
+  else                                                                                                      \
+    hipLaunchKernelGGL((k_lnl<0, false, KD, false>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES);         \
+  break;
   switch (kd) {
-    case 0: hipLaunchKernelGGL((k_lnl<0, false, 0>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES); break;
-    case 1: hipLaunchKernelGGL((k_lnl<0, false, 1>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES); break;
-    case 2: hipLaunchKernelGGL((k_lnl<0, false, 2>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES); break;
-    default: hipLaunchKernelGGL((k_lnl<0, false, 3>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES); break;
+    case 0: PES_LNL_FWD(0)
+    case 1: PES_LNL_FWD(1)
+    case 2: PES_LNL_FWD(2)
+    default: PES_LNL_FWD(3)
   }
+#undef PES_LNL_FWD
   return hipGetLastError();
 }
 #else
@@ -1069,6 +1141,21 @@ struct pes_context {
          *d_partial = nullptr;
   int* d_work_counter = nullptr;
   unsigned long long* d_off_bits = nullptr;  // [cap_P][off_words] duty off-tile flags (duty contexts)
+  // panels of the tiles that the panel kernel takes (none: pan.tile_pan is null); per row the
+  // tiles that go bin by bin all the same, and per tile the last batch in which a row does
+  PanelDev pan{};
+  int *d_tile_pan = nullptr, *d_pan_i = nullptr, *d_bin_work = nullptr;
+  BinWork bin_work{};
+  double* d_pan_d = nullptr;
+  double2* d_pan_rec = nullptr;
+  unsigned long long* d_dbits = nullptr;  // [cap_P][off_words]
+  int n_bin_tiles = 0;  // tiles without panels
+  std::vector<int> tile_panels;  // panels per tile
+  std::vector<int> tile_pan0;    // panels before each tile, and their number
+  std::vector<int> groups;       // first tile of each tile group (build_groups), and n_tiles
+  int* d_groups = nullptr;
+  double* d_fine = nullptr;  // per-tile sums of small batches (fine_doubles)
+  size_t cap_fine = 0;
   int n_cu = 256;
   // optional timing of the fused kernel (HIP events on the launch stream)
   bool profiling = false;
@@ -1204,42 +1291,74 @@ extern "C" int pes_context_set_duty_cycle(pes_context* ctx, int det_index, doubl
   return PES_OK;
 }
 
-// The fused kernel's launches: maximal runs of consecutive detectors with the same duty flag,
-// each split into groups of tiles_per_group tiles (a group never straddles two runs), with the
-// partial sums of run r's groups at group_offset(r) + 0, 1, ...
+// Runs of consecutive detectors with the same orbit kind and duty flag: each is launched in the
+// fused kernels' instantiation for that kind (only its code, so that its register allocation is
+// not that of the other kind's code as well), with the partial sums of run r's tile groups at
+// group_offset + 0, 1, ...
 struct TileRange {
-  int tile_begin, tile_end, duty, kind, group_offset;
+  int tile_begin, tile_end, duty, kind, group_offset, n_groups;
 };
-// runs of consecutive detectors with the same orbit kind and duty flag: each is launched in the
-// fused kernel's instantiation for that kind (only its code, so that its register allocation is
-// not that of the other kind's code as well)
 static int tile_ranges(const pes_context* ctx, TileRange* out) {
-  int n = 0, groups = 0;
+  int n = 0;
   for (const auto& h : ctx->hdets) {
     const int t0 = h.d.bin_offset / TILE, t1 = t0 + h.d.n_tiles, duty = h.d.duty ? 1 : 0, kind = h.d.kind;
     if (n > 0 && out[n - 1].duty == duty && out[n - 1].kind == kind && out[n - 1].tile_end == t0) {
       out[n - 1].tile_end = t1;
     } else {
-      out[n++] = {t0, t1, duty, kind, 0};
+      out[n++] = {t0, t1, duty, kind, 0, 0};
     }
   }
-  for (int r = 0; r < n; ++r) {
-    out[r].group_offset = groups;
-    groups += (out[r].tile_end - out[r].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
+  for (int r = 0, g = 0; r < n && !ctx->groups.empty(); ++r) {
+    out[r].group_offset = g;
+    while (ctx->groups[g] < out[r].tile_end) ++g;
+    out[r].n_groups = g - out[r].group_offset;
   }
   return n;
+}
+
+// The tile groups (first tile of each, and the number of tiles): at most tiles_per_group tiles
+// each, none across two runs; with panels also at most GROUP_PANELS panels, so that the work items
+// of the low frequencies, whose tiles are cut into several panels or go bin by bin, do not outlast
+// the others (the network, P = 45 with the gradient: 16.8 -> 10.2 ms)
+constexpr int GROUP_PANELS = 12, GROUP_BIN_TILE = 4;
+static int build_groups(pes_context* ctx) {
+  TileRange r[MAX_TILE_RANGES];
+  ctx->groups.clear();
+  const int n = tile_ranges(ctx, r);
+  for (int i = 0; i < n; ++i) {
+    int tiles = 0, cost = 0;
+    for (int t = r[i].tile_begin; t < r[i].tile_end; ++t) {
+      int c = 0;
+      if (ctx->pan.tile_pan) c = ctx->tile_panels[t] > 0 ? ctx->tile_panels[t] : GROUP_BIN_TILE;
+      if (t == r[i].tile_begin || tiles == ctx->tiles_per_group || cost + c > GROUP_PANELS) {
+        ctx->groups.push_back(t);
+        tiles = cost = 0;
+      }
+      ++tiles;
+      cost += c;
+    }
+  }
+  ctx->groups.push_back(ctx->n_tiles);
+  if (!ctx->d_groups) HIP_TRY(hipMalloc(&ctx->d_groups, ((size_t)ctx->n_tiles + 1) * sizeof(int)));
+  HIP_TRY(hipMemcpy(ctx->d_groups, ctx->groups.data(), ctx->groups.size() * sizeof(int), hipMemcpyHostToDevice));
+  if (ctx->pan.tile_pan) {  // group and range of each tile (BinWork)
+    std::vector<int> tg(ctx->n_tiles), tr(ctx->n_tiles);
+    for (size_t g = 0; g + 1 < ctx->groups.size(); ++g)
+      for (int t = ctx->groups[g]; t < ctx->groups[g + 1]; ++t) tg[t] = (int)g;
+    for (int i = 0; i < n; ++i)
+      for (int t = r[i].tile_begin; t < r[i].tile_end; ++t) tr[t] = i;
+    int* to = ctx->d_bin_work + (ctx->bin_work.tile_group - ctx->d_bin_work);
+    HIP_TRY(hipMemcpy(to, tg.data(), tg.size() * sizeof(int), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(to + ctx->n_tiles, tr.data(), tr.size() * sizeof(int), hipMemcpyHostToDevice));
+  }
+  return PES_OK;
 }
 
 // 64-bit words per row of the duty off-tile flags (one bit per tile of the context; the fused
 // kernel forms the same count from n_tiles)
 static int off_words_of(const pes_context* ctx) { return (ctx->n_tiles + 63) / 64; }
 
-static int n_groups_of(const pes_context* ctx) {
-  TileRange r[MAX_TILE_RANGES];
-  const int n = tile_ranges(ctx, r);
-  return r[n - 1].group_offset +
-         (r[n - 1].tile_end - r[n - 1].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
-}
+static int n_groups_of(const pes_context* ctx) { return (int)ctx->groups.size() - 1; }
 
 // ---- the entry point that allocates nothing ---------------------------------------------------
 // Its scratch (work counter, per-row setup and constants, node tables, per-tile-group partials)
@@ -1268,8 +1387,25 @@ static int noalloc_base(int device, char** out) {
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// byte offsets of the scratch buffers of a batch of P rows inside the array, and their total
-static size_t noalloc_layout(const pes_context* ctx, int P, bool grad, size_t off[8]) {
+// What a batch is accounted for against the array: the layout of a batch whose tile groups all
+// hold tiles_per_group tiles, without the panels' flags
+static size_t noalloc_account(const pes_context* ctx, int P, bool grad) {
+  const size_t NNS = (size_t)ctx->n_nodes + 1, rows = (size_t)P, nm = (size_t)ctx->modes.n;
+  TileRange r[MAX_TILE_RANGES];
+  const int n = tile_ranges(ctx, r);
+  size_t groups = 0;
+  for (int i = 0; i < n; ++i)
+    groups += (r[i].tile_end - r[i].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
+  size_t o = align256(N_WORK_COUNTERS * sizeof(int)) + align256(rows * N_SETUP * 5 * sizeof(double)) +
+             align256(rows * PC_STRIDE * sizeof(double)) + align256(rows * nm * NNS * 4 * sizeof(double));
+  if (grad) o += align256(rows * nm * NNS * 16 * sizeof(double));
+  o += align256(groups * (grad ? 1 + PES_N_PARAMS : 1) * rows * sizeof(double));
+  if (ctx->any_duty) o += align256(rows * off_words_of(ctx) * sizeof(unsigned long long)) + align256(groups * rows);
+  return o;
+}
+// byte offsets of the scratch buffers of P rows inside the array, and their total.  A batch that
+// is accounted within the array but needs more runs in parts (rows do not depend on their batch)
+static size_t noalloc_layout(const pes_context* ctx, int P, bool grad, size_t off[9]) {
   const size_t NNS = (size_t)ctx->n_nodes + 1, rows = (size_t)P, nm = (size_t)ctx->modes.n;
   size_t o = 0;
   off[0] = o; o += align256(N_WORK_COUNTERS * sizeof(int));                // work counters
@@ -1280,11 +1416,110 @@ static size_t noalloc_layout(const pes_context* ctx, int P, bool grad, size_t of
   off[5] = o; o += align256((size_t)n_groups_of(ctx) * (grad ? 1 + PES_N_PARAMS : 1) * rows * sizeof(double));
   off[6] = o; if (ctx->any_duty) o += align256(rows * off_words_of(ctx) * sizeof(unsigned long long));  // off tiles
   off[7] = o; if (ctx->any_duty) o += align256((size_t)n_groups_of(ctx) * rows);  // work items: plain or duty
+  off[8] = o; if (ctx->pan.tile_pan) o += align256(rows * off_words_of(ctx) * sizeof(unsigned long long));
   return o;
 }
 
 static void free_dev(void* p) {
   if (p) (void)hipFree(p);
+}
+
+// Panels (panel.hpp): each tile is cut at its node interval ends, and each part into equal panels
+// within the truncation bounds; a tile of more than PANEL_MAX_PIECES stays bin by bin (its panels
+// would hold too few bins to pay for their points).  bf, bj: frequency and node interval per bin.
+static int build_panels(pes_context* ctx, const std::vector<double>& bf, const std::vector<int>& bj) {
+  if (ctx->direct) return PES_OK;
+  const int nt = ctx->n_tiles;
+  std::vector<int> tp(2 * (size_t)nt, 0), pi;
+  std::vector<double> pd;
+  for (const auto& h : ctx->hdets) {
+    const int t0 = h.d.bin_offset / TILE;
+    for (int t = t0; t < t0 + h.d.n_tiles; ++t) {
+      const int bin0 = t * TILE, nb = std::min(TILE, h.d.n_bins - (t - t0) * TILE);
+      int parts[3 * PANEL_MAX_PIECES], np = 0;  // (first bin in the tile, bins, node interval)
+      for (int a = 0; a < nb && np >= 0;) {
+        int e = a + 1;
+        while (e < nb && bj[bin0 + e] == bj[bin0 + a]) ++e;
+        const double lo = bf[bin0 + a], hi = bf[bin0 + e - 1];
+        const double cuts = std::max((hi - lo) / ((hi + lo) * PANEL_EPS), 4.0 * PI * h.d.L * (hi - lo) / PANEL_SWING);
+        const int k = cuts < (double)(e - a) ? std::max(1, (int)std::ceil(cuts)) : e - a;
+        if (np + k > PANEL_MAX_PIECES) {
+          np = -1;
+          break;
+        }
+        for (int i = 0; i < k; ++i) {
+          const int b0 = a + (int)((long long)(e - a) * i / k), b1 = a + (int)((long long)(e - a) * (i + 1) / k);
+          parts[3 * np] = b0;
+          parts[3 * np + 1] = b1 - b0;
+          parts[3 * np + 2] = bj[bin0 + a];
+          ++np;
+        }
+        a = e;
+      }
+      if (np <= 0) continue;
+      tp[2 * (size_t)t] = (int)(pi.size() / 4);
+      tp[2 * (size_t)t + 1] = np;
+      for (int k = 0; k < np; ++k) {
+        const int b0 = parts[3 * k], n = parts[3 * k + 1], j = parts[3 * k + 2];
+        const double lo = bf[bin0 + b0], hi = bf[bin0 + b0 + n - 1];
+        const double mid = 0.5 * (lo + hi), half = std::max(0.5 * (hi - lo), 1e-9 * mid);  // one bin: any width
+        double d[PAN_D] = {mid, 1.0 / half, half};
+        auto place = [&](double f) { return (std::log(f) - ctx->u0) / ctx->du - (double)j; };
+        d[3] = place(mid - half);
+        d[4] = place(mid + half);
+        for (int q = 0; q < PANEL_K; ++q) {  // bin_prepare at the point
+          double* pt = d + PAN_PT + q * PAN_PT_D;
+          const double f = mid + half * panel_x(q), sq = place(f), s1 = 1.0 - sq, du = ctx->du;
+          const double g = 1.0 / (2.0 * PI * du * f);
+          pt[0] = f;
+          pt[1] = sq * sq * (3.0 - 2.0 * sq);
+          pt[2] = sq * s1 * s1 * du;
+          pt[3] = -sq * sq * s1 * du;
+          pt[4] = 6.0 * sq * s1 * g;
+          pt[5] = s1 * (1.0 - 3.0 * sq) * du * g;
+          pt[6] = sq * (3.0 * sq - 2.0) * du * g;
+          pt[7] = std::sin(PI * f * h.d.L);
+          pt[8] = std::cos(PI * f * h.d.L);
+        }
+        pi.insert(pi.end(), {j, b0, n, t});
+        pd.insert(pd.end(), d, d + PAN_D);
+      }
+    }
+  }
+  if (pi.empty()) return PES_OK;
+  for (int t = 0; t < nt; ++t) ctx->n_bin_tiles += tp[2 * (size_t)t + 1] == 0 ? 1 : 0;
+  // a context's rows all go the same way, whatever the batch (a row's result does not depend on
+  // it), so short grids, whose few panel tiles are not worth the two further launches of a small
+  // batch (~12 us), have no panels
+  if (nt - ctx->n_bin_tiles < PANEL_MIN_TILES) {
+    ctx->n_bin_tiles = 0;
+    return PES_OK;
+  }
+  HIP_TRY(hipMalloc(&ctx->d_tile_pan, tp.size() * sizeof(int)));
+  HIP_TRY(hipMalloc(&ctx->d_pan_i, pi.size() * sizeof(int)));
+  HIP_TRY(hipMalloc(&ctx->d_pan_d, pd.size() * sizeof(double)));
+  HIP_TRY(hipMalloc(&ctx->d_pan_rec, (size_t)ctx->NB * PANEL_REC * sizeof(double2)));
+  constexpr int STATE = 64;  // ints before the first array
+  HIP_TRY(hipMalloc(&ctx->d_bin_work, (STATE + 5 * (size_t)nt) * sizeof(int)));
+  HIP_TRY(hipMemcpy(ctx->d_tile_pan, tp.data(), tp.size() * sizeof(int), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(ctx->d_pan_i, pi.data(), pi.size() * sizeof(int), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(ctx->d_pan_d, pd.data(), pd.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemset(ctx->d_bin_work, 0, (STATE + 5 * (size_t)nt) * sizeof(int)));
+  int* w = ctx->d_bin_work + STATE;
+  ctx->bin_work = {ctx->d_bin_work, w, w + nt, w + 2 * (size_t)nt, w + 3 * (size_t)nt, w + 4 * (size_t)nt};
+  for (int i = 0; i < (int)ctx->hdets.size(); ++i)
+    hipLaunchKernelGGL(k_panel_rec, dim3(ctx->hdets[i].d.n_tiles), dim3(TILE), 0, nullptr, ctx->d_dets, i,
+                       ctx->d_bin_f, ctx->d_bin_s, ctx->d_bin_j, ctx->d_bin_rec, ctx->du, ctx->d_pan_rec);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipDeviceSynchronize());  // the record is read on the callers' streams
+  ctx->tile_panels.resize(nt);
+  ctx->tile_pan0.assign(nt + 1, 0);
+  for (int t = 0; t < nt; ++t) {
+    ctx->tile_panels[t] = tp[2 * (size_t)t + 1];
+    ctx->tile_pan0[t + 1] = ctx->tile_pan0[t] + ctx->tile_panels[t];
+  }
+  ctx->pan = {ctx->d_tile_pan, ctx->d_pan_i, ctx->d_pan_d, ctx->d_pan_rec};
+  return PES_OK;
 }
 
 extern "C" int pes_context_finalize(pes_context* ctx) {
@@ -1418,6 +1653,11 @@ extern "C" int pes_context_finalize(pes_context* ctx) {
     HIP_TRY(hipMemcpy(ctx->d_tile_jr, tjr.data(), 2 * (size_t)nt * sizeof(int), hipMemcpyHostToDevice));
   }
   if (ctx->direct) ctx->d_node_f = ctx->d_bin_f;
+  {
+    int rc = build_panels(ctx, bf, bj);
+    if (rc == PES_OK) rc = build_groups(ctx);
+    if (rc != PES_OK) return rc;
+  }
   HIP_TRY(hipMalloc(&ctx->d_work_counter, N_WORK_COUNTERS * sizeof(int)));  // one per fused-kernel launch
   {  // the device address of the no-allocation entry point's scratch, once per device
     char* base = nullptr;
@@ -1445,6 +1685,14 @@ extern "C" void pes_context_destroy(pes_context* ctx) {
   free_dev(ctx->d_nodes);
   free_dev(ctx->d_nodes_grad);
   free_dev(ctx->d_off_bits);
+  free_dev(ctx->d_dbits);
+  free_dev(ctx->d_tile_pan);
+  free_dev(ctx->d_pan_i);
+  free_dev(ctx->d_pan_d);
+  free_dev(ctx->d_pan_rec);
+  free_dev(ctx->d_bin_work);
+  free_dev(ctx->d_fine);
+  free_dev(ctx->d_groups);
   free_dev(ctx->d_partial);
   free_dev(ctx->d_live);
   for (auto e : ctx->ev_start) (void)hipEventDestroy(e);
@@ -1472,10 +1720,28 @@ static size_t partial_doubles(const pes_context* ctx, size_t cap) {
   return n;
 }
 
+// Batches of fewer rows than this run one tile per work item (k_group_sums): those whose groups of
+// tiles_per_group tiles would give less than about one item to each wave (panels) or block of the
+// chip (16 rows of six modes on short data with the gradient: 64 items on 256 CUs, 1.24 -> 0.25 ms)
+static int fine_rows(const pes_context* ctx) {
+  const int groups = n_groups_of(ctx);
+  return ctx->pan.tile_pan ? 2048 * PANEL_ROWS / groups : 1024 * 8 / groups;
+}
+// their per-tile sums, and the duty flags of their work items, for every batch of up to cap rows
+static size_t fine_doubles(const pes_context* ctx, int cap, bool grad) {
+  const size_t rows = (size_t)std::max(0, std::min(cap, fine_rows(ctx) - 1));
+  const size_t slots = (size_t)(TILE / 64) * ctx->n_tiles + (ctx->pan.tile_pan ? ctx->tile_pan0.back() : 0);
+  size_t n = slots * (grad ? 1 + PES_N_PARAMS : 1) * rows;
+  if (ctx->any_duty) n += ((size_t)ctx->n_tiles * rows + 7) / 8;
+  return n;
+}
+
 static int ensure_scratch(pes_context* ctx, int P, bool grad) {
   {
     const size_t need = partial_doubles(ctx, (size_t)(P > ctx->cap_P ? P : ctx->cap_P));
-    const bool grow = need > ctx->cap_partial || P > ctx->cap_P || (grad && !ctx->cap_grad);
+    const size_t fine = fine_doubles(ctx, P > ctx->cap_P ? P : ctx->cap_P, grad || ctx->cap_grad);
+    const bool grow =
+        need > ctx->cap_partial || fine > ctx->cap_fine || P > ctx->cap_P || (grad && !ctx->cap_grad);
     if (grow && ctx->pinned)
       return fail(PES_ERR_STATE,
                   "scratch is pinned (a captured HIP graph holds its pointers) and this call needs more: "
@@ -1485,6 +1751,12 @@ static int ensure_scratch(pes_context* ctx, int P, bool grad) {
       ctx->d_partial = nullptr;
       HIP_TRY(hipMalloc(&ctx->d_partial, need * sizeof(double)));
       ctx->cap_partial = need;
+    }
+    if (fine > ctx->cap_fine) {
+      free_dev(ctx->d_fine);
+      ctx->d_fine = nullptr;
+      HIP_TRY(hipMalloc(&ctx->d_fine, fine * sizeof(double)));
+      ctx->cap_fine = fine;
     }
   }
   if (P <= ctx->cap_P && (!grad || ctx->cap_grad)) return PES_OK;
@@ -1496,8 +1768,9 @@ static int ensure_scratch(pes_context* ctx, int P, bool grad) {
   free_dev(ctx->d_nodes);
   free_dev(ctx->d_nodes_grad);
   free_dev(ctx->d_off_bits);
+  free_dev(ctx->d_dbits);
   ctx->d_setup = ctx->d_pconst = ctx->d_nodes = ctx->d_nodes_grad = nullptr;
-  ctx->d_off_bits = nullptr;
+  ctx->d_off_bits = ctx->d_dbits = nullptr;
   size_t NNS = (size_t)ctx->n_nodes + 1;
   HIP_TRY(hipMalloc(&ctx->d_setup, (size_t)cap * N_SETUP * 5 * sizeof(double)));
   HIP_TRY(hipMalloc(&ctx->d_pconst, (size_t)cap * PC_STRIDE * sizeof(double)));
@@ -1505,6 +1778,8 @@ static int ensure_scratch(pes_context* ctx, int P, bool grad) {
   if (g) HIP_TRY(hipMalloc(&ctx->d_nodes_grad, (size_t)cap * ctx->modes.n * NNS * 16 * sizeof(double)));
   if (ctx->any_duty)
     HIP_TRY(hipMalloc(&ctx->d_off_bits, (size_t)cap * off_words_of(ctx) * sizeof(unsigned long long)));
+  if (ctx->pan.tile_pan)
+    HIP_TRY(hipMalloc(&ctx->d_dbits, (size_t)cap * off_words_of(ctx) * sizeof(unsigned long long)));
   ctx->cap_P = cap;
   ctx->cap_grad = g;
   return PES_OK;
@@ -1516,6 +1791,8 @@ struct BatchScratch {
   int* work_counter;
   unsigned long long* off_bits;  // duty contexts only
   unsigned char* items;          // duty contexts only: [groups][chunks] plain (1) or duty (0)
+  unsigned long long* dbits;     // panels: per row the tiles that go bin by bin (null: all of them)
+  double* fine;                  // per-tile sums of a small batch (null: items of tiles_per_group tiles)
 };
 
 static BatchScratch context_scratch(const pes_context* ctx) {
@@ -1524,7 +1801,8 @@ static BatchScratch context_scratch(const pes_context* ctx) {
           ? reinterpret_cast<unsigned char*>(ctx->d_partial + items_offset_doubles(ctx, (size_t)ctx->cap_P))
           : nullptr;
   return {ctx->d_setup,   ctx->d_pconst,       ctx->d_nodes,    ctx->d_nodes_grad,
-          ctx->d_partial, ctx->d_work_counter, ctx->d_off_bits, items};
+          ctx->d_partial, ctx->d_work_counter, ctx->d_off_bits, items, ctx->d_dbits,
+          ctx->d_fine};
 }
 
 static int check_batch_args(const pes_context* ctx, const double* d_params, int P) {
@@ -1538,8 +1816,9 @@ static int check_batch_args(const pes_context* ctx, const double* d_params, int 
 // k_setup (which also zeroes the work counters) and k_nodes for P >= 1 rows
 static int launch_setup_nodes(const pes_context* ctx, const BatchScratch& sc, const double* d_params, int P, bool grad,
                               hipStream_t st) {
-  hipLaunchKernelGGL(k_setup, dim3((P + SETUP_ROWS - 1) / SETUP_ROWS), dim3(192), 0, st, d_params, P, ctx->modes,
-                     ctx->f_ref, sc.setup, sc.pconst, sc.work_counter);
+  const dim3 sg((P + SETUP_ROWS - 1) / SETUP_ROWS);
+  hipLaunchKernelGGL(k_setup, sg, dim3(192), 0, st, d_params, P, ctx->modes, ctx->f_ref, sc.setup, sc.pconst,
+                     sc.work_counter, ctx->bin_work.state);
   HIP_TRY(hipGetLastError());
   const int NNS = ctx->n_nodes + 1;
   dim3 g((NNS + 127) / 128, P * ctx->modes.n);
@@ -1565,11 +1844,16 @@ static int prepare(pes_context* ctx, const double* d_params, int P, bool grad, h
 }
 
 // rows per work item of the fused kernel: the kernel's chunk, fewer when the grid has too few
-// tile groups to give every persistent block about four work items (small grids, e.g. 16k bins)
-static int rows_per_item(const pes_context* ctx, int P, bool grad, int grid) {
+// tile groups to give every persistent block about four work items (small grids, e.g. 16k bins).
+// With panels the bin-by-bin kernel has little beyond the tiles without any (a year of LISA data:
+// 3 of 769 groups), so it is those that have to fill the chip: P = 512, 1.68 ms with 160 rows per
+// item, 0.57 with 8
+static int rows_per_item(const pes_context* ctx, int P, bool grad, int grid, bool panels, bool fine) {
   const int max_rows = grad ? chunk_rows<true>() : chunk_rows<false>();
   if (ctx->rows_override > 0) return std::min(ctx->rows_override, max_rows);
-  const long long fit = (long long)P * n_groups_of(ctx) / (4LL * grid);
+  const int per = fine ? 1 : std::min(ctx->tiles_per_group, GROUP_PANELS / GROUP_BIN_TILE);
+  const int groups = panels ? ctx->n_bin_tiles / per + 1 : (fine ? ctx->n_tiles : n_groups_of(ctx));
+  const long long fit = (long long)P * groups / ((panels ? 2LL : 4LL) * grid);
   return (int)std::max(8LL, std::min((long long)max_rows, fit));
 }
 
@@ -1580,7 +1864,9 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   const int NNS = ctx->n_nodes + 1;
   const int n_groups = n_groups_of(ctx);
   int grid = ctx->n_cu * ctx->blocks_per_cu;
-  const int rows = rows_per_item(ctx, P, grad, grid);
+  const bool panels = sc.dbits != nullptr;
+  const bool fine = sc.fine && P < fine_rows(ctx);
+  const int rows = rows_per_item(ctx, P, grad, grid, panels, fine);
   const int n_chunks = (P + rows - 1) / rows;
   const int nout = grad ? 1 + PES_N_PARAMS : 1;
   // one launch per run of detectors with the same duty flag (two for a duty-cycled run, below):
@@ -1588,6 +1874,13 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   // register allocation is that of a kernel without the window code)
   TileRange ranges[MAX_TILE_RANGES];
   const int n_ranges = tile_ranges(ctx, ranges);
+  double *part_pan = sc.partial, *part_bin = sc.partial;
+  unsigned char* items_buf = sc.items;
+  if (fine) {
+    part_bin = sc.fine;
+    part_pan = part_bin + (size_t)(TILE / 64) * ctx->n_tiles * nout * P;
+    items_buf = reinterpret_cast<unsigned char*>(part_pan + (panels ? (size_t)ctx->tile_pan0.back() * nout * P : 0));
+  }
   const int off_words = off_words_of(ctx);
   if (ctx->any_duty) {  // tiles that a duty cycle's off periods cover for every mode of a row
     hipLaunchKernelGGL(k_duty_off, dim3(off_words, std::min(P, 65535)), dim3(64), 0, st, ctx->d_dets,
@@ -1596,16 +1889,27 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     HIP_TRY(hipGetLastError());
   }
   const int n_det = (int)ctx->hdets.size();
+  if (panels) {  // which (tile, row)s of the tiles with panels go bin by bin all the same
+    RangeBases rb{};
+    for (int r = 0; r < n_ranges; ++r) {
+      rb.tile0[r] = ranges[r].tile_begin;
+      rb.group0[r] = ranges[r].group_offset;
+    }
+    hipLaunchKernelGGL(k_panel_class, dim3(off_words, std::min(P, 65535)), dim3(64), 0, st, ctx->d_dets, n_det,
+                       ctx->n_tiles, ctx->d_tile_f0, ctx->d_bin_f, sc.pconst, sc.nodes, NNS, ctx->du, ctx->modes, P,
+                       off_words, ctx->any_duty ? sc.off_bits : nullptr, ctx->pan, ctx->bin_work, rb, fine ? 1 : 0,
+                       sc.dbits);
+    HIP_TRY(hipGetLastError());
+  }
   // a duty-cycled range's work items on the window's plateau (for every row and mode of the item)
   // run in the plain instantiation, the others in the duty one: two launches of the range
   for (int r = 0; r < n_ranges; ++r) {
     if (!ranges[r].duty) continue;
-    const int n_work =
-        (ranges[r].tile_end - ranges[r].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group * n_chunks;
+    const int n_grp = fine ? ranges[r].tile_end - ranges[r].tile_begin : ranges[r].n_groups, n_work = n_grp * n_chunks;
     hipLaunchKernelGGL(k_duty_items, dim3(n_work), dim3(64), 0, st, ctx->d_dets, n_det, ctx->d_tile_f0,
                        ctx->d_tile_jr, sc.pconst, sc.nodes, NNS, ctx->u0, ctx->du, ctx->modes, P, rows, n_chunks,
-                       ranges[r].tile_begin, ranges[r].tile_end, ctx->tiles_per_group, ranges[r].group_offset,
-                       ctx->direct ? 0 : 1, sc.items, sc.work_counter + 2 * MAX_TILE_RANGES + r);
+                       ranges[r].tile_begin, fine ? nullptr : ctx->d_groups + ranges[r].group_offset,
+                       fine ? ranges[r].tile_begin : ranges[r].group_offset, ctx->direct ? 0 : 1, items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, sc.dbits);
     HIP_TRY(hipGetLastError());
   }
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1615,23 +1919,55 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     HIP_TRY(hipEventRecord(e0, st));
   }
   for (int r = 0; r < n_ranges; ++r) {
-    const int tile_begin = ranges[r].tile_begin, tile_end = ranges[r].tile_end;
-    const int group_offset = ranges[r].group_offset;
-    const int n_work = (tile_end - tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group * n_chunks;
+    const int tile_begin = ranges[r].tile_begin;
+    const int group_offset = fine ? tile_begin : ranges[r].group_offset;  // fine: a partial per tile
+    const int* grp = fine ? nullptr : ctx->d_groups + group_offset;
+    const int n_grp = fine ? ranges[r].tile_end - tile_begin : ranges[r].n_groups;
+    const int n_work = n_grp * n_chunks;
     const int grid_r = std::min(grid, n_work);
+    if (panels) {
+      int* counter = sc.work_counter + 3 * MAX_TILE_RANGES + r;
+      const unsigned long long* off = ranges[r].duty ? sc.off_bits : nullptr;
+      // fine: an item is a panel, with sums of its own
+      const int pan_begin = ctx->tile_pan0[tile_begin], pan_end = ctx->tile_pan0[ranges[r].tile_end];
+      const int n_pg = fine ? pan_end - pan_begin : n_grp;
+      const int n_items = n_pg * ((P + PANEL_ROWS - 1) / PANEL_ROWS);
+      // two blocks per CU are resident; a wave takes an item
+      const int grid_p = std::min(2 * ctx->n_cu, (n_items + TILE / 64 - 1) / (TILE / 64));
+#define PES_PANEL_ARGS                                                                                        \
+  ctx->d_dets, n_det, ctx->n_tiles, ctx->d_tile_f0, ctx->d_tile_dd, grp, n_pg, sc.pconst, sc.nodes,            \
+      sc.nodes_grad, NNS, ctx->du, ctx->modes, P, fine ? pan_begin : group_offset, counter,                   \
+      part_pan, off, sc.dbits, ctx->pan, pan_begin
+#define PES_PANEL(G, KD) \
+  hipLaunchKernelGGL((k_lnl_panel<G, KD>), dim3(grid_p), dim3(TILE), 0, st, PES_PANEL_ARGS)
+      if (grad) {
+        if (ranges[r].kind == 0) PES_PANEL(true, 0);
+        else PES_PANEL(true, 1);
+      } else {
+        if (ranges[r].kind == 0) PES_PANEL(false, 0);
+        else PES_PANEL(false, 1);
+      }
+#undef PES_PANEL
+#undef PES_PANEL_ARGS
+      HIP_TRY(hipGetLastError());
+    }
     for (int pass = 0; pass < (ranges[r].duty ? 2 : 1); ++pass) {
       // pass 0: the plain instantiation (all items of a plain range; the plateau items of a
       // duty-cycled one), pass 1: the duty instantiation (the other items); both for the range's
       // orbit kind only
       const int kd = ranges[r].kind | (pass == 1 ? 2 : 0);
-      const unsigned char* items = ranges[r].duty ? sc.items : nullptr;
+      const unsigned char* items = ranges[r].duty ? items_buf : nullptr;
       int* counter = sc.work_counter + (pass == 0 ? r : MAX_TILE_RANGES + r);
 #define PES_LNL_ARGS                                                                                         \
   ctx->d_dets, n_det, ctx->n_tiles, ctx->d_bin_f, ctx->d_bin_j, ctx->d_bin_s, ctx->d_bin_rec,                 \
-      ctx->d_tile_f0, ctx->d_tile_dd, ctx->tiles_per_group, sc.pconst, sc.nodes, sc.nodes_grad, NNS, ctx->du, \
-      ctx->modes, P, rows, ctx->d_tile_jr, tile_begin, tile_end, group_offset, counter, sc.partial,       \
-      sc.off_bits, items
-#define PES_LNL_GRAD(PR, KD) hipLaunchKernelGGL((k_lnl<PR, true, KD>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS)
+      ctx->d_tile_f0, ctx->d_tile_dd, grp, n_grp, sc.pconst, sc.nodes, sc.nodes_grad, NNS, ctx->du,           \
+      ctx->modes, P, rows, ctx->d_tile_jr, tile_begin, group_offset, counter, part_bin,                       \
+      sc.off_bits, items, ctx->pan.tile_pan, ctx->bin_work, r, group_offset, sc.dbits, fine ? 1 : 0
+#define PES_LNL_GRAD(PR, KD)                                                                                  \
+  if (panels)                                                                                                \
+    hipLaunchKernelGGL((k_lnl<PR, true, KD, true>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS);          \
+  else                                                                                                       \
+    hipLaunchKernelGGL((k_lnl<PR, true, KD, false>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS)
       if (!grad) {
         HIP_TRY(launch_lnl_fwd(precision, kd, grid_r, st, PES_LNL_ARGS));
       } else if (precision == 0) {
@@ -1661,16 +1997,26 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     ctx->live_P = P;  // the work is counted by pes_profile_work, outside the caller's timed steps
     ctx->live_seq = ctx->scratch_seq;
   }
-  hipLaunchKernelGGL(k_reduce, dim3((P + 63) / 64, nout), dim3(64 * REDUCE_WAVES), 0, st, sc.partial, n_groups, P,
-                     nout, sc.pconst, d_lnl, d_grad);
+  if (fine) {
+    hipLaunchKernelGGL(k_group_sums, dim3((unsigned)(((size_t)n_groups * nout * P + 255) / 256)), dim3(256), 0, st,
+                       ctx->d_groups, n_groups, P, nout, panels ? part_pan : nullptr, part_bin, ctx->pan.tile_pan,
+                       ctx->bin_work, sc.partial);
+    HIP_TRY(hipGetLastError());
+  }
+#define PES_REDUCE(RB)                                                                                        \
+  hipLaunchKernelGGL(k_reduce<RB>, dim3((P + RB - 1) / RB, nout), dim3(256), 0, st, sc.partial, n_groups, P, \
+                     nout, sc.pconst, d_lnl, d_grad)
+  if (P > 512) PES_REDUCE(64);
+  else if (P > 32) PES_REDUCE(16);
+  else PES_REDUCE(4);
+#undef PES_REDUCE
   HIP_TRY(hipGetLastError());
   return PES_OK;
 }
 
 extern "C" size_t pes_lnl_batch_noalloc_bytes(const pes_context* ctx, int P, int grad) {
   if (!ctx || !ctx->finalized || P < 1) return 0;
-  size_t off[8];
-  return noalloc_layout(ctx, P, grad != 0, off);
+  return noalloc_account(ctx, P, grad != 0);
 }
 
 extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, int P, double* d_lnl, double* d_grad,
@@ -1681,8 +2027,7 @@ extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, i
   int rc = check_batch_args(ctx, d_params, P);
   if (rc != PES_OK || P == 0) return rc;
   const bool grad = d_grad != nullptr;
-  size_t off[8];
-  const size_t need = noalloc_layout(ctx, P, grad, off);
+  const size_t need = noalloc_account(ctx, P, grad);
   if (need > (size_t)PES_NOALLOC_SCRATCH_BYTES) {
     char msg[256];
     std::snprintf(msg, sizeof msg,
@@ -1695,19 +2040,34 @@ extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, i
   char* base = nullptr;
   rc = noalloc_base(ctx->device, &base);
   if (rc != PES_OK) return rc;
-  BatchScratch sc;
-  sc.work_counter = reinterpret_cast<int*>(base + off[0]);
-  sc.setup = reinterpret_cast<double*>(base + off[1]);
-  sc.pconst = reinterpret_cast<double*>(base + off[2]);
-  sc.nodes = reinterpret_cast<double*>(base + off[3]);
-  sc.nodes_grad = grad ? reinterpret_cast<double*>(base + off[4]) : nullptr;
-  sc.partial = reinterpret_cast<double*>(base + off[5]);
-  sc.off_bits = ctx->any_duty ? reinterpret_cast<unsigned long long*>(base + off[6]) : nullptr;
-  sc.items = ctx->any_duty ? reinterpret_cast<unsigned char*>(base + off[7]) : nullptr;
+  size_t off[9];
+  int part = P;
+  while (part > 1 && noalloc_layout(ctx, part, grad, off) > (size_t)PES_NOALLOC_SCRATCH_BYTES) part = (part + 1) / 2;
+  if (noalloc_layout(ctx, part, grad, off) > (size_t)PES_NOALLOC_SCRATCH_BYTES)
+    return fail(PES_ERR_INVALID, "pes_lnl_batch_noalloc: one row needs more than the fixed scratch");
   hipStream_t st = (hipStream_t)stream;
-  rc = launch_setup_nodes(ctx, sc, d_params, P, grad, st);
-  if (rc != PES_OK) return rc;
-  return launch_lnl_reduce(ctx, sc, P, d_lnl, d_grad, precision, st, false);
+  for (int p0 = 0; p0 < P; p0 += part) {
+    const int n = std::min(part, P - p0);
+    noalloc_layout(ctx, n, grad, off);
+    BatchScratch sc;
+    sc.work_counter = reinterpret_cast<int*>(base + off[0]);
+    sc.setup = reinterpret_cast<double*>(base + off[1]);
+    sc.pconst = reinterpret_cast<double*>(base + off[2]);
+    sc.nodes = reinterpret_cast<double*>(base + off[3]);
+    sc.nodes_grad = grad ? reinterpret_cast<double*>(base + off[4]) : nullptr;
+    sc.partial = reinterpret_cast<double*>(base + off[5]);
+    sc.off_bits = ctx->any_duty ? reinterpret_cast<unsigned long long*>(base + off[6]) : nullptr;
+    sc.items = ctx->any_duty ? reinterpret_cast<unsigned char*>(base + off[7]) : nullptr;
+    sc.dbits = ctx->pan.tile_pan ? reinterpret_cast<unsigned long long*>(base + off[8]) : nullptr;
+    sc.fine = nullptr;
+    const double* params = d_params + (size_t)p0 * PES_N_PARAMS;
+    rc = launch_setup_nodes(ctx, sc, params, n, grad, st);
+    if (rc == PES_OK)
+      rc = launch_lnl_reduce(ctx, sc, n, d_lnl + p0, grad ? d_grad + (size_t)p0 * PES_N_PARAMS : nullptr, precision, st,
+                             false);
+    if (rc != PES_OK) return rc;
+  }
+  return PES_OK;
 }
 
 extern "C" int pes_lnl_batch(pes_context* ctx, const double* d_params, int P, double* d_lnl, double* d_grad,
@@ -1953,9 +2313,13 @@ extern "C" int pes_context_set_schedule(pes_context* ctx, int tiles_per_group, i
   if (!ctx) return fail(PES_ERR_INVALID, "ctx is NULL");
   if (tiles_per_group < 1 || tiles_per_group > 4096 || blocks_per_cu < 1 || blocks_per_cu > 64)
     return fail(PES_ERR_INVALID, "schedule: tiles_per_group in [1, 4096], blocks_per_cu in [1, 64]");
+  const bool regroup = ctx->finalized && tiles_per_group != ctx->tiles_per_group;
   ctx->tiles_per_group = tiles_per_group;
   ctx->blocks_per_cu = blocks_per_cu;
-  return PES_OK;
+  if (!regroup) return PES_OK;
+  HIP_TRY(hipSetDevice(ctx->device));
+  HIP_TRY(hipDeviceSynchronize());  // a batch in flight reads the groups
+  return build_groups(ctx);
 }
 
 extern "C" int pes_context_set_rows_per_item(pes_context* ctx, int rows) {

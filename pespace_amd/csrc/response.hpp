@@ -72,6 +72,27 @@ struct ModeList {  // the modes of a context (ids into kModeM etc.), passed to k
   int id[6];
 };
 
+struct PanelDev {  // device arrays of a context's panels (panel.hpp)
+  const int* tile_pan;     // [n_tiles][2]: first panel and number of panels (0: bin by bin)
+  const int* pan_i;        // [n][4]: node interval, first bin in its tile, bins, -
+  const double* pan_d;     // [n][56]
+  const double2* rec;      // [n_tiles][8][256]
+};
+
+
+// What a batch leaves to the bin-by-bin kernel in a context with panels, filled by k_panel_class:
+// state[0] the batch's number, state[1 + r] the number of entries of tile range r in list; a tile
+// (tile_any) and a group (group_any; a tile where an item is one tile) are marked with the batch's
+// number, so that nothing is cleared between batches
+struct BinWork {
+  int* state;
+  int* tile_any;
+  int* group_any;
+  int* list;
+  const int* tile_group;  // group and range of each tile
+  const int* tile_range;
+};
+
 // Host side: the orbit constants of a detector (heliocentric orbit.py:189-228; geocentric
 // orbit.py:112-139 with the given rotation rate and reference source); arguments validated by
 // the caller.
