@@ -176,6 +176,11 @@ template <int KIND>
 constexpr bool kGeo = (KIND & 1) != 0;
 template <int KIND>
 constexpr bool kDuty = (KIND & 2) != 0;
+// the waveform evaluated at the bin itself instead of interpolated between node table entries: a
+// mode's A, Psi, dPsi/du of a tile's bins are at nodes[0 .. 3 TILE - 1] (lane <-> bin), their
+// adjoints go to the same places of the array that holds the node gradients otherwise
+template <int KIND>
+constexpr bool kDirect = (KIND & 4) != 0;
 
 struct ModeG {
   double A, t;      // amplitude, t_f + t_c
@@ -250,12 +255,19 @@ template <int PREC, int KIND, int UPH = 0>
 __device__ inline void mode_geom(const DetectorDev& det, const double* __restrict__ mf,
                                  const double* __restrict__ n0, const BinPre& b, const RowC& rc, ModeG& g,
                                  double* __restrict__ uslot = nullptr) {
-  const double A0 = n0[0], dA0 = n0[1], P0 = n0[2], dP0 = n0[3];
-  const double A1 = n0[4], dA1 = n0[5], P1 = n0[6], dP1 = n0[7];
-  g.A = fma(b.hb1, A1 - A0, fma(b.hb2, dA0, fma(b.hb3, dA1, A0)));
-  const double dP = P1 - P0;
-  const double Psi = fma(b.hb1, dP, fma(b.hb2, dP0, fma(b.hb3, dP1, P0)));
-  g.t = mode_time(n0, b, rc.tc);
+  double Psi;
+  if constexpr (kDirect<KIND>) {
+    g.A = n0[0];
+    Psi = n0[TILE];
+    g.t = fma(b.he2, n0[2 * TILE], rc.tc);
+  } else {
+    const double A0 = n0[0], dA0 = n0[1], P0 = n0[2], dP0 = n0[3];
+    const double A1 = n0[4], dA1 = n0[5], P1 = n0[6], dP1 = n0[7];
+    g.A = fma(b.hb1, A1 - A0, fma(b.hb2, dA0, fma(b.hb3, dA1, A0)));
+    const double dP = P1 - P0;
+    Psi = fma(b.hb1, dP, fma(b.hb2, dP0, fma(b.hb3, dP1, P0)));
+    g.t = mode_time(n0, b, rc.tc);
+  }
   double w = 1.0;  // duty window at t (its slope is recomputed by the adjoint)
   if constexpr (kDuty<KIND>) {
     double dw;
@@ -610,6 +622,13 @@ __device__ inline void mode_adjoint(const DetectorDev& det, const double* __rest
     acc.iota = fma(tt.re, g.hm.re, fma(-tt.im, g.hm.im, acc.iota));  // += Re(tt hm)
   }
   acc.tc = fma(2.0 * b.pif, phib, acc.tc + tb);
+  if constexpr (kDirect<KIND>) {
+    double* a = const_cast<double*>(g0);
+    a[0] = Ab;
+    a[TILE] = phib;
+    a[2 * TILE] = tb * b.he2;
+    return;
+  }
   // intrinsic parameters through the node tables: weights of the eight node entries
   const double cA1 = Ab * b.hb1, cA0 = Ab - cA1, cdA0 = Ab * b.hb2, cdA1 = Ab * b.hb3;
   const double tP = tb * b.he1;
@@ -860,6 +879,12 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
         nstride = (size_t)nj * 4;
         gstride = (size_t)nj * 16;
         buf ^= 1;
+      } else if constexpr (kDirect<KIND>) {
+        if constexpr (kRecEarly) load_rec();
+        const size_t at = ((size_t)p * modes.n * n_tiles + tile) * (3 * TILE) + threadIdx.x;
+        nb = nodes + at;
+        gb = nodes_grad + at;
+        nstride = gstride = (size_t)n_tiles * (3 * TILE);
       } else {
         if constexpr (kRecEarly) load_rec();
         nb = nodes + (pbase + b.j) * 4;
@@ -978,6 +1003,7 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
 // plain instantiation takes (1) and those the duty one takes (0).
 // PAN: the context has panels: this kernel takes the tiles and rows that they leave, and adds to
 // the panel kernel's sums
+// KD bit 2: kDirect
 template <int PREC, bool GRAD, int KD, bool PAN>
 __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* __restrict__ dets, int n_det, int n_tiles,
                                               const double* __restrict__ bin_f, const int* __restrict__ bin_j,
@@ -996,8 +1022,8 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
   constexpr int NOUT = GRAD ? 1 + PES_N_PARAMS : 1;
   constexpr int CH = chunk_rows<GRAD>();  // 4x the rows without the gradient: 1.3% faster
   __shared__ double acc[TILE / 64][CH][NOUT];
-  __shared__ double stage_n[2 * MAX_MODES * NJ_STAGE * 4];
-  __shared__ typename std::conditional<GRAD, double[2 * MAX_MODES * NJ_STAGE * 16], double[1]>::type stage_g;
+  __shared__ typename std::conditional<kDirect<KD>, double[1], double[2 * MAX_MODES * NJ_STAGE * 4]>::type stage_n;
+  __shared__ typename std::conditional<GRAD && !kDirect<KD>, double[2 * MAX_MODES * NJ_STAGE * 16], double[1]>::type stage_g;
   int buf = 0;
   __shared__ int next_work;
   // each lane's own LDS column: forward-only, the tile's bin records [record entry][lane];
@@ -1064,11 +1090,11 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
       const int j0 = tile_jr[2 * tile], nj = tile_jr[2 * tile + 1];
 #define PES_TILE_ARGS                                                                                         \
   det, tile, f0, p0, p1, bin_f, bin_j, bin_s, bin_rec, tile_dd, pconst, nodes, nodes_grad, NNS, du, \
-      modes, lane, wave, &acc[0][0][0], j0, nj, stage_n, &stage_g[0], buf, off_bits, n_tiles, &lane_lds[0], db
+      modes, lane, wave, &acc[0][0][0], j0, nj, &stage_n[0], &stage_g[0], buf, off_bits, n_tiles, &lane_lds[0], db
       // the host's tile ranges give this launch detectors of one orbit kind (KD bit 0), all
       // duty-cycled or none (bit 1)
-      if (nj <= NJ_STAGE)
-        tile_rows<PREC, GRAD, KD, true, PAN>(PES_TILE_ARGS);
+      if (!kDirect<KD> && nj <= NJ_STAGE)
+        tile_rows<PREC, GRAD, KD, !kDirect<KD>, PAN>(PES_TILE_ARGS);
       else
         tile_rows<PREC, GRAD, KD, false, PAN>(PES_TILE_ARGS);
 #undef PES_TILE_ARGS

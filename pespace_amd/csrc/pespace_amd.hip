@@ -123,8 +123,8 @@ __global__ __launch_bounds__(192) void k_setup(const double* __restrict__ params
     double* su = setup + (size_t)p * N_SETUP * 5;
 #pragma unroll
     for (int i = 0; i < N_SETUP; ++i) {
-      if (k == 0) su[i * 5] = ph.c[i].v;
-      su[i * 5 + 1 + k] = ph.c[i].d[0];
+      if (k == 0) su[i] = ph.c[i].v;
+      su[(1 + k) * N_SETUP + i] = ph.c[i].d[0];
     }
     if (k != 0) return;
     double* pc = pconst + (size_t)p * PC_STRIDE;
@@ -197,12 +197,32 @@ __global__ __launch_bounds__(192) void k_setup(const double* __restrict__ params
   mf[MF_DFPR] = dFp.re; mf[MF_DFPI] = dFp.im; mf[MF_DFCR] = dFc.re; mf[MF_DFCI] = dFc.im;
 }
 
+// the powers of n frequencies (t[0 .. n - 1]) that node_eval.hpp takes, once per context
+__global__ __launch_bounds__(128) void k_fpow(int n, double* __restrict__ t) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= n) return;
+  const double f = t[j], c = cbrt(f), ic = 1.0 / c;
+  t[n + j] = c;
+  t[2 * (size_t)n + j] = ic;
+  t[3 * (size_t)n + j] = log(f);
+  t[4 * (size_t)n + j] = ic * ic * ic * sqrt(ic);
+}
+
 // ---- k_nodes ---------------------------------------------------------------------------
 // node table: [P][n_modes][NNS][4] = (A, dA/du, Psi, dPsi/du); NNS = n_nodes + 1 (padding)
 // grad table: [P][n_modes][NNS][16] = d/dtheta_i of the same four, i = Mc, q, chi1, chi2
-template <bool GRAD>
-__global__ __launch_bounds__(128) void k_nodes(const double* __restrict__ setup, int P, ModeList modes, int n_nodes, double u0, double du,
-                        const double* __restrict__ node_f, double* __restrict__ nodes,
+// OUT: NODES_VALUES the node table; NODES_GRAD both; NODES_DIRECT, for the fused kernel of a context
+// that is evaluated at every bin (kDirect), A, Psi and dPsi/du alone: [P][n_modes][n_tiles][3][TILE].
+// The values come from tabulated powers of the frequency (node_eval.hpp): 4096 rows of 1024 nodes 96 ->
+// 46 us, bound by the instructions of the ringdown's elementary functions and the table's stores.
+enum NodeOut { NODES_VALUES, NODES_GRAD, NODES_DIRECT };
+// where a (row, mode)'s stretch of a tile starts in a [P][n_modes][n_tiles][3][TILE] array
+__host__ __device__ inline size_t direct_at(size_t row_mode, int tile, int n_tiles) {
+  return (row_mode * n_tiles + tile) * (3 * TILE);
+}
+template <int OUT>
+__global__ __launch_bounds__(128) void k_nodes(const double* __restrict__ setup, int P, ModeList modes, int n_nodes,
+                        const double* __restrict__ fpow, double* __restrict__ nodes,
                         double* __restrict__ nodes_grad) {
   int jn = blockIdx.x * blockDim.x + threadIdx.x;
   int pm = blockIdx.y;
@@ -210,49 +230,45 @@ __global__ __launch_bounds__(128) void k_nodes(const double* __restrict__ setup,
   const int NNS = n_nodes + 1;
   if (jn >= NNS || p >= P) return;
   size_t row = ((size_t)p * modes.n + mi) * NNS + jn;
+  if (OUT == NODES_DIRECT && jn == n_nodes) return;
   if (jn == n_nodes) {  // padding node (read as the right end of the last direct-mode bin)
     for (int k = 0; k < 4; ++k) nodes[row * 4 + k] = 0.0;
-    if (GRAD)
+    if (OUT == NODES_GRAD)
       for (int k = 0; k < 16; ++k) nodes_grad[row * 16 + k] = 0.0;
     return;
   }
-  double f = node_f ? node_f[jn] : exp(u0 + du * (double)jn);
+  const FreqPow fq = load_fpow(fpow, n_nodes, jn);
   const double* su = setup + (size_t)p * N_SETUP * 5;
   int id = modes.id[mi];
-  if (!GRAD) {
-    typedef Dual<double, 1> S;
-    Phenom<S, SetupView<S>> ph{SetupView<S>{su}};
-    S Mf;
-    Mf.v = f * su[SU_MSEC * 5];
-    Mf.d[0] = Mf.v;  // dMf/du
-    S A, Ps;
-    ph.amp_phase(id, Mf, A, Ps);
-    nodes[row * 4 + 0] = A.v;
-    nodes[row * 4 + 1] = A.d[0];
-    nodes[row * 4 + 2] = Ps.v;
-    nodes[row * 4 + 3] = Ps.d[0];
-  } else {
+  double A, dA, P0, dP;
+  node_values(su, id, fq, A, dA, P0, dP);
+  if constexpr (OUT == NODES_DIRECT) {
+    double* o = nodes + direct_at(pm, jn / TILE, n_nodes / TILE) + jn % TILE;
+    o[0] = A;
+    o[TILE] = P0;
+    o[2 * TILE] = dP;
+    return;
+  }
+  double2* out = reinterpret_cast<double2*>(nodes + row * 4);
+  out[0] = make_double2(A, dA);
+  out[1] = make_double2(P0, dP);
+  if constexpr (OUT == NODES_GRAD) {
     typedef Dual<double, 1> D1;
     typedef Dual<D1, 4> S;
     Phenom<S, SetupView<S>> ph{SetupView<S>{su}};
     S Mf;
-    Mf.v.v = f * su[SU_MSEC * 5];
+    Mf.v.v = fq.f * su[SU_MSEC];
     Mf.v.d[0] = Mf.v.v;
     for (int k = 0; k < 4; ++k) {
-      Mf.d[k].v = f * su[SU_MSEC * 5 + 1 + k];
+      Mf.d[k].v = fq.f * su[(1 + k) * N_SETUP + SU_MSEC];
       Mf.d[k].d[0] = Mf.d[k].v;
     }
-    S A, Ps;
-    ph.amp_phase(id, Mf, A, Ps);
-    nodes[row * 4 + 0] = A.v.v;
-    nodes[row * 4 + 1] = A.v.d[0];
-    nodes[row * 4 + 2] = Ps.v.v;
-    nodes[row * 4 + 3] = Ps.v.d[0];
+    S At, Ps;
+    ph.amp_phase(id, Mf, At, Ps);
+    double2* og = reinterpret_cast<double2*>(nodes_grad + row * 16);
     for (int k = 0; k < 4; ++k) {
-      nodes_grad[row * 16 + k * 4 + 0] = A.d[k].v;
-      nodes_grad[row * 16 + k * 4 + 1] = A.d[k].d[0];
-      nodes_grad[row * 16 + k * 4 + 2] = Ps.d[k].v;
-      nodes_grad[row * 16 + k * 4 + 3] = Ps.d[k].d[0];
+      og[2 * k] = make_double2(At.d[k].v, At.d[k].d[0]);
+      og[2 * k + 1] = make_double2(Ps.d[k].v, Ps.d[k].d[0]);
     }
   }
 }
@@ -298,6 +314,52 @@ struct BinData {
 #include "hotpath.hpp"
 #ifndef PES_LNL_FWD_UNIT
 #include "panel.hpp"
+
+// ---- k_direct_grad, k_direct_sums: the gradient in Mc, q, chi1, chi2 of a context evaluated at every bin
+// The fused kernel leaves the adjoints of A, Psi and dPsi/du of every (row, mode, bin) at or below
+// the mode's cut in adj [P][n_modes][n_tiles][3][TILE].  k_direct_grad: one block per (tile, mode, row),
+// node_adjoint at each bin and the sum over the tile: sums [n_tiles][n_modes][4][P].  48 B move per (row,
+// mode, bin), against 320 for the waveform's gradient written to a table and read back, which is what
+// bound this path: 2048 rows, 16384 bins and the 22 mode 2210 + 1880 us through the tables, now 260
+// (k_nodes) + 1270 (k_lnl) + 520.  One tile per block: a block that loops over tiles keeps the
+// loop-invariant constants of the elementary functions in registers and runs one wave per SIMD (2240).
+__global__ __launch_bounds__(TILE) void k_direct_grad(const double* __restrict__ setup,
+                                                      const double* __restrict__ pconst,
+                                                      const double* __restrict__ fpow, int n_tiles,
+                                                      const double* __restrict__ adj, ModeList modes, int P,
+                                                      double* __restrict__ sums) {
+  __shared__ double red[TILE / 64][4];
+  const int mi = blockIdx.x / n_tiles, tile = blockIdx.x % n_tiles, p = blockIdx.y;
+  const double* pc = pconst + (size_t)p * PC_STRIDE;
+  const FreqPow q = load_fpow(fpow, (size_t)n_tiles * TILE, (size_t)tile * TILE + threadIdx.x);
+  const double* a = adj + direct_at((size_t)p * modes.n + mi, tile, n_tiles) + threadIdx.x;
+  const double wA = a[0], wP = a[TILE], wD = a[2 * TILE];  // not used above the cut, where adj holds nothing
+  double g[4] = {0.0, 0.0, 0.0, 0.0};
+  if (pc[PC_VALID] != 0.0 && q.f <= pc[PC_MODE + mi * PC_MODE_STRIDE + MF_CUT]) {
+    node_adjoint(setup + (size_t)p * (N_SETUP * 5), modes.id[mi], q, wA, wP, wD, g);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const double v = wave_sum(g[k]);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < 4) {
+    const int k = threadIdx.x;
+    sums[(((size_t)tile * modes.n + mi) * 4 + k) * P + p] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+  }
+}
+// the tiles and modes of each group, in order: the group's partial sums of the four parameters
+__global__ __launch_bounds__(256) void k_direct_sums(const double* __restrict__ sums, int n_modes, int P,
+                                                     const int* __restrict__ grp, int n_groups,
+                                                     double* __restrict__ partial) {
+  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (size_t)n_groups * 4 * P) return;
+  const int p = (int)(idx % P), k = (int)(idx / P % 4), g = (int)(idx / ((size_t)P * 4));
+  double s = 0.0;
+  for (int i = grp[g] * n_modes; i < grp[g + 1] * n_modes; ++i) s += sums[((size_t)i * 4 + k) * P + p];
+  partial[((size_t)g * (1 + PES_N_PARAMS) + 1 + k) * P + p] = s;
+}
 #endif
 
 #ifndef PES_LNL_FWD_UNIT
@@ -1098,8 +1160,8 @@ hipError_t pes::launch_lnl_fwd(int precision, int kd, int grid, hipStream_t st, 
   // lnL alone is the FP64 forward in every precision mode (the modes differ in the adjoint only)
   (void)precision;
 #define PES_LNL_FWD(KD)                                                                                     \
-  if (dbits)                                                                                                \
-    hipLaunchKernelGGL((k_lnl<0, false, KD, true>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES);          \
+  if (dbits && !kDirect<KD>)                                                                                \
+    hipLaunchKernelGGL((k_lnl<0, false, KD, !kDirect<KD>>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES);          \
   else                                                                                                      \
     hipLaunchKernelGGL((k_lnl<0, false, KD, false>), dim3(grid), dim3(TILE), 0, st, PES_LNL_NAMES);         \
   break;
@@ -1107,7 +1169,9 @@ hipError_t pes::launch_lnl_fwd(int precision, int kd, int grid, hipStream_t st, 
     case 0: PES_LNL_FWD(0)
     case 1: PES_LNL_FWD(1)
     case 2: PES_LNL_FWD(2)
-    default: PES_LNL_FWD(3)
+    case 3: PES_LNL_FWD(3)
+    case 4: PES_LNL_FWD(4)
+    default: PES_LNL_FWD(5)
   }
 #undef PES_LNL_FWD
   return hipGetLastError();
@@ -1123,6 +1187,10 @@ struct pes_context {
   double f_node_min = 0.0, f_node_max = 0.0, u0 = 0.0, du = 1.0;
   bool finalized = false;
   bool any_duty = false;  // a detector has a duty cycle (selects the duty-window kernel variants)
+  // lnL through the direct variant of the fused kernel (kDirect) and k_direct_grad: the waveform is
+  // evaluated at every bin, and no detector has a duty cycle (the classification of its tiles reads
+  // the node tables).  2048 rows, 16384 bins, 22: lnL 1240 -> 780 us, with the gradient 4160 -> 2080
+  bool direct_lnl() const { return direct && !any_duty; }
   struct HostDet {
     DetectorDev d;
     std::vector<double> f, w, dre, dim;  // w, dre, dim: [3][n]
@@ -1136,7 +1204,7 @@ struct pes_context {
   int* d_bin_j = nullptr;
   double *d_tile_f0 = nullptr, *d_tile_dd = nullptr;  // first frequency and sum w |d|^2 per tile
   int* d_tile_jr = nullptr;  // per tile: first node index and number of node rows its bins use
-  double* d_node_f = nullptr;  // direct mode only
+  double* d_fpow = nullptr;  // [N_FPOW][n_nodes] the nodes' (direct mode: the bins') frequencies and their powers
   // scratch, grown on demand; while pinned (a captured HIP graph holds its pointers) it is
   // never reallocated and a call that would need more is rejected
   int cap_P = 0;
@@ -1399,6 +1467,7 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // What a batch is accounted for against the array: the layout of a batch whose tile groups all
 // hold tiles_per_group tiles, without the panels' flags
+constexpr size_t N_SETUP_ACC = N_SU_USED - 7;  // without the precomputed powers
 static size_t noalloc_account(const pes_context* ctx, int P, bool grad) {
   const size_t NNS = (size_t)ctx->n_nodes + 1, rows = (size_t)P, nm = (size_t)ctx->modes.n;
   TileRange r[MAX_TILE_RANGES];
@@ -1406,7 +1475,7 @@ static size_t noalloc_account(const pes_context* ctx, int P, bool grad) {
   size_t groups = 0;
   for (int i = 0; i < n; ++i)
     groups += (r[i].tile_end - r[i].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
-  size_t o = align256(N_WORK_COUNTERS * sizeof(int)) + align256(rows * N_SETUP * 5 * sizeof(double)) +
+  size_t o = align256(N_WORK_COUNTERS * sizeof(int)) + align256(rows * N_SETUP_ACC * 5 * sizeof(double)) +
              align256(rows * PC_STRIDE * sizeof(double)) + align256(rows * nm * NNS * 4 * sizeof(double));
   if (grad) o += align256(rows * nm * NNS * 16 * sizeof(double));
   o += align256(groups * (grad ? 1 + PES_N_PARAMS : 1) * rows * sizeof(double));
@@ -1422,7 +1491,8 @@ static size_t noalloc_layout(const pes_context* ctx, int P, bool grad, size_t of
   off[1] = o; o += align256(rows * N_SETUP * 5 * sizeof(double));          // setup
   off[2] = o; o += align256(rows * PC_STRIDE * sizeof(double));            // per-row constants
   off[3] = o; o += align256(rows * nm * NNS * 4 * sizeof(double));         // node tables
-  off[4] = o; if (grad) o += align256(rows * nm * NNS * 16 * sizeof(double));  // their gradients
+  // their gradients (direct: the waveform's adjoints)
+  off[4] = o; if (grad) o += align256(rows * nm * (ctx->direct_lnl() ? (size_t)ctx->n_nodes * 3 : NNS * 16) * sizeof(double));
   off[5] = o; o += align256((size_t)n_groups_of(ctx) * (grad ? 1 + PES_N_PARAMS : 1) * rows * sizeof(double));
   off[6] = o; if (ctx->any_duty) o += align256(rows * off_words_of(ctx) * sizeof(unsigned long long));  // off tiles
   off[7] = o; if (ctx->any_duty) o += align256((size_t)n_groups_of(ctx) * rows);  // work items: plain or duty
@@ -1662,7 +1732,20 @@ extern "C" int pes_context_finalize(pes_context* ctx) {
     HIP_TRY(hipMalloc(&ctx->d_tile_jr, 2 * (size_t)nt * sizeof(int)));
     HIP_TRY(hipMemcpy(ctx->d_tile_jr, tjr.data(), 2 * (size_t)nt * sizeof(int), hipMemcpyHostToDevice));
   }
-  if (ctx->direct) ctx->d_node_f = ctx->d_bin_f;
+  {
+    const int n = ctx->n_nodes;
+    HIP_TRY(hipMalloc(&ctx->d_fpow, (size_t)N_FPOW * n * sizeof(double)));
+    if (ctx->direct) {
+      HIP_TRY(hipMemcpy(ctx->d_fpow, ctx->d_bin_f, (size_t)n * sizeof(double), hipMemcpyDeviceToDevice));
+    } else {
+      std::vector<double> f(n);
+      for (int j = 0; j < n; ++j) f[j] = std::exp(ctx->u0 + ctx->du * (double)j);
+      HIP_TRY(hipMemcpy(ctx->d_fpow, f.data(), (size_t)n * sizeof(double), hipMemcpyHostToDevice));
+    }
+    hipLaunchKernelGGL(k_fpow, dim3((n + 127) / 128), dim3(128), 0, nullptr, n, ctx->d_fpow);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(nullptr));
+  }
   {
     int rc = build_panels(ctx, bf, bj);
     if (rc == PES_OK) rc = build_groups(ctx);
@@ -1684,6 +1767,7 @@ extern "C" void pes_context_destroy(pes_context* ctx) {
   free_dev(ctx->d_dets);
   free_dev(ctx->d_bin_f);
   free_dev(ctx->d_bin_s);
+  free_dev(ctx->d_fpow);
   free_dev(ctx->d_bin_j);
   free_dev(ctx->d_bin_rec);
   free_dev(ctx->d_tile_f0);
@@ -1785,7 +1869,9 @@ static int ensure_scratch(pes_context* ctx, int P, bool grad) {
   HIP_TRY(hipMalloc(&ctx->d_setup, (size_t)cap * N_SETUP * 5 * sizeof(double)));
   HIP_TRY(hipMalloc(&ctx->d_pconst, (size_t)cap * PC_STRIDE * sizeof(double)));
   HIP_TRY(hipMalloc(&ctx->d_nodes, (size_t)cap * ctx->modes.n * NNS * 4 * sizeof(double)));
-  if (g) HIP_TRY(hipMalloc(&ctx->d_nodes_grad, (size_t)cap * ctx->modes.n * NNS * 16 * sizeof(double)));
+  // (direct: the adjoints of three waveform values per bin)
+  const size_t per = ctx->direct_lnl() ? (size_t)ctx->n_nodes * 3 : NNS * 16;
+  if (g) HIP_TRY(hipMalloc(&ctx->d_nodes_grad, (size_t)cap * ctx->modes.n * per * sizeof(double)));
   if (ctx->any_duty)
     HIP_TRY(hipMalloc(&ctx->d_off_bits, (size_t)cap * off_words_of(ctx) * sizeof(unsigned long long)));
   if (ctx->pan.tile_pan)
@@ -1823,26 +1909,30 @@ static int check_batch_args(const pes_context* ctx, const double* d_params, int 
   return PES_OK;
 }
 
-// k_setup (which also zeroes the work counters) and k_nodes for P >= 1 rows
+// k_setup (which also zeroes the work counters) and k_nodes for P >= 1 rows; direct: the tables of
+// the direct fused kernel
 static int launch_setup_nodes(const pes_context* ctx, const BatchScratch& sc, const double* d_params, int P, bool grad,
-                              hipStream_t st) {
+                              bool direct, hipStream_t st) {
   const dim3 sg((P + SETUP_ROWS - 1) / SETUP_ROWS);
   hipLaunchKernelGGL(k_setup, sg, dim3(192), 0, st, d_params, P, ctx->modes, ctx->f_ref, sc.setup, sc.pconst,
                      sc.work_counter, ctx->bin_work.state);
   HIP_TRY(hipGetLastError());
   const int NNS = ctx->n_nodes + 1;
   dim3 g((NNS + 127) / 128, P * ctx->modes.n);
-  if (grad)
-    hipLaunchKernelGGL(k_nodes<true>, g, dim3(128), 0, st, sc.setup, P, ctx->modes, ctx->n_nodes, ctx->u0, ctx->du,
-                       ctx->d_node_f, sc.nodes, sc.nodes_grad);
+  if (direct)
+    hipLaunchKernelGGL(k_nodes<NODES_DIRECT>, g, dim3(128), 0, st, sc.setup, P, ctx->modes, ctx->n_nodes, ctx->d_fpow,
+                       sc.nodes, nullptr);
+  else if (grad)
+    hipLaunchKernelGGL(k_nodes<NODES_GRAD>, g, dim3(128), 0, st, sc.setup, P, ctx->modes, ctx->n_nodes, ctx->d_fpow,
+                       sc.nodes, sc.nodes_grad);
   else
-    hipLaunchKernelGGL(k_nodes<false>, g, dim3(128), 0, st, sc.setup, P, ctx->modes, ctx->n_nodes, ctx->u0, ctx->du,
-                       ctx->d_node_f, sc.nodes, nullptr);
+    hipLaunchKernelGGL(k_nodes<NODES_VALUES>, g, dim3(128), 0, st, sc.setup, P, ctx->modes, ctx->n_nodes, ctx->d_fpow,
+                       sc.nodes, nullptr);
   HIP_TRY(hipGetLastError());
   return PES_OK;
 }
 
-static int prepare(pes_context* ctx, const double* d_params, int P, bool grad, hipStream_t st) {
+static int prepare(pes_context* ctx, const double* d_params, int P, bool grad, hipStream_t st, bool direct = false) {
   int rc = check_batch_args(ctx, d_params, P);
   if (rc != PES_OK) return rc;
   HIP_TRY(hipSetDevice(ctx->device));
@@ -1850,7 +1940,7 @@ static int prepare(pes_context* ctx, const double* d_params, int P, bool grad, h
   if (rc != PES_OK) return rc;
   if (P == 0) return PES_OK;
   ++ctx->scratch_seq;
-  return launch_setup_nodes(ctx, context_scratch(ctx), d_params, P, grad, st);
+  return launch_setup_nodes(ctx, context_scratch(ctx), d_params, P, grad, direct, st);
 }
 
 // rows per work item of the fused kernel: the kernel's chunk, fewer when the grid has too few
@@ -1875,6 +1965,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   const int n_groups = n_groups_of(ctx);
   int grid = ctx->n_cu * ctx->blocks_per_cu;
   const bool panels = sc.dbits != nullptr;
+  const bool direct = ctx->direct_lnl();
   const bool fine = sc.fine && P < fine_rows(ctx);
   const int rows = rows_per_item(ctx, P, grad, grid, panels, fine);
   const int n_chunks = (P + rows - 1) / rows;
@@ -1965,7 +2056,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
       // pass 0: the plain instantiation (all items of a plain range; the plateau items of a
       // duty-cycled one), pass 1: the duty instantiation (the other items); both for the range's
       // orbit kind only
-      const int kd = ranges[r].kind | (pass == 1 ? 2 : 0);
+      const int kd = ranges[r].kind | (pass == 1 ? 2 : 0) | (direct ? 4 : 0);
       const unsigned char* items = ranges[r].duty ? items_buf : nullptr;
       int* counter = sc.work_counter + (pass == 0 ? r : MAX_TILE_RANGES + r);
 #define PES_LNL_ARGS                                                                                         \
@@ -1974,8 +2065,8 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
       ctx->modes, P, rows, ctx->d_tile_jr, tile_begin, group_offset, counter, part_bin,                       \
       sc.off_bits, items, ctx->pan.tile_pan, ctx->bin_work, r, group_offset, sc.dbits, fine ? 1 : 0
 #define PES_LNL_GRAD(PR, KD)                                                                                  \
-  if (panels)                                                                                                \
-    hipLaunchKernelGGL((k_lnl<PR, true, KD, true>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS);          \
+  if (panels && !kDirect<KD>)                                                                                \
+    hipLaunchKernelGGL((k_lnl<PR, true, KD, !kDirect<KD>>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS);          \
   else                                                                                                       \
     hipLaunchKernelGGL((k_lnl<PR, true, KD, false>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS)
       if (!grad) {
@@ -1985,14 +2076,18 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
           case 0: PES_LNL_GRAD(0, 0); break;
           case 1: PES_LNL_GRAD(0, 1); break;
           case 2: PES_LNL_GRAD(0, 2); break;
-          default: PES_LNL_GRAD(0, 3); break;
+          case 3: PES_LNL_GRAD(0, 3); break;
+          case 4: PES_LNL_GRAD(0, 4); break;
+          default: PES_LNL_GRAD(0, 5); break;
         }
       } else {
         switch (kd) {
           case 0: PES_LNL_GRAD(1, 0); break;
           case 1: PES_LNL_GRAD(1, 1); break;
           case 2: PES_LNL_GRAD(1, 2); break;
-          default: PES_LNL_GRAD(1, 3); break;
+          case 3: PES_LNL_GRAD(1, 3); break;
+          case 4: PES_LNL_GRAD(1, 4); break;
+          default: PES_LNL_GRAD(1, 5); break;
         }
       }
 #undef PES_LNL_GRAD
@@ -2011,6 +2106,15 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     hipLaunchKernelGGL(k_group_sums, dim3((unsigned)(((size_t)n_groups * nout * P + 255) / 256)), dim3(256), 0, st,
                        ctx->d_groups, n_groups, P, nout, panels ? part_pan : nullptr, part_bin, ctx->pan.tile_pan,
                        ctx->bin_work, sc.partial);
+    HIP_TRY(hipGetLastError());
+  }
+  if (direct && grad) {
+    // the tiles' sums go where the node values were: the fused kernel is done with them
+    hipLaunchKernelGGL(k_direct_grad, dim3(ctx->n_tiles * ctx->modes.n, P), dim3(TILE), 0, st,
+                       sc.setup, sc.pconst, ctx->d_fpow, ctx->n_tiles, sc.nodes_grad, ctx->modes, P, sc.nodes);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_direct_sums, dim3((unsigned)(((size_t)n_groups * 4 * P + 255) / 256)), dim3(256), 0, st,
+                       sc.nodes, ctx->modes.n, P, ctx->d_groups, n_groups, sc.partial);
     HIP_TRY(hipGetLastError());
   }
 #define PES_REDUCE(RB)                                                                                        \
@@ -2071,7 +2175,7 @@ extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, i
     sc.dbits = ctx->pan.tile_pan ? reinterpret_cast<unsigned long long*>(base + off[8]) : nullptr;
     sc.fine = nullptr;
     const double* params = d_params + (size_t)p0 * PES_N_PARAMS;
-    rc = launch_setup_nodes(ctx, sc, params, n, grad, st);
+    rc = launch_setup_nodes(ctx, sc, params, n, grad, ctx->direct_lnl(), st);
     if (rc == PES_OK)
       rc = launch_lnl_reduce(ctx, sc, n, d_lnl + p0, grad ? d_grad + (size_t)p0 * PES_N_PARAMS : nullptr, precision, st,
                              false);
@@ -2087,7 +2191,7 @@ extern "C" int pes_lnl_batch(pes_context* ctx, const double* d_params, int P, do
   if (P > 0 && !d_lnl) return fail(PES_ERR_INVALID, "lnl output is NULL");
   hipStream_t st = (hipStream_t)stream;
   bool grad = d_grad != nullptr;
-  int rc = prepare(ctx, d_params, P, grad, st);
+  int rc = prepare(ctx, d_params, P, grad, st, ctx->direct_lnl());
   if (rc != PES_OK || P == 0) return rc;
   return launch_lnl_reduce(ctx, context_scratch(ctx), P, d_lnl, d_grad, precision, st, ctx->profiling);
 }

@@ -141,34 +141,28 @@ enum SetupId {
   SU_S1, SU_S2, SU_S3, SU_S4, SU_B1, SU_B2, SU_B3, SU_AL1, SU_AL2, SU_AL3, SU_AL4, SU_AL5,
   SU_C1INT, SU_C2INT, SU_C1MRD, SU_C2MRD, SU_T0, SU_PHIREF0, SU_MFREF,
   SU_FRD21, SU_FRD33, SU_FRD32, SU_FRD44, SU_FRD43,
-  N_SETUP
+  // 1 / eta, sqrt(2 eta / 3) pi^(-1/6) AMPSCALE and its logarithm, and powers and logarithm of the
+  // mass in seconds
+  SU_IETA, SU_PRE, SU_LNPRE, SU_M13, SU_IM13, SU_LNM, SU_M76,
+  N_SU_USED,
+  N_SETUP = (N_SU_USED + 1) & ~1  // even: rows of whole 16-byte pieces
 };
 
 // Coefficient store of Phenom: an array (written by phenom_setup) or, in the node kernels,
-// SetupView: a read-only view of one row of the setup table [N_SETUP][5] (value and d/dtheta
-// for Mc, q, chi1, chi2), building each coefficient as the requested dual on access, so the
+// SetupView: a read-only view of one row of the setup table [5][N_SETUP] (values, then d/dtheta
+// for Mc, q, chi1, chi2: a kernel that needs the values alone reads them from one stretch), building each coefficient as the requested dual on access, so the
 // kernels hold no per-lane copy of the ~60 coefficients.
 template <class S>
 struct SetupView;
-template <>
-struct SetupView<Dual<double, 1>> {
-  const double* su;
-  PES_HD Dual<double, 1> operator[](int i) const {
-    Dual<double, 1> r;
-    r.v = su[i * 5];
-    r.d[0] = 0.0;
-    return r;
-  }
-};
 template <>
 struct SetupView<Dual<Dual<double, 1>, 4>> {
   const double* su;
   PES_HD Dual<Dual<double, 1>, 4> operator[](int i) const {
     Dual<Dual<double, 1>, 4> r;
-    r.v.v = su[i * 5];
+    r.v.v = su[i];
     r.v.d[0] = 0.0;
     for (int k = 0; k < 4; ++k) {
-      r.d[k].v = su[i * 5 + 1 + k];
+      r.d[k].v = su[(1 + k) * N_SETUP + i];
       r.d[k].d[0] = 0.0;
     }
     return r;
@@ -381,6 +375,13 @@ PES_HD void phenom_setup(Phenom<S>& P, const S& Mc, const S& q, const S& chi1_in
   for (int i = 0; i < N_SETUP; ++i) c[i] = lift<S>(0.0);
   c[SU_MSEC] = M * MTSUN_SI;
   c[SU_AMPSCALE] = (M * MRSUN_SI) * (M * MTSUN_SI);
+  c[SU_IETA] = 1.0 / eta;
+  c[SU_PRE] = dsqrt(eta * (2.0 / 3.0)) * c[SU_AMPSCALE] * pow(PI, -1.0 / 6.0);
+  c[SU_LNPRE] = dlog(c[SU_PRE]);
+  c[SU_M13] = dcbrt(c[SU_MSEC]);
+  c[SU_IM13] = 1.0 / c[SU_M13];
+  c[SU_LNM] = dlog(c[SU_MSEC]);
+  c[SU_M76] = c[SU_IM13] * c[SU_IM13] * c[SU_IM13] * dsqrt(c[SU_IM13]);
   c[SU_ETA] = eta;
   c[SU_DELTA] = delta;
   c[SU_CHIS] = chis;
@@ -587,3 +588,5 @@ PES_HD S sw_y(int l, int m, const S& theta) {
 }
 
 }  // namespace pes
+
+#include "node_eval.hpp"
