@@ -161,6 +161,14 @@ int pes_links(pes_context* ctx, int det, const double* d_params, int P, double* 
 int pes_links_from_waveform(pes_context* ctx, int det, int n_modes, const double* d_wf, double lam, double beta,
                             double psi, double tc, double* d_out, void* stream);
 
+/* The same with every mode's arrays read where they lie: host arrays of n_modes <=
+ * PES_CONTAINER_MODES device pointers, d_plus[m] and d_cross[m] [n_bins][2] (re, im), d_tf[m]
+ * [n_bins]. */
+#define PES_CONTAINER_MODES 8
+int pes_links_from_modes(pes_context* ctx, int det, int n_modes, const double* const* d_plus,
+                         const double* const* d_cross, const double* const* d_tf, double lam, double beta, double psi,
+                         double tc, double* d_out, void* stream);
+
 /* TDI combination of detector det from single links: device links [P][6][n_bins][2] ->
  * device out [P][3][n_bins][2] (A, E, T = (X+Y+Z)/sqrt3 or X, Y, Z, the reference's own
  * formulas).  Replaces update_tdi_response (tdi.py:1705-1793) and the JAX twin's
@@ -190,6 +198,12 @@ int pes_td_links(int orbit_kind, double arm_length_m, double rotation_initial, d
                  double omega_rotation, double lambda_ref, double beta_ref, const double* d_hp, const double* d_hc,
                  double wave_t0, double wave_dt, int wave_n, double lam, double beta, double psi, double t0, double dt,
                  int n, double* d_out, void* stream);
+/* pes_td_links with h+ and hx wave_stride doubles from sample to sample (2: columns of one
+ * [wave_n][2] array). */
+int pes_td_links_strided(int orbit_kind, double arm_length_m, double rotation_initial, double revolution_initial,
+                         double omega_rotation, double lambda_ref, double beta_ref, const double* d_hp,
+                         const double* d_hc, int wave_stride, double wave_t0, double wave_dt, int wave_n, double lam,
+                         double beta, double psi, double t0, double dt, int n, double* d_out, void* stream);
 int pes_td_tdi_added_samples(double arm_length_m, double dt, int tdi_generation);
 int pes_td_tdi(double arm_length_m, double dt, int tdi_generation, int orthogonal, const double* d_links, int n_ext,
                double* d_out, void* stream);

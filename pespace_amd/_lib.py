@@ -15,6 +15,7 @@ _lib = None
 
 c_double_p = ctypes.POINTER(ctypes.c_double)
 c_int_p = ctypes.POINTER(ctypes.c_int)
+c_void_pp = ctypes.POINTER(ctypes.c_void_p)
 
 # (name, restype, argtypes) for every symbol include/pespace_amd.h declares
 SIGNATURES = [
@@ -53,6 +54,9 @@ SIGNATURES = [
     ("pes_links_from_waveform", ctypes.c_int,
      [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_double, ctypes.c_double,
       ctypes.c_double, ctypes.c_double, ctypes.c_void_p, ctypes.c_void_p]),
+    ("pes_links_from_modes", ctypes.c_int,
+     [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, c_void_pp, c_void_pp, c_void_pp, ctypes.c_double, ctypes.c_double,
+      ctypes.c_double, ctypes.c_double, ctypes.c_void_p, ctypes.c_void_p]),
     ("pes_tdi_from_links", ctypes.c_int,
      [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     ("pes_orbit_vectors", ctypes.c_int,
@@ -71,6 +75,11 @@ SIGNATURES = [
     ("pes_td_links", ctypes.c_int,
      [ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
       ctypes.c_double, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_double, ctypes.c_double, ctypes.c_int,
+      ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_int,
+      ctypes.c_void_p, ctypes.c_void_p]),
+    ("pes_td_links_strided", ctypes.c_int,
+     [ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+      ctypes.c_double, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_int,
       ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_int,
       ctypes.c_void_p, ctypes.c_void_p]),
     ("pes_td_tdi_added_samples", ctypes.c_int, [ctypes.c_double, ctypes.c_double, ctypes.c_int]),

@@ -304,9 +304,13 @@ class LikelihoodCore:
         out = torch.view_as_complex(out)
         return out[0] if squeeze else out
 
+    @staticmethod
+    def _container_modes(waveform):
+        return [waveform] if {"plus", "cross", "tf"} <= set(waveform.keys()) else list(waveform.values())
+
     def _container(self, det, waveform):
         n = self._n_bins[det]
-        modes = [waveform] if {"plus", "cross", "tf"} <= set(waveform.keys()) else list(waveform.values())
+        modes = self._container_modes(waveform)
         dev = torch.device(f"cuda:{self.device}")
         wf = torch.empty(len(modes), n, 5, dtype=torch.float64, device=dev)
         for i, m in enumerate(modes):
@@ -327,8 +331,23 @@ class LikelihoodCore:
     def links_from_container(self, det, waveform, lam, beta, psi, tc):
         """Complex (6, N) single links of detector det for a reference-style container."""
         self._build()
+        n = self._n_bins[det]
+        dev = torch.device(f"cuda:{self.device}")
+        modes = self._container_modes(waveform)
+        arrays = [[m[k] for m in modes] for k in ("plus", "cross", "tf")]
+        # up to eight modes of contiguous device arrays are read where they lie; anything else (numpy,
+        # other types, strides or devices) is gathered into one array first
+        if len(modes) <= 8 and all(
+                type(a) is torch.Tensor and a.device == dev and a.shape == (n,) and a.is_contiguous()
+                and a.dtype == t and not a.is_conj() and not a.is_neg()
+                for row, t in zip(arrays, (torch.complex128, torch.complex128, torch.float64)) for a in row):
+            ptrs = [(ctypes.c_void_p * len(modes))(*[a.data_ptr() for a in row]) for row in arrays]
+            out = torch.empty(6, n, 2, dtype=torch.float64, device=dev)
+            check(lib().pes_links_from_modes(self._ctx, det, len(modes), *ptrs, float(lam), float(beta), float(psi),
+                                             float(tc), out.data_ptr(), torch.cuda.current_stream(dev).cuda_stream))
+            return torch.view_as_complex(out)
         wf, n_modes, dev = self._container(det, waveform)
-        out = torch.empty(6, self._n_bins[det], 2, dtype=torch.float64, device=dev)
+        out = torch.empty(6, n, 2, dtype=torch.float64, device=dev)
         check(lib().pes_links_from_waveform(self._ctx, det, n_modes, wf.data_ptr(), float(lam), float(beta),
                                             float(psi), float(tc), out.data_ptr(),
                                             torch.cuda.current_stream(dev).cuda_stream))
@@ -392,8 +411,13 @@ def td_links(orbit_kind, arm_length, rotation_initial, revolution_initial, hp, h
     (linearly interpolated, zero outside the samples), with the constellation at each sample
     time (the reference's commented TDResponseModelCornish2003, antenna.py:681-800)."""
     dev = hp.device if isinstance(hp, torch.Tensor) and hp.is_cuda else _device(device)
-    hp = torch.as_tensor(hp, dtype=torch.float64, device=dev).reshape(-1).contiguous()
-    hc = torch.as_tensor(hc, dtype=torch.float64, device=dev).reshape(-1).contiguous()
+    hp = torch.as_tensor(hp, dtype=torch.float64, device=dev).reshape(-1)
+    hc = torch.as_tensor(hc, dtype=torch.float64, device=dev).reshape(-1)
+    # the two columns of one (n, 2) array are read where they lie (a copy of a year of samples costs a
+    # third of the links); other strides are gathered first
+    stride = 2 if hp.stride(0) == hc.stride(0) == 2 and not (hp.is_neg() or hc.is_neg()) else 1
+    if stride == 1:
+        hp, hc = hp.contiguous(), hc.contiguous()
     if hp.numel() != hc.numel():
         raise ValueError(f"h+ and hx differ in length ({hp.numel()} vs {hc.numel()})")
     n = int(n)
@@ -401,10 +425,11 @@ def td_links(orbit_kind, arm_length, rotation_initial, revolution_initial, hp, h
         out = torch.empty(6, n, dtype=torch.float64, device=dev)
     else:
         LikelihoodCore._check_out(out, "out", (6, n), dev)
-    check(lib().pes_td_links(int(orbit_kind), float(arm_length), float(rotation_initial), float(revolution_initial),
-                             float(omega_rotation), float(lambda_ref), float(beta_ref), hp.data_ptr(), hc.data_ptr(),
-                             float(wave_t0), float(wave_dt), hp.numel(), float(lam), float(beta), float(psi),
-                             float(t0), float(dt), n, out.data_ptr(), torch.cuda.current_stream(dev).cuda_stream))
+    check(lib().pes_td_links_strided(int(orbit_kind), float(arm_length), float(rotation_initial),
+                                     float(revolution_initial), float(omega_rotation), float(lambda_ref),
+                                     float(beta_ref), hp.data_ptr(), hc.data_ptr(), stride, float(wave_t0),
+                                     float(wave_dt), hp.numel(), float(lam), float(beta), float(psi), float(t0),
+                                     float(dt), n, out.data_ptr(), torch.cuda.current_stream(dev).cuda_stream))
     return out
 
 

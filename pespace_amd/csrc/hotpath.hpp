@@ -250,13 +250,17 @@ __device__ inline bool interval_on(const DetectorDev& det, const double* __restr
 
 // UPH: 0 forms the unit phasor u; 1 forms it and stores it at uslot (this lane's LDS slot for
 // the mode: the gradient kernel's forward pass); 2 takes it from uslot (the adjoint's
-// recompute, which then needs neither the phase nor k.x0)
+// recompute, which then needs neither the phase nor k.x0); 3 a supplied waveform instead of node
+// entries: n0 holds h+ (re, im), hx (re, im) and t_f, and t may be far from the data (both reduction
+// steps for the orbit's angles)
 template <int PREC, int KIND, int UPH = 0>
 __device__ inline void mode_geom(const DetectorDev& det, const double* __restrict__ mf,
                                  const double* __restrict__ n0, const BinPre& b, const RowC& rc, ModeG& g,
                                  double* __restrict__ uslot = nullptr) {
-  double Psi;
-  if constexpr (kDirect<KIND>) {
+  double Psi = 0.0;
+  if constexpr (UPH == 3) {
+    g.t = n0[4] + rc.tc;
+  } else if constexpr (kDirect<KIND>) {
     g.A = n0[0];
     Psi = n0[TILE];
     g.t = fma(b.he2, n0[2 * TILE], rc.tc);
@@ -273,7 +277,10 @@ __device__ inline void mode_geom(const DetectorDev& det, const double* __restric
     double dw;
     duty_window(det, g.t, w, dw);
   }
-  sincos_tab_s(fma(kOmegaYear, g.t, det.rev0), &g.sa, &g.ca);
+  if constexpr (UPH == 3)
+    sincos_tab_sum(0.0, 0, fma(kOmegaYear, g.t, det.rev0), &g.sa, &g.ca);
+  else
+    sincos_tab_s(fma(kOmegaYear, g.t, det.rev0), &g.sa, &g.ca);
   const double sa = g.sa, ca = g.ca;
   g.kx0 = AU_SEC * fma(rc.k.x, ca, rc.k.y * sa);
   double kx_0, kx_1;
@@ -294,7 +301,10 @@ __device__ inline void mode_geom(const DetectorDev& det, const double* __restric
     kx_1 = fma(det.hsk[1], kU, det.hck[1] * kV);
   } else {
     double s1, c1;
-    sincos_tab_s(fma(det.omega_rot, g.t, det.rot0), &s1, &c1);
+    if constexpr (UPH == 3)
+      sincos_tab_sum(0.0, 0, fma(det.omega_rot, g.t, det.rot0), &s1, &c1);
+    else
+      sincos_tab_s(fma(det.omega_rot, g.t, det.rot0), &s1, &c1);
     const double cr = -0.5, sr = 0.5 * SQRT3;  // rotation by 2 pi / 3
     g.al[0] = s1;
     g.be[0] = c1;
@@ -348,6 +358,12 @@ __device__ inline void mode_geom(const DetectorDev& det, const double* __restric
     }
     g.u = {cp, -sp};
     if constexpr (UPH == 1) *reinterpret_cast<double2*>(uslot) = make_double2(cp, -sp);
+  }
+  if constexpr (UPH == 3) {
+    const Cx u = kDuty<KIND> ? scale(g.u, w) : g.u;
+    g.hp = mul(u, Cx{n0[0], n0[1]});
+    g.hc = mul(u, Cx{2.0 * n0[2], 2.0 * n0[3]});
+    return;
   }
   g.hm = scale(g.u, kDuty<KIND> ? g.A * w : g.A);
   g.hp = mul(Cx{mf[MF_FPR], mf[MF_FPI]}, g.hm);

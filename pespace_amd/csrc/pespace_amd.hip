@@ -658,27 +658,79 @@ __global__ __launch_bounds__(128) void k_response_container(const DetectorDev* _
 // combination (tdi.py:1705-1793, the JAX twin _tdi_jax.py:70-102), and the constellation
 // vectors (orbit.py:260-322, 363-419) ----------------------------------------------------------
 // links: [6][n_bins][2] in the order 12, 21, 23, 32, 31, 13 (antenna.py:24-31)
+// The modes' arrays: packed [n_modes][n_bins][5] at wf, or (wf null) where the caller has them, h+ and
+// hx [n_bins][2] and t_f [n_bins] per mode.
+struct WaveIn {
+  const double* wf;
+  const double *hp[PES_CONTAINER_MODES], *hc[PES_CONTAINER_MODES], *tf[PES_CONTAINER_MODES];
+};
+// The geometry, the pair phasors and the sincs are those of the fused kernel (a table sincos instead of
+// twelve library sines per mode): 6 modes of 300k bins 69 -> 24 us.  Bins whose angles the
+// table's reductions are not made for (t or tc beyond ~1e9 years, f beyond ~100 Hz, or not finite) take
+// add_mode_links.
+template <int KIND>
 __global__ __launch_bounds__(128) void k_links_container(const DetectorDev* __restrict__ dets, int det_i,
-                                                         const double* __restrict__ bin_f, int n_modes,
-                                                         const double* __restrict__ wf, Extrinsic ex,
-                                                         double* __restrict__ out) {
+                                                         const double* __restrict__ bin_f, int n_modes, WaveIn w,
+                                                         Extrinsic ex, double* __restrict__ out) {
+  trig_table_load();
   const DetectorDev det = dets[det_i];
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= det.n_bins) return;
-  double f = bin_f[det.bin_offset + k];
-  Cplx etc;
-  sincos(-2.0 * PI * f * ex.tc, &etc.im, &etc.re);
-  Links L = {};
+  const double f = bin_f[det.bin_offset + k];
+  BinPre b;
+  b.f = f;
+  b.pif = PI * f;
+  b.xL = PI * f * det.L;
+  sincos_d(b.xL, &b.sxL, &b.cxL);
+  RowC rc;
+  rc.tc = ex.tc;
+  rc.p = {ex.p.x, ex.p.y, ex.p.z};
+  rc.q = {ex.q.x, ex.q.y, ex.q.z};
+  rc.k = {ex.k.x, ex.k.y, ex.k.z};
+  tab_reduce(2.0 * b.pif * rc.tc, rc.tc_r, rc.tc_k);
+  row_geo(det, rc);
+  const bool bin_ok = fabs(2.0 * b.pif * rc.tc) < 1e12 && fabs(b.xL) < 1e3 && fabs(b.pif) < 1e9;
+  LinksT S = {};   // the links without their common factor (-i xL) exp(-i xL)
+  Links slow = {};
   for (int m = 0; m < n_modes; ++m) {
-    const double* w = wf + ((size_t)m * det.n_bins + k) * 5;
-    Cplx hp = cmul({w[0], w[1]}, etc);
-    Cplx hc = cmul({w[2], w[3]}, etc);
-    add_mode_links(det, f, w[4] + ex.tc, hp, hc, ex.p, ex.q, ex.k, L);
+    double v[5];
+    if (w.wf) {
+      const double* q = w.wf + ((size_t)m * det.n_bins + k) * 5;
+#pragma unroll
+      for (int i = 0; i < 5; ++i) v[i] = q[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        v[i] = w.hp[m][2 * (size_t)k + i];
+        v[2 + i] = w.hc[m][2 * (size_t)k + i];
+      }
+      v[4] = w.tf[m][k];
+    }
+    const double t = v[4] + ex.tc;
+    if (bin_ok && fabs(kOmegaYear * t) < 1e10 && fabs(det.omega_rot * t) < 1e12) {
+      ModeG g;
+      mode_geom<0, KIND, 3>(det, nullptr, v, b, rc, g);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        PairV pv;
+        pair_eval<0>(det, b, g, a, pv);
+        const int lp = a == 0 ? 2 : (a == 1 ? 4 : 0), lm = lp + 1;
+        S.l[lp] = axpy(pv.sp, pv.C, S.l[lp]);
+        S.l[lm] = axpy(pv.sm, pv.C, S.l[lm]);
+      }
+    } else {
+      Cplx etc;
+      sincos(-2.0 * PI * f * ex.tc, &etc.im, &etc.re);
+      add_mode_links(det, f, t, cmul({v[0], v[1]}, etc), cmul({v[2], v[3]}, etc), ex.p, ex.q, ex.k, slow);
+    }
   }
-  const Cplx l[6] = {L.l12, L.l21, L.l23, L.l32, L.l31, L.l13};
+  const Cx cf = {-b.xL * b.sxL, -b.xL * b.cxL};
+  const Cplx l[6] = {slow.l12, slow.l21, slow.l23, slow.l32, slow.l31, slow.l13};
+#pragma unroll
   for (int i = 0; i < 6; ++i) {
-    out[((size_t)i * det.n_bins + k) * 2] = l[i].re;
-    out[((size_t)i * det.n_bins + k) * 2 + 1] = l[i].im;
+    const Cx s = mul(cf, S.l[i]);
+    out[((size_t)i * det.n_bins + k) * 2] = l[i].re + s.re;
+    out[((size_t)i * det.n_bins + k) * 2 + 1] = l[i].im + s.im;
   }
 }
 
@@ -730,6 +782,7 @@ struct TdWave {  // h+, hx sampled at t0 + m dt, m = 0 .. n - 1; zero outside
   const double* hc;
   double t0, inv_dt;
   int n;
+  int stride;  // doubles between samples (2: h+ and hx interleaved, read where the caller has them)
 };
 // h+, hx at the fractional sample x = (t - t0) / dt: linear between samples, zero outside (and
 // for NaN).  In two steps, so that a thread forms all its positions before it loads, and its
@@ -815,8 +868,8 @@ __global__ __launch_bounds__(256) void k_links_td(DetectorDev det, TdWave w, Ext
     for (int k = 0; k < KW; ++k) {
       const int q = threadIdx.x + 256 * k, s = wlo + q;
       const bool ok = q < wlen && s >= 0 && s < w.n;
-      vp[k] = ok ? w.hp[s] : 0.0;
-      vc[k] = ok ? w.hc[s] : 0.0;
+      vp[k] = ok ? w.hp[(size_t)s * w.stride] : 0.0;
+      vc[k] = ok ? w.hc[(size_t)s * w.stride] : 0.0;
     }
   } else if (i >= n) {
     return;
@@ -912,14 +965,14 @@ __global__ __launch_bounds__(256) void k_links_td(DetectorDev det, TdWave w, Ext
       hr[a][2] = win_c[jr];
       hr[a][3] = win_c[jr + 1];
     } else {
-      hs[a][0] = w.hp[qs[a].j];
-      hs[a][1] = w.hp[qs[a].j + 1];
-      hs[a][2] = w.hc[qs[a].j];
-      hs[a][3] = w.hc[qs[a].j + 1];
-      hr[a][0] = w.hp[qr[a].j];
-      hr[a][1] = w.hp[qr[a].j + 1];
-      hr[a][2] = w.hc[qr[a].j];
-      hr[a][3] = w.hc[qr[a].j + 1];
+      hs[a][0] = w.hp[(size_t)qs[a].j * w.stride];
+      hs[a][1] = w.hp[((size_t)qs[a].j + 1) * w.stride];
+      hs[a][2] = w.hc[(size_t)qs[a].j * w.stride];
+      hs[a][3] = w.hc[((size_t)qs[a].j + 1) * w.stride];
+      hr[a][0] = w.hp[(size_t)qr[a].j * w.stride];
+      hr[a][1] = w.hp[((size_t)qr[a].j + 1) * w.stride];
+      hr[a][2] = w.hc[(size_t)qr[a].j * w.stride];
+      hr[a][3] = w.hc[((size_t)qr[a].j + 1) * w.stride];
     }
   }
   double Pp[3], Pc[3], sp[3], sc[3], rp[3], rc[3];
@@ -2271,17 +2324,47 @@ static Extrinsic extrinsic_of(double lam, double beta, double psi, double tc) {
   return ex;
 }
 
+static int launch_links_container(pes_context* ctx, int det, int n_modes, const WaveIn& w, double lam, double beta,
+                                  double psi, double tc, double* d_out, void* stream) {
+  HIP_TRY(hipSetDevice(ctx->device));
+  const DetectorDev& d = ctx->hdets[det].d;
+  const Extrinsic ex = extrinsic_of(lam, beta, psi, tc);
+#define PES_LC(K)                                                                                                \
+  case K:                                                                                                        \
+    hipLaunchKernelGGL(k_links_container<K>, dim3((d.n_bins + 127) / 128), dim3(128), 0, (hipStream_t)stream,      \
+                       ctx->d_dets, det, ctx->d_bin_f, n_modes, w, ex, d_out);                                    \
+    break;
+  switch (d.kind | (d.duty ? 2 : 0)) { PES_LC(0) PES_LC(1) PES_LC(2) PES_LC(3) }
+#undef PES_LC
+  HIP_TRY(hipGetLastError());
+  return PES_OK;
+}
+
 extern "C" int pes_links_from_waveform(pes_context* ctx, int det, int n_modes, const double* d_wf, double lam,
                                        double beta, double psi, double tc, double* d_out, void* stream) {
   if (!ctx || !ctx->finalized) return fail(PES_ERR_STATE, "context missing or not finalized");
   if (det < 0 || det >= (int)ctx->hdets.size()) return fail(PES_ERR_INVALID, "bad detector index");
   if (n_modes < 1 || !d_wf || !d_out) return fail(PES_ERR_INVALID, "waveform/out must be non-NULL, n_modes >= 1");
-  HIP_TRY(hipSetDevice(ctx->device));
-  const int n = ctx->hdets[det].d.n_bins;
-  hipLaunchKernelGGL(k_links_container, dim3((n + 127) / 128), dim3(128), 0, (hipStream_t)stream, ctx->d_dets, det,
-                     ctx->d_bin_f, n_modes, d_wf, extrinsic_of(lam, beta, psi, tc), d_out);
-  HIP_TRY(hipGetLastError());
-  return PES_OK;
+  WaveIn w{};
+  w.wf = d_wf;
+  return launch_links_container(ctx, det, n_modes, w, lam, beta, psi, tc, d_out, stream);
+}
+
+extern "C" int pes_links_from_modes(pes_context* ctx, int det, int n_modes, const double* const* d_plus,
+                                    const double* const* d_cross, const double* const* d_tf, double lam, double beta,
+                                    double psi, double tc, double* d_out, void* stream) {
+  if (!ctx || !ctx->finalized) return fail(PES_ERR_STATE, "context missing or not finalized");
+  if (det < 0 || det >= (int)ctx->hdets.size()) return fail(PES_ERR_INVALID, "bad detector index");
+  if (n_modes < 1 || n_modes > PES_CONTAINER_MODES || !d_plus || !d_cross || !d_tf || !d_out)
+    return fail(PES_ERR_INVALID, "modes/out must be non-NULL, 1 <= n_modes <= PES_CONTAINER_MODES");
+  WaveIn w{};
+  for (int m = 0; m < n_modes; ++m) {
+    if (!d_plus[m] || !d_cross[m] || !d_tf[m]) return fail(PES_ERR_INVALID, "a mode's array is NULL");
+    w.hp[m] = d_plus[m];
+    w.hc[m] = d_cross[m];
+    w.tf[m] = d_tf[m];
+  }
+  return launch_links_container(ctx, det, n_modes, w, lam, beta, psi, tc, d_out, stream);
 }
 
 extern "C" int pes_tdi_from_links(pes_context* ctx, int det, int P, const double* d_links, double* d_out,
@@ -2318,6 +2401,17 @@ extern "C" int pes_td_links(int orbit_kind, double arm_length_m, double rotation
                             double omega_rotation, double lambda_ref, double beta_ref, const double* d_hp,
                             const double* d_hc, double wave_t0, double wave_dt, int wave_n, double lam, double beta,
                             double psi, double t0, double dt, int n, double* d_out, void* stream) {
+  return pes_td_links_strided(orbit_kind, arm_length_m, rotation_initial, revolution_initial, omega_rotation, lambda_ref,
+                              beta_ref, d_hp, d_hc, 1, wave_t0, wave_dt, wave_n, lam, beta, psi, t0, dt, n, d_out,
+                              stream);
+}
+
+extern "C" int pes_td_links_strided(int orbit_kind, double arm_length_m, double rotation_initial,
+                                    double revolution_initial, double omega_rotation, double lambda_ref,
+                                    double beta_ref, const double* d_hp, const double* d_hc, int wave_stride,
+                                    double wave_t0, double wave_dt, int wave_n, double lam, double beta, double psi,
+                                    double t0, double dt, int n, double* d_out, void* stream) {
+  if (wave_stride < 1) return fail(PES_ERR_INVALID, "td links: the waveform's stride must be positive");
   if (n < 0 || wave_n < 2) return fail(PES_ERR_INVALID, "td links: n >= 0 and at least two waveform samples");
   if (!(wave_dt > 0.0) || !(dt > 0.0)) return fail(PES_ERR_INVALID, "td links: sample spacings must be positive");
   if (n > 0 && (!d_hp || !d_hc || !d_out)) return fail(PES_ERR_INVALID, "td links: arrays must be non-NULL");
@@ -2326,7 +2420,7 @@ extern "C" int pes_td_links(int orbit_kind, double arm_length_m, double rotation
   const int rc = fill_orbit(d, orbit_kind, arm_length_m, rotation_initial, revolution_initial, omega_rotation,
                             lambda_ref, beta_ref);
   if (rc != PES_OK || n == 0) return rc;
-  const TdWave w{d_hp, d_hc, wave_t0, 1.0 / wave_dt, wave_n};
+  const TdWave w{d_hp, d_hc, wave_t0, 1.0 / wave_dt, wave_n, wave_stride};
   const Extrinsic ex = extrinsic_of(lam, beta, psi, 0.0);
   // every block's waveform window has length floor(b_hi + R) - floor(b_lo - R - L / dt_w) + 6
   // (td_links_window), at most 255 dt / dt_w + 2 R + L / dt_w + 8: stage it in LDS when that fits
