@@ -60,24 +60,6 @@ WORKLOADS = {
     "lisa_22_log16k": dict(detectors=("LISA",), modes=("22",), grid="log16k", cloud="local"),
 }
 
-# Algorithmic FP64 work of the fused kernel, counted from its source with add/sub/mul = 1 and
-# FMA = 2; sines, cosines and reciprocals are counted apart (not converted to flops).
-#   forward, per (bin, mode, row) evaluated: Hermite interpolation 20, orbit angle, the six
-#     scalar products and the nine link projections 76, pair phasors, total phase and
-#     polarization factors 33, three link pairs (sincs, n.e.n, link terms) 126, link sums 24;
-#     transcendentals: 4 sincos, 3 reciprocals
-#   forward, per (bin, row) evaluated: TDI constants 29, X, Y, Z -> A, E, T (T from the
-#     pair differences of the link sums) 82, residual and accumulation 24
-#   adjoint (lnL + gradient adds): per (bin, mode, row) the recomputed forward 253 (the forward
-#     less the total phase Psi + 2 pi f (t_c + k.x0), 14, whose phasor the adjoint reads back
-#     from the forward pass) and the adjoint 416 (link pairs 141, constellation and time 90,
-#     waveform side and node-table contraction 185); per (bin, row) 199 (link adjoints with the
-#     T channel's folded in, the p, q, k adjoints contracted with their lambda, beta, psi
-#     derivatives)
-# "evaluated" = the bin lies at or below the mode's cut (the (bin, row) pairs: below the row's
-# largest cut); the kernel skips the rest, whose response is exactly zero.
-OPS_BM_FWD, OPS_BR_FWD = 279, 135
-OPS_BM_ADJ, OPS_BR_ADJ = 669, 199
 PEAK_FP64 = 78.6e12  # MI355X FP64 vector, FLOP/s
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_lnl_traffic.json")
 
@@ -193,18 +175,19 @@ def prior_sweep(core, sizes=(256, 3001, 8192), seed=2027):
 
 
 def traffic_of(workload, precision, grad):
-    """HBM bytes per step of the fused kernel and the fraction of cycles its SIMDs issue VALU
-    work, from the committed rocprofv3 counter summaries (FETCH_SIZE / WRITE_SIZE scaled by a
-    plain copy; SQ_ACTIVE_INST_VALU over GRBM_GUI_ACTIVE); (None, None) for a workload they do
-    not cover."""
+    """HBM bytes per step of the lnL kernels, the fraction of cycles their SIMDs issue VALU work
+    and their FP64 flops (add, mul = 1, FMA = 2), from the committed rocprofv3 counter summaries
+    (FETCH_SIZE / WRITE_SIZE scaled by a plain copy; SQ_ACTIVE_INST_VALU over GRBM_GUI_ACTIVE;
+    SQ_INSTS_VALU_{ADD,MUL,FMA}_F64) of a 4096-row step; None each for a workload they do not
+    cover."""
     try:
         with open(TRAFFIC_FILE) as fh:
             doc = json.load(fh)
         e = doc["runs"][f"{workload}/{precision}/{'grad' if grad else 'lnl'}"]
         return (e["fetch_kib"] * 1024 * doc["fetch_scale"] + e["write_kib"] * 1024 * doc["write_scale"],
-                e.get("valu_busy"))
+                e.get("valu_busy"), e.get("flops"))
     except (OSError, KeyError, ValueError):
-        return None, None
+        return None, None, None
 
 
 def cpu_baseline(dets, wf, rows, n_rows=2):
@@ -444,11 +427,8 @@ def main():
                 head = prec
     h = res[head]
     value = K * P / h["dt"]
-    flops = h["bm"] * OPS_BM_FWD + h["br"] * OPS_BR_FWD
-    if grad:
-        flops += h["bm"] * OPS_BM_ADJ + h["br"] * OPS_BR_ADJ
-    achieved = flops / (h["kernel_ms"] * 1e-3)
-    traffic, valu_busy = traffic_of(args.workload, head, grad)
+    traffic, valu_busy, flops = traffic_of(args.workload, head, grad) if P == 4096 else (None, None, None)
+    achieved = flops / (h["kernel_ms"] * 1e-3) if flops else None
     line = {
         "metric": "lnL+grad evals/s, 4096-particle batch, mixed vs FP64 on 1 GPU, |dlnL|<1e-3" if grad
         else "lnL evals/s (no gradient)",
@@ -467,16 +447,16 @@ def main():
                    "nodes": wf.n_nodes, "gradient": grad, "precision": head,
                    "duty_cycle": {d.name: dict(d.duty_cycle._asdict()) for d in dets if d.duty_cycle is not None},
                    "schedule": tune if tune else dict(zip(("tiles_per_group", "blocks_per_cu"), core.schedule()))},
-        "roofline": {"bound": "valu", "achieved": achieved / 1e12, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_FP64, "traffic": traffic,
+        "roofline": {"bound": "valu", "achieved": achieved / 1e12 if achieved else None, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
+                     "frac": achieved / PEAK_FP64 if achieved else None, "traffic": traffic,
                      "hbm_GB_per_s": traffic / (h["kernel_ms"] * 1e-3) / 1e9 if traffic else None,
                      "valu_busy": valu_busy,
                      "work": {"bin_mode_rows": h["bm"], "bin_rows": h["br"], "flops": flops},
-                     "note": "algorithmic FP64 flops of the fused lnL(+grad) kernel over its HIP-event time; "
-                             "sines/cosines/reciprocals not counted as flops; all algebra is FP64 in every "
-                             "precision mode (mixed takes FP32 sin/cos/rcp in the adjoint only); traffic and "
-                             "valu_busy from the committed rocprofv3 counter summaries (profiles/), "
-                             "hbm_GB_per_s = traffic over this run's kernel time"},
+                     "note": "FP64 flops issued by the lnL(+grad) kernels (panel and bin-by-bin launches) over "
+                             "their HIP-event time; flops, traffic and valu_busy from the committed rocprofv3 "
+                             "counter summaries (profiles/) of this workload at 4096 particles, hbm_GB_per_s = "
+                             "traffic over this run's kernel time; work: (bin, mode, row) and (bin, row) "
+                             "triples at or below the cuts"},
     }
     for prec in precs:
         line[f"{prec}_evals_per_s"] = K * P / res[prec]["dt"]

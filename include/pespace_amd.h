@@ -42,10 +42,11 @@ extern "C" {
 #define PES_P_COALESCENCE_TIME 10   /* seconds                       */
 
 /* precision modes of pes_lnl_batch / pes_response.  lnL and the response are the FP64 forward in
- * both modes (identical results).  PES_PREC_MIXED changes the gradient only: the adjoint's
- * recompute of each mode takes the pair phasors and the total-phase phasor (phase reduced in
- * FP64) from the FP32 hardware sine/cosine and the sinc denominators from the FP32 reciprocal,
- * so the gradient carries FP32-level relative errors (~1e-7).  Any other value is rejected
+ * both modes (identical results).  PES_PREC_MIXED changes the gradient only, and only where the
+ * response is formed bin by bin (short grids, the lowest tiles; panels of bins are FP64 in both
+ * modes): the adjoint's recompute of each mode there takes the pair phasors from the FP32 hardware
+ * sine/cosine and the sinc denominators from the FP32 reciprocal, so that part of the gradient
+ * carries FP32-level relative errors (~1e-7).  Any other value is rejected
  * with PES_ERR_INVALID. */
 #define PES_PREC_FP64 0
 #define PES_PREC_MIXED 1
@@ -117,8 +118,9 @@ int pes_lnl_batch(pes_context* ctx, const double* d_params, int P, double* d_lnl
  * hipMalloc).  Same arguments, kernels and results as pes_lnl_batch, but the per-batch scratch
  * (work counter, per-row setup, node tables and their gradients, per-tile-group partials) lives
  * in a fixed array of PES_NOALLOC_SCRATCH_BYTES that every GPU holds once for the whole process;
- * pes_lnl_batch_noalloc_bytes(ctx, P, grad) gives what a batch needs (0 for a bad argument) and
- * a batch that needs more is rejected with PES_ERR_INVALID before anything is launched.  Every
+ * pes_lnl_batch_noalloc_bytes(ctx, P, grad) gives what a batch is accounted for (0 for a bad
+ * argument) and a batch accounted for more is rejected with PES_ERR_INVALID before anything is
+ * launched; one whose buffers take more than its account runs in parts, with the same results.  Every
  * call on a GPU shares that GPU's array and leaves its contents behind (each call rewrites all it
  * reads): calls that overlap on one GPU race, so serialise them (one stream, or events).  The
  * context's profiling (pes_context_set_profiling) does not apply to this entry point.
