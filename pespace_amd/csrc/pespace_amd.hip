@@ -2006,6 +2006,16 @@ static int rows_per_item(const pes_context* ctx, int P, bool grad, int grid, boo
   if (ctx->rows_override > 0) return std::min(ctx->rows_override, max_rows);
   const int per = fine ? 1 : std::min(ctx->tiles_per_group, GROUP_PANELS / GROUP_BIN_TILE);
   const int groups = panels ? ctx->n_bin_tiles / per + 1 : (fine ? ctx->n_tiles : n_groups_of(ctx));
+  if (fine) {
+    // about three items per resident block (two per CU with the gradient, three without): an item's
+    // rows follow one another, so a batch that does not fill the chip takes the time of its
+    // longest item; forward items of few modes cost some rows' time to start.  Short LISA data,
+    // gradient, six modes: 4 rows 151 -> 81 us (8 rows an item -> 1), 16 rows 256 -> 121 (2), 64 rows
+    // 292 -> 264 (6); without it 16 rows 104 -> 74 (2); one mode 300 rows 143 -> 119 (17)
+    const long long slots = 3LL * ctx->n_cu * (grad ? 2 : 3);
+    const long long lo = grad ? 1 : std::max(2, 4 / ctx->modes.n);
+    return (int)std::max(lo, std::min((long long)max_rows, ((long long)P * groups + slots - 1) / slots));
+  }
   const long long fit = (long long)P * groups / ((panels ? 2LL : 4LL) * grid);
   return (int)std::max(8LL, std::min((long long)max_rows, fit));
 }
