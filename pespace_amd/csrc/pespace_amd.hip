@@ -1247,6 +1247,7 @@ struct pes_context {
   struct HostDet {
     DetectorDev d;
     std::vector<double> f, w, dre, dim;  // w, dre, dim: [3][n]
+    bool observed = false;  // a channel enters the likelihood
   };
   std::vector<HostDet> hdets;
   // device constant data
@@ -1389,6 +1390,7 @@ extern "C" int pes_context_add_detector(pes_context* ctx, int orbit_kind, double
     double dfk = weight ? weight[k] : df;
     for (int ch = 0; ch < 3; ++ch) {
       if (!channel_mask[ch]) continue;
+      h.observed = true;
       double s = psd[(size_t)ch * n_bins + k];
       if (!(s > 0.0)) return fail(PES_ERR_INVALID, "PSD must be positive on used channels");
       h.w[(size_t)ch * n_bins + k] = 2.0 * dfk / s;  // likelihood_ti.py:63-67: -2 df |d-h|^2 / S
@@ -1562,6 +1564,8 @@ static void free_dev(void* p) {
 // would hold too few bins to pay for their points).  bf, bj: frequency and node interval per bin.
 static int build_panels(pes_context* ctx, const std::vector<double>& bf, const std::vector<int>& bj) {
   if (ctx->direct) return PES_OK;
+  // a context for responses alone (no channel enters the likelihood: lnL = 0) does without
+  if (std::none_of(ctx->hdets.begin(), ctx->hdets.end(), [](const auto& h) { return h.observed; })) return PES_OK;
   const int nt = ctx->n_tiles;
   std::vector<int> tp(2 * (size_t)nt, 0), pi;
   std::vector<double> pd;
