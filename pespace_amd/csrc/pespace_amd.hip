@@ -2011,14 +2011,16 @@ static int rows_per_item(const pes_context* ctx, int P, bool grad, int grid, boo
   const int per = fine ? 1 : std::min(ctx->tiles_per_group, GROUP_PANELS / GROUP_BIN_TILE);
   const int groups = panels ? ctx->n_bin_tiles / per + 1 : (fine ? ctx->n_tiles : n_groups_of(ctx));
   if (fine) {
-    // about three items per resident block (two per CU with the gradient, three without): an item's
-    // rows follow one another, so a batch that does not fill the chip takes the time of its
-    // longest item; forward items of few modes cost some rows' time to start.  Short LISA data,
-    // gradient, six modes: 4 rows 151 -> 81 us (8 rows an item -> 1), 16 rows 256 -> 121 (2), 64 rows
-    // 292 -> 264 (6); without it 16 rows 104 -> 74 (2); one mode 300 rows 143 -> 119 (17)
-    const long long slots = 3LL * ctx->n_cu * (grad ? 2 : 3);
-    const long long lo = grad ? 1 : std::max(2, 4 / ctx->modes.n);
-    return (int)std::max(lo, std::min((long long)max_rows, ((long long)P * groups + slots - 1) / slots));
+    // about three items per resident block (two per CU with the gradient, three without), five where
+    // a row is long (gradient of three modes or more): an item's rows follow one another, so a batch
+    // that does not fill the chip takes the time of its longest item; forward items of few modes
+    // cost some rows' time to start.  Against items of 8 rows, short LISA data, gradient, six modes:
+    // 4 rows 149 -> 81 us (1 row an item), 16 rows 256 -> 121 (2), 64 rows 309 -> 284 (4); without
+    // it 16 rows 102 -> 74 (2); one mode 300 rows 143 -> 122 (17)
+    const long long slots = (long long)ctx->n_cu * (grad ? 2 : 3), work = (long long)P * groups;
+    const long long want = slots * (grad && ctx->modes.n >= 3 ? 5 : 3);
+    const long long lo = !grad ? std::max(2, 4 / ctx->modes.n) : work > 3 * slots ? 2 : 1;
+    return (int)std::max(lo, std::min((long long)max_rows, (work + want - 1) / want));
   }
   const long long fit = (long long)P * groups / ((panels ? 2LL : 4LL) * grid);
   return (int)std::max(8LL, std::min((long long)max_rows, fit));
