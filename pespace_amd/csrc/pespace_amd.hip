@@ -1,8 +1,8 @@
 // MI355X (gfx950) kernels and C-ABI for the FD lnL(+grad) hot path.
 //
 // Pipeline per batch of P parameter rows (one launch each, all on one stream):
-//   k_setup     one thread per row: PhenomD/HM coefficients (+ d/dtheta_int) and
-//               the extrinsic constants (polarization basis, harmonic factors)
+//   k_setup     a lane per (row, derivative): PhenomD/HM coefficients (+ d/dtheta_int), and
+//               per (row, mode): extrinsic constants (polarization basis, harmonic factors)
 //   k_nodes     one thread per (row, mode, node): A, dA/du, Psi, dPsi/du on the
 //               log-spaced interpolation nodes (u = ln f)
 //   k_panel_class, k_lnl_panel  (long grids) lnL and gradient from short polynomials of the

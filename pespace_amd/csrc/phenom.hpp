@@ -149,9 +149,10 @@ enum SetupId {
 };
 
 // Coefficient store of Phenom: an array (written by phenom_setup) or, in the node kernels,
-// SetupView: a read-only view of one row of the setup table [5][N_SETUP] (values, then d/dtheta
-// for Mc, q, chi1, chi2: a kernel that needs the values alone reads them from one stretch), building each coefficient as the requested dual on access, so the
-// kernels hold no per-lane copy of the ~60 coefficients.
+// SetupView: a read-only view of one row of the setup table [5][N_SETUP] (values, then d/dtheta for
+// Mc, q, chi1, chi2: a kernel that needs the values alone reads them from one stretch), building
+// each coefficient as the requested dual on access, so the kernels hold no per-lane copy of the
+// ~70 coefficients.
 template <class S>
 struct SetupView;
 template <>
