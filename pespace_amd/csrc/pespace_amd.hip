@@ -2095,12 +2095,13 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     const int n_grp = fine ? ranges[r].tile_end - tile_begin : ranges[r].n_groups;
     const int n_work = n_grp * n_chunks;
     const int grid_r = std::min(grid, n_work);
-    if (panels) {
+    // fine: an item is a panel, with sums of its own (none in a range all of whose tiles go bin by
+    // bin); otherwise one per group, whose sums k_lnl adds to
+    const int pan_begin = panels ? ctx->tile_pan0[tile_begin] : 0;
+    const int n_pg = !panels ? 0 : fine ? ctx->tile_pan0[ranges[r].tile_end] - pan_begin : n_grp;
+    if (n_pg > 0) {
       int* counter = sc.work_counter + 3 * MAX_TILE_RANGES + r;
       const unsigned long long* off = ranges[r].duty ? sc.off_bits : nullptr;
-      // fine: an item is a panel, with sums of its own
-      const int pan_begin = ctx->tile_pan0[tile_begin], pan_end = ctx->tile_pan0[ranges[r].tile_end];
-      const int n_pg = fine ? pan_end - pan_begin : n_grp;
       const int n_items = n_pg * ((P + PANEL_ROWS - 1) / PANEL_ROWS);
       // two blocks per CU are resident; a wave takes an item
       const int grid_p = std::min(2 * ctx->n_cu, (n_items + TILE / 64 - 1) / (TILE / 64));
