@@ -1025,11 +1025,11 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
                                               const double* __restrict__ bin_f, const int* __restrict__ bin_j,
                                               const double* __restrict__ bin_s, const double* __restrict__ bin_rec,
                                               const double* __restrict__ tile_f0, const double* __restrict__ tile_dd,
-                                              const int* __restrict__ grp, int n_grp, const double* __restrict__ pconst,
+                                              RangeGroups grp, int n_grp, const double* __restrict__ pconst,
                                               const double* __restrict__ nodes,
                                               const double* __restrict__ nodes_grad, int NNS, double du,
                                               ModeList modes, int P, int rows, const int* __restrict__ tile_jr,
-                                              int tile_begin, int group_offset,
+                                              int group_offset,
                                               int* __restrict__ work_counter, double* __restrict__ partial,
                                               const unsigned long long* __restrict__ off_bits,
                                               const unsigned char* __restrict__ items,
@@ -1052,8 +1052,7 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
   const int lane = threadIdx.x & 63;
   const int wave = GRAD ? (int)(threadIdx.x >> 6) : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // rows (1 <= rows <= CH) per work item, chosen by the host.  This launch covers the n_grp groups
-  // of a tile range (group gl: tiles grp[gl] .. grp[gl + 1] - 1; grp null: the one tile
-  // tile_begin + gl), whose partial sums go to groups group_offset + 0, 1, ...: one launch (and
+  // of a tile range, whose partial sums go to groups group_offset + 0, 1, ...: one launch (and
   // counter) per tile range of one orbit kind and duty flag, two for a duty-cycled range
   const int n_chunks = (P + rows - 1) / rows;
   // with panels only the groups of the batch's list have work left here
@@ -1082,7 +1081,7 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
       continue;
     }
     const int p0 = c * rows, p1 = min(P, p0 + rows);
-    const int t_first = grp ? grp[gl] : tile_begin + gl, t_end = grp ? grp[gl + 1] : t_first + 1;
+    const int t_first = grp.begin(gl), t_end = grp.end(gl);
     for (int i = threadIdx.x; i < (TILE / 64) * CH * NOUT; i += TILE) (&acc[0][0][0])[i] = 0.0;
     double chunk_cut = 0.0;
     for (int p = p0; p < p1; ++p) chunk_cut = fmax(chunk_cut, pconst[(size_t)p * PC_STRIDE + PC_FCUT]);

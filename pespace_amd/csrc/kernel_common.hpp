@@ -39,6 +39,24 @@ enum PConst {
 };
 enum { MF_FPR = 0, MF_FPI, MF_FCR, MF_FCI, MF_CUT, MF_DFPR, MF_DFPI, MF_DFCR, MF_DFCI };
 
+// ---- tile groups -----------------------------------------------------------------------
+// The groups (RangeGroups) of all tile ranges in turn (range r: tiles tile0[r] .., groups group0[r] ..)
+struct TileGroups {
+  const int* first;
+  int per, n_ranges, tile0[MAX_TILE_RANGES + 1], group0[MAX_TILE_RANGES];
+  __device__ void tiles(int g, int& t0, int& t1) const {
+    if (first) {
+      t0 = first[g];
+      t1 = first[g + 1];
+      return;
+    }
+    int r = 0;
+    while (r + 1 < n_ranges && group0[r + 1] <= g) ++r;
+    t0 = tile0[r] + (g - group0[r]) * per;
+    t1 = min(tile0[r + 1], t0 + per);
+  }
+};
+
 // detector owning tile `tile` (detectors are concatenated in tile order)
 __device__ inline int tile_detector(const DetectorDev* dets, int n_det, int tile) {
   int acc = 0;

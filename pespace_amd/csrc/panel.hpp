@@ -680,10 +680,6 @@ __global__ __launch_bounds__(TILE) void k_panel_rec(const DetectorDev* __restric
   o[224] = make_double2(p2.im, 0.0);
 }
 
-struct RangeBases {  // first tile and first group of each tile range
-  int tile0[MAX_TILE_RANGES], group0[MAX_TILE_RANGES];
-};
-
 // Per (tile, row): bit 1 when the pair goes bin by bin: the tile has no panels, a mode's cut lies
 // inside it, a mode's orbit angle (geocentric: the rotation angle) turns by more than PANEL_SWING
 // over a panel, or a duty-cycled detector's window is not flat 1 over a panel (off tiles aside:
@@ -695,7 +691,7 @@ __global__ __launch_bounds__(64) void k_panel_class(const DetectorDev* __restric
                                                     const double* __restrict__ pconst, const double* __restrict__ nodes,
                                                     int NNS, double du, ModeList modes, int P, int words,
                                                     const unsigned long long* __restrict__ off_bits, PanelDev pan,
-                                                    BinWork bw, RangeBases rb, int fine,
+                                                    BinWork bw, TileGroups rb, int fine,
                                                     unsigned long long* __restrict__ dbits) {
   const int tile = blockIdx.x * 64 + threadIdx.x;
   const int tl_ = min(tile, n_tiles - 1);

@@ -351,13 +351,14 @@ __global__ __launch_bounds__(TILE) void k_direct_grad(const double* __restrict__
 }
 // the tiles and modes of each group, in order: the group's partial sums of the four parameters
 __global__ __launch_bounds__(256) void k_direct_sums(const double* __restrict__ sums, int n_modes, int P,
-                                                     const int* __restrict__ grp, int n_groups,
-                                                     double* __restrict__ partial) {
+                                                     TileGroups grp, int n_groups, double* __restrict__ partial) {
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (size_t)n_groups * 4 * P) return;
   const int p = (int)(idx % P), k = (int)(idx / P % 4), g = (int)(idx / ((size_t)P * 4));
   double s = 0.0;
-  for (int i = grp[g] * n_modes; i < grp[g + 1] * n_modes; ++i) s += sums[((size_t)i * 4 + k) * P + p];
+  int t0, t1;
+  grp.tiles(g, t0, t1);
+  for (int i = t0 * n_modes; i < t1 * n_modes; ++i) s += sums[((size_t)i * 4 + k) * P + p];
   partial[((size_t)g * (1 + PES_N_PARAMS) + 1 + k) * P + p] = s;
 }
 #endif
@@ -406,7 +407,7 @@ __global__ __launch_bounds__(256) void k_reduce(const double* __restrict__ parti
 // their sums (fine_pan: per panel; fine_bin: per tile of the four waves of the bin-by-bin kernel) are put
 // together here in the order in which an item of a whole group adds them, so that a row's
 // result does not depend on its batch.  One thread per (group, output, row).
-__global__ __launch_bounds__(256) void k_group_sums(const int* __restrict__ grp, int n_groups, int P, int nout,
+__global__ __launch_bounds__(256) void k_group_sums(TileGroups grp, int n_groups, int P, int nout,
                                                     const double* __restrict__ fine_pan,
                                                     const double* __restrict__ fine_bin,
                                                     const int* __restrict__ tile_pan, BinWork bw,
@@ -414,7 +415,8 @@ __global__ __launch_bounds__(256) void k_group_sums(const int* __restrict__ grp,
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (size_t)n_groups * nout * P) return;
   const int p = (int)(idx % P), o = (int)(idx / P % nout), g = (int)(idx / ((size_t)P * nout));
-  const int t0 = grp[g], t1 = grp[g + 1];
+  int t0, t1;
+  grp.tiles(g, t0, t1);
   double a = 0.0, d[TILE / 64];
   bool any = !fine_pan;
 #pragma unroll
@@ -555,12 +557,11 @@ __global__ __launch_bounds__(64) void k_duty_items(const DetectorDev* __restrict
                                                    const double* __restrict__ tile_f0, const int* __restrict__ tile_jr,
                                                    const double* __restrict__ pconst, const double* __restrict__ nodes,
                                                    int NNS, double u0, double du, ModeList modes, int P, int rows,
-                                                   int n_chunks, int tile_begin, const int* __restrict__ grp,
-                                                   int group_offset, int enable, unsigned char* __restrict__ items,
+                                                   int n_chunks, RangeGroups grp, int group_offset, int enable, unsigned char* __restrict__ items,
                                                    int* __restrict__ n_duty_items, int words,
                                                    const unsigned long long* __restrict__ dbits) {
   const int gl = blockIdx.x / n_chunks, c = blockIdx.x % n_chunks;
-  const int t_first = grp ? grp[gl] : tile_begin + gl, t_end = grp ? grp[gl + 1] : t_first + 1;
+  const int t_first = grp.begin(gl), t_end = grp.end(gl);
   const int p0 = c * rows, p1 = min(P, p0 + rows);
   const int nt = t_end - t_first, np = p1 - p0;
   int ok = enable;
@@ -1188,14 +1189,14 @@ __global__ __launch_bounds__(TILE) void k_whittle_final(const double* __restrict
 #define PES_LNL_PARAMS                                                                                       \
   const DetectorDev *dets, int n_det, int n_tiles, const double *bin_f, const int *bin_j, const double *bin_s, \
       const double *bin_rec, const double *tile_f0,                                                       \
-      const double *tile_dd, const int *grp, int n_grp, const double *pconst, const double *nodes,           \
+      const double *tile_dd, RangeGroups grp, int n_grp, const double *pconst, const double *nodes,          \
       const double *nodes_grad, int NNS, double du, ModeList modes, int P, int rows, const int *tile_jr,     \
-      int tile_begin, int group_offset, int *work_counter, double *partial,                                  \
+      int group_offset, int *work_counter, double *partial,                                                  \
       const unsigned long long *off_bits, const unsigned char *items, const int *tile_pan,                   \
       BinWork bw, int range, int list_base, const unsigned long long *dbits, int fine
 #define PES_LNL_NAMES                                                                                     \
   dets, n_det, n_tiles, bin_f, bin_j, bin_s, bin_rec, tile_f0, tile_dd, grp, n_grp, pconst,  \
-      nodes, nodes_grad, NNS, du, modes, P, rows, tile_jr, tile_begin, group_offset, work_counter, partial, \
+      nodes, nodes_grad, NNS, du, modes, P, rows, tile_jr, group_offset, work_counter, partial, \
       off_bits, items, tile_pan, bw, range, list_base, dbits, fine
 
 }  // namespace
@@ -1231,6 +1232,13 @@ hipError_t pes::launch_lnl_fwd(int precision, int kd, int grid, hipStream_t st, 
 }
 #else
 // ================================= host side ================================================
+// The first tile of each tile group, and n_tiles, under one tiles_per_group; on the device those and
+// the group of each tile
+struct GroupTable {
+  std::vector<int> first;
+  const int *d_first = nullptr, *d_tile_group = nullptr;
+};
+
 struct pes_context {
   int device = 0;
   ModeList modes{};
@@ -1284,7 +1292,8 @@ struct pes_context {
   int n_bin_tiles = 0;  // tiles without panels
   std::vector<int> tile_panels;  // panels per tile
   std::vector<int> tile_pan0;    // panels before each tile, and their number
-  std::vector<int> groups;       // first tile of each tile group (build_groups), and n_tiles
+  // tile groups of a context with panels (build_groups), for each tiles_per_group
+  std::vector<GroupTable> groups;
   int* d_groups = nullptr;
   double* d_fine = nullptr;  // per-tile sums of small batches (fine_doubles)
   size_t cap_fine = 0;
@@ -1431,6 +1440,17 @@ extern "C" int pes_context_set_duty_cycle(pes_context* ctx, int det_index, doubl
 struct TileRange {
   int tile_begin, tile_end, duty, kind, group_offset, n_groups;
 };
+// The tile groups: at most tiles_per_group tiles each, none across two runs; with panels also at
+// most GROUP_PANELS panels, so that the work items of the low frequencies, whose tiles are cut into
+// several panels or go bin by bin, do not outlast the others (the network, P = 45 with the gradient:
+// 16.8 -> 10.2 ms).  Without panels they are equal and formed where they are used; with panels they
+// are tables, one for each tiles_per_group that makes a difference (a tile costs at least one
+// panel), uploaded once: a captured graph keeps those that it was captured with, whatever schedule is
+// set later
+constexpr int GROUP_PANELS = 12, GROUP_BIN_TILE = 4;
+static const GroupTable& group_table(const pes_context* ctx) {
+  return ctx->groups[std::min(ctx->tiles_per_group, GROUP_PANELS) - 1];
+}
 static int tile_ranges(const pes_context* ctx, TileRange* out) {
   int n = 0;
   for (const auto& h : ctx->hdets) {
@@ -1441,49 +1461,54 @@ static int tile_ranges(const pes_context* ctx, TileRange* out) {
       out[n++] = {t0, t1, duty, kind, 0, 0};
     }
   }
-  for (int r = 0, g = 0; r < n && !ctx->groups.empty(); ++r) {
+  for (int r = 0, g = 0; r < n; ++r) {
     out[r].group_offset = g;
-    while (ctx->groups[g] < out[r].tile_end) ++g;
+    if (ctx->groups.empty())
+      g += (out[r].tile_end - out[r].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
+    else
+      while (group_table(ctx).first[g] < out[r].tile_end) ++g;
     out[r].n_groups = g - out[r].group_offset;
   }
   return n;
 }
-
-// The tile groups (first tile of each, and the number of tiles): at most tiles_per_group tiles
-// each, none across two runs; with panels also at most GROUP_PANELS panels, so that the work items
-// of the low frequencies, whose tiles are cut into several panels or go bin by bin, do not outlast
-// the others (the network, P = 45 with the gradient: 16.8 -> 10.2 ms)
-constexpr int GROUP_PANELS = 12, GROUP_BIN_TILE = 4;
 static int build_groups(pes_context* ctx) {
+  if (!ctx->pan.tile_pan) return PES_OK;
   TileRange r[MAX_TILE_RANGES];
-  ctx->groups.clear();
-  const int n = tile_ranges(ctx, r);
-  for (int i = 0; i < n; ++i) {
-    int tiles = 0, cost = 0;
-    for (int t = r[i].tile_begin; t < r[i].tile_end; ++t) {
-      int c = 0;
-      if (ctx->pan.tile_pan) c = ctx->tile_panels[t] > 0 ? ctx->tile_panels[t] : GROUP_BIN_TILE;
-      if (t == r[i].tile_begin || tiles == ctx->tiles_per_group || cost + c > GROUP_PANELS) {
-        ctx->groups.push_back(t);
-        tiles = cost = 0;
+  const int n = tile_ranges(ctx, r), nt = ctx->n_tiles;
+  std::vector<GroupTable> tables(GROUP_PANELS);
+  std::vector<int> up, tile_range(nt);
+  for (int per = 1; per <= GROUP_PANELS; ++per) {
+    std::vector<int>& first = tables[per - 1].first;
+    const size_t at = up.size();
+    up.resize(at + nt);  // the group of each tile, then the groups' first tiles
+    for (int i = 0; i < n; ++i) {
+      int tiles = 0, cost = 0;
+      for (int t = r[i].tile_begin; t < r[i].tile_end; ++t) {
+        const int c = ctx->tile_panels[t] > 0 ? ctx->tile_panels[t] : GROUP_BIN_TILE;
+        if (t == r[i].tile_begin || tiles == per || cost + c > GROUP_PANELS) {
+          first.push_back(t);
+          tiles = cost = 0;
+        }
+        ++tiles;
+        cost += c;
+        up[at + t] = (int)first.size() - 1;
+        tile_range[t] = i;
       }
-      ++tiles;
-      cost += c;
     }
+    first.push_back(nt);
+    up.insert(up.end(), first.begin(), first.end());
   }
-  ctx->groups.push_back(ctx->n_tiles);
-  if (!ctx->d_groups) HIP_TRY(hipMalloc(&ctx->d_groups, ((size_t)ctx->n_tiles + 1) * sizeof(int)));
-  HIP_TRY(hipMemcpy(ctx->d_groups, ctx->groups.data(), ctx->groups.size() * sizeof(int), hipMemcpyHostToDevice));
-  if (ctx->pan.tile_pan) {  // group and range of each tile (BinWork)
-    std::vector<int> tg(ctx->n_tiles), tr(ctx->n_tiles);
-    for (size_t g = 0; g + 1 < ctx->groups.size(); ++g)
-      for (int t = ctx->groups[g]; t < ctx->groups[g + 1]; ++t) tg[t] = (int)g;
-    for (int i = 0; i < n; ++i)
-      for (int t = r[i].tile_begin; t < r[i].tile_end; ++t) tr[t] = i;
-    int* to = ctx->d_bin_work + (ctx->bin_work.tile_group - ctx->d_bin_work);
-    HIP_TRY(hipMemcpy(to, tg.data(), tg.size() * sizeof(int), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(to + ctx->n_tiles, tr.data(), tr.size() * sizeof(int), hipMemcpyHostToDevice));
+  HIP_TRY(hipMalloc(&ctx->d_groups, up.size() * sizeof(int)));
+  HIP_TRY(hipMemcpy(ctx->d_groups, up.data(), up.size() * sizeof(int), hipMemcpyHostToDevice));
+  const int* d = ctx->d_groups;
+  for (auto& t : tables) {
+    t.d_tile_group = d;
+    t.d_first = d + nt;
+    d = t.d_first + t.first.size();
   }
+  ctx->groups = std::move(tables);
+  int* to = ctx->d_bin_work + (ctx->bin_work.tile_range - ctx->d_bin_work);
+  HIP_TRY(hipMemcpy(to, tile_range.data(), nt * sizeof(int), hipMemcpyHostToDevice));
   return PES_OK;
 }
 
@@ -1491,7 +1516,11 @@ static int build_groups(pes_context* ctx) {
 // kernel forms the same count from n_tiles)
 static int off_words_of(const pes_context* ctx) { return (ctx->n_tiles + 63) / 64; }
 
-static int n_groups_of(const pes_context* ctx) { return (int)ctx->groups.size() - 1; }
+static int n_groups_of(const pes_context* ctx) {
+  TileRange r[MAX_TILE_RANGES];
+  const int n = tile_ranges(ctx, r);
+  return r[n - 1].group_offset + r[n - 1].n_groups;
+}
 
 // ---- the entry point that allocates nothing ---------------------------------------------------
 // Its scratch (work counter, per-row setup and constants, node tables, per-tile-group partials)
@@ -1637,13 +1666,14 @@ static int build_panels(pes_context* ctx, const std::vector<double>& bf, const s
   HIP_TRY(hipMalloc(&ctx->d_pan_d, pd.size() * sizeof(double)));
   HIP_TRY(hipMalloc(&ctx->d_pan_rec, (size_t)ctx->NB * PANEL_REC * sizeof(double2)));
   constexpr int STATE = 64;  // ints before the first array
-  HIP_TRY(hipMalloc(&ctx->d_bin_work, (STATE + 5 * (size_t)nt) * sizeof(int)));
+  HIP_TRY(hipMalloc(&ctx->d_bin_work, (STATE + 4 * (size_t)nt) * sizeof(int)));
   HIP_TRY(hipMemcpy(ctx->d_tile_pan, tp.data(), tp.size() * sizeof(int), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(ctx->d_pan_i, pi.data(), pi.size() * sizeof(int), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(ctx->d_pan_d, pd.data(), pd.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemset(ctx->d_bin_work, 0, (STATE + 5 * (size_t)nt) * sizeof(int)));
+  HIP_TRY(hipMemset(ctx->d_bin_work, 0, (STATE + 4 * (size_t)nt) * sizeof(int)));
   int* w = ctx->d_bin_work + STATE;
-  ctx->bin_work = {ctx->d_bin_work, w, w + nt, w + 2 * (size_t)nt, w + 3 * (size_t)nt, w + 4 * (size_t)nt};
+  // (tile_group is that of the batch's groups)
+  ctx->bin_work = {ctx->d_bin_work, w, w + nt, w + 2 * (size_t)nt, nullptr, w + 3 * (size_t)nt};
   for (int i = 0; i < (int)ctx->hdets.size(); ++i)
     hipLaunchKernelGGL(k_panel_rec, dim3(ctx->hdets[i].d.n_tiles), dim3(TILE), 0, nullptr, ctx->d_dets, i,
                        ctx->d_bin_f, ctx->d_bin_s, ctx->d_bin_j, ctx->d_bin_rec, ctx->du, ctx->d_pan_rec);
@@ -2059,15 +2089,26 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     HIP_TRY(hipGetLastError());
   }
   const int n_det = (int)ctx->hdets.size();
+  TileGroups groups{};
+  groups.n_ranges = n_ranges;
+  for (int r = 0; r < n_ranges; ++r) {
+    groups.tile0[r] = ranges[r].tile_begin;
+    groups.group0[r] = ranges[r].group_offset;
+  }
+  groups.tile0[n_ranges] = ctx->n_tiles;
+  groups.per = ctx->tiles_per_group;
+  groups.first = panels ? group_table(ctx).d_first : nullptr;
+  BinWork bin_work = ctx->bin_work;
+  if (panels) bin_work.tile_group = group_table(ctx).d_tile_group;
+  // a launch's groups in range r; fine: its tiles
+  auto range_groups = [&](int r) -> RangeGroups {
+    return {fine || !panels ? nullptr : groups.first + ranges[r].group_offset, ranges[r].tile_begin, ranges[r].tile_end,
+            fine ? 1 : groups.per};
+  };
   if (panels) {  // which (tile, row)s of the tiles with panels go bin by bin all the same
-    RangeBases rb{};
-    for (int r = 0; r < n_ranges; ++r) {
-      rb.tile0[r] = ranges[r].tile_begin;
-      rb.group0[r] = ranges[r].group_offset;
-    }
     hipLaunchKernelGGL(k_panel_class, dim3(off_words, std::min(P, 65535)), dim3(64), 0, st, ctx->d_dets, n_det,
                        ctx->n_tiles, ctx->d_tile_f0, ctx->d_bin_f, sc.pconst, sc.nodes, NNS, ctx->du, ctx->modes, P,
-                       off_words, ctx->any_duty ? sc.off_bits : nullptr, ctx->pan, ctx->bin_work, rb, fine ? 1 : 0,
+                       off_words, ctx->any_duty ? sc.off_bits : nullptr, ctx->pan, bin_work, groups, fine ? 1 : 0,
                        sc.dbits);
     HIP_TRY(hipGetLastError());
   }
@@ -2078,8 +2119,8 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     const int n_grp = fine ? ranges[r].tile_end - ranges[r].tile_begin : ranges[r].n_groups, n_work = n_grp * n_chunks;
     hipLaunchKernelGGL(k_duty_items, dim3(n_work), dim3(64), 0, st, ctx->d_dets, n_det, ctx->d_tile_f0,
                        ctx->d_tile_jr, sc.pconst, sc.nodes, NNS, ctx->u0, ctx->du, ctx->modes, P, rows, n_chunks,
-                       ranges[r].tile_begin, fine ? nullptr : ctx->d_groups + ranges[r].group_offset,
-                       fine ? ranges[r].tile_begin : ranges[r].group_offset, ctx->direct ? 0 : 1, items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, sc.dbits);
+                       range_groups(r), fine ? ranges[r].tile_begin : ranges[r].group_offset, ctx->direct ? 0 : 1,
+                       items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, sc.dbits);
     HIP_TRY(hipGetLastError());
   }
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -2091,7 +2132,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   for (int r = 0; r < n_ranges; ++r) {
     const int tile_begin = ranges[r].tile_begin;
     const int group_offset = fine ? tile_begin : ranges[r].group_offset;  // fine: a partial per tile
-    const int* grp = fine ? nullptr : ctx->d_groups + group_offset;
+    const RangeGroups grp = range_groups(r);
     const int n_grp = fine ? ranges[r].tile_end - tile_begin : ranges[r].n_groups;
     const int n_work = n_grp * n_chunks;
     const int grid_r = std::min(grid, n_work);
@@ -2106,7 +2147,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
       // two blocks per CU are resident; a wave takes an item
       const int grid_p = std::min(2 * ctx->n_cu, (n_items + TILE / 64 - 1) / (TILE / 64));
 #define PES_PANEL_ARGS                                                                                        \
-  ctx->d_dets, n_det, ctx->n_tiles, ctx->d_tile_f0, ctx->d_tile_dd, grp, n_pg, sc.pconst, sc.nodes,            \
+  ctx->d_dets, n_det, ctx->n_tiles, ctx->d_tile_f0, ctx->d_tile_dd, grp.first, n_pg, sc.pconst, sc.nodes,            \
       sc.nodes_grad, NNS, ctx->du, ctx->modes, P, fine ? pan_begin : group_offset, counter,                   \
       part_pan, off, sc.dbits, ctx->pan, pan_begin
 #define PES_PANEL(G, KD) \
@@ -2132,8 +2173,8 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
 #define PES_LNL_ARGS                                                                                         \
   ctx->d_dets, n_det, ctx->n_tiles, ctx->d_bin_f, ctx->d_bin_j, ctx->d_bin_s, ctx->d_bin_rec,                 \
       ctx->d_tile_f0, ctx->d_tile_dd, grp, n_grp, sc.pconst, sc.nodes, sc.nodes_grad, NNS, ctx->du,           \
-      ctx->modes, P, rows, ctx->d_tile_jr, tile_begin, group_offset, counter, part_bin,                       \
-      sc.off_bits, items, ctx->pan.tile_pan, ctx->bin_work, r, group_offset, sc.dbits, fine ? 1 : 0
+      ctx->modes, P, rows, ctx->d_tile_jr, group_offset, counter, part_bin,                                   \
+      sc.off_bits, items, ctx->pan.tile_pan, bin_work, r, group_offset, sc.dbits, fine ? 1 : 0
 #define PES_LNL_GRAD(PR, KD)                                                                                  \
   if (panels && !kDirect<KD>)                                                                                \
     hipLaunchKernelGGL((k_lnl<PR, true, KD, !kDirect<KD>>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS);          \
@@ -2174,8 +2215,8 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   }
   if (fine) {
     hipLaunchKernelGGL(k_group_sums, dim3((unsigned)(((size_t)n_groups * nout * P + 255) / 256)), dim3(256), 0, st,
-                       ctx->d_groups, n_groups, P, nout, panels ? part_pan : nullptr, part_bin, ctx->pan.tile_pan,
-                       ctx->bin_work, sc.partial);
+                       groups, n_groups, P, nout, panels ? part_pan : nullptr, part_bin, ctx->pan.tile_pan, bin_work,
+                       sc.partial);
     HIP_TRY(hipGetLastError());
   }
   if (direct && grad) {
@@ -2184,7 +2225,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
                        sc.setup, sc.pconst, ctx->d_fpow, ctx->n_tiles, sc.nodes_grad, ctx->modes, P, sc.nodes);
     HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL(k_direct_sums, dim3((unsigned)(((size_t)n_groups * 4 * P + 255) / 256)), dim3(256), 0, st,
-                       sc.nodes, ctx->modes.n, P, ctx->d_groups, n_groups, sc.partial);
+                       sc.nodes, ctx->modes.n, P, groups, n_groups, sc.partial);
     HIP_TRY(hipGetLastError());
   }
 #define PES_REDUCE(RB)                                                                                        \
@@ -2538,13 +2579,9 @@ extern "C" int pes_context_set_schedule(pes_context* ctx, int tiles_per_group, i
   if (!ctx) return fail(PES_ERR_INVALID, "ctx is NULL");
   if (tiles_per_group < 1 || tiles_per_group > 4096 || blocks_per_cu < 1 || blocks_per_cu > 64)
     return fail(PES_ERR_INVALID, "schedule: tiles_per_group in [1, 4096], blocks_per_cu in [1, 64]");
-  const bool regroup = ctx->finalized && tiles_per_group != ctx->tiles_per_group;
   ctx->tiles_per_group = tiles_per_group;
   ctx->blocks_per_cu = blocks_per_cu;
-  if (!regroup) return PES_OK;
-  HIP_TRY(hipSetDevice(ctx->device));
-  HIP_TRY(hipDeviceSynchronize());  // a batch in flight reads the groups
-  return build_groups(ctx);
+  return PES_OK;
 }
 
 extern "C" int pes_context_set_rows_per_item(pes_context* ctx, int rows) {

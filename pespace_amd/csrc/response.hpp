@@ -93,6 +93,16 @@ struct BinWork {
   const int* tile_range;
 };
 
+// The groups of one tile range: a table (the first tile of each, and the end of the last), or equal
+// ones of `per` tiles (first null)
+struct RangeGroups {
+  const int* first;
+  int tile_begin, tile_end, per;
+  PES_HD int last(int t) const { return t < tile_end ? t : tile_end; }
+  PES_HD int begin(int g) const { return first ? first[g] : tile_begin + g * per; }
+  PES_HD int end(int g) const { return first ? first[g + 1] : last(tile_begin + (g + 1) * per); }
+};
+
 // Host side: the orbit constants of a detector (heliocentric orbit.py:189-228; geocentric
 // orbit.py:112-139 with the given rotation rate and reference source); arguments validated by
 // the caller.
