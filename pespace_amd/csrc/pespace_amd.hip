@@ -1920,7 +1920,8 @@ static size_t fine_doubles(const pes_context* ctx, int cap, bool grad) {
 static int ensure_scratch(pes_context* ctx, int P, bool grad) {
   {
     const size_t need = partial_doubles(ctx, (size_t)(P > ctx->cap_P ? P : ctx->cap_P));
-    const size_t fine = fine_doubles(ctx, P > ctx->cap_P ? P : ctx->cap_P, grad || ctx->cap_grad);
+    // (pinned: a small batch that the per-tile sums have no room for runs in items of whole groups)
+    const size_t fine = ctx->pinned ? 0 : fine_doubles(ctx, P > ctx->cap_P ? P : ctx->cap_P, grad || ctx->cap_grad);
     const bool grow =
         need > ctx->cap_partial || fine > ctx->cap_fine || P > ctx->cap_P || (grad && !ctx->cap_grad);
     if (grow && ctx->pinned)
@@ -1976,6 +1977,7 @@ struct BatchScratch {
   unsigned char* items;          // duty contexts only: [groups][chunks] plain (1) or duty (0)
   unsigned long long* dbits;     // panels: per row the tiles that go bin by bin (null: all of them)
   double* fine;                  // per-tile sums of a small batch (null: items of tiles_per_group tiles)
+  size_t cap_fine;               // doubles
 };
 
 static BatchScratch context_scratch(const pes_context* ctx) {
@@ -1985,7 +1987,7 @@ static BatchScratch context_scratch(const pes_context* ctx) {
           : nullptr;
   return {ctx->d_setup,   ctx->d_pconst,       ctx->d_nodes,    ctx->d_nodes_grad,
           ctx->d_partial, ctx->d_work_counter, ctx->d_off_bits, items, ctx->d_dbits,
-          ctx->d_fine};
+          ctx->d_fine,    ctx->cap_fine};
 }
 
 static int check_batch_args(const pes_context* ctx, const double* d_params, int P) {
@@ -2065,7 +2067,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   int grid = ctx->n_cu * ctx->blocks_per_cu;
   const bool panels = sc.dbits != nullptr;
   const bool direct = ctx->direct_lnl();
-  const bool fine = sc.fine && P < fine_rows(ctx);
+  const bool fine = sc.fine && P < fine_rows(ctx) && fine_doubles(ctx, P, grad) <= sc.cap_fine;
   const int rows = rows_per_item(ctx, P, grad, grid, panels, fine);
   const int n_chunks = (P + rows - 1) / rows;
   const int nout = grad ? 1 + PES_N_PARAMS : 1;
@@ -2285,6 +2287,7 @@ extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, i
     sc.items = ctx->any_duty ? reinterpret_cast<unsigned char*>(base + off[7]) : nullptr;
     sc.dbits = ctx->pan.tile_pan ? reinterpret_cast<unsigned long long*>(base + off[8]) : nullptr;
     sc.fine = nullptr;
+    sc.cap_fine = 0;
     const double* params = d_params + (size_t)p0 * PES_N_PARAMS;
     rc = launch_setup_nodes(ctx, sc, params, n, grad, ctx->direct_lnl(), st);
     if (rc == PES_OK)

@@ -71,3 +71,28 @@ def test_replays_keep_their_groups(span, P):
                 assert torch.equal(l_e, eager[now][k][0]) and torch.equal(g_e, eager[now][k][1]), (now, k)
     core.pin_scratch(False)
     del graphs
+
+
+@pytest.mark.parametrize("span", [4.0e6, 655360.0])
+def test_pinned_scratch_takes_a_schedule_with_fewer_groups(span):
+    """Fewer tile groups need no more scratch: more batches count as small then, and those that the
+    pinned sums of single tiles have no room for run in items of whole groups."""
+    from pespace_amd._lib import PespaceError
+    core = _core(span, ((2, 2), (3, 3)))
+    P = 400
+    rows = particle_cloud(P, seed=60, rel=1e-3, center=inj_row(coalescence_time=0.7 * span))
+    core.set_schedule(4, 4)
+    core.reserve(P, grad=True)
+    core.pin_scratch(True)
+    ref = core.lnl(rows, grad=True)
+    for per in (8, 64, 4096):
+        core.set_schedule(per, 4)
+        lnl, g = core.lnl(rows, grad=True)
+        assert torch.allclose(lnl, ref[0], rtol=1e-12, atol=0.0)
+        for p in (1, 150):  # batches of single tiles that fit: the same to the last bit
+            l_p, g_p = core.lnl(rows[:p], grad=True)
+            assert torch.equal(l_p, lnl[:p]) and torch.equal(g_p, g[:p])
+    core.set_schedule(1, 4)
+    with pytest.raises(PespaceError, match="pinned"):
+        core.lnl(rows, grad=True)
+    core.pin_scratch(False)
