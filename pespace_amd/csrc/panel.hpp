@@ -37,11 +37,6 @@
 #pragma once
 
 constexpr int PANEL_K = 5;              // interpolation points
-constexpr double PANEL_EPS = 1.4e-3;    // relative half-width of a panel, at most
-constexpr double PANEL_SWING = 3.0e-3;  // 2 pi (2 L) (f_hi - f_lo) and the orbit angles' turn, at most
-// tiles cut into more panels go bin by bin: a panel costs its points whatever its bins (a year of
-// the network, 1024 rows with the gradient: 5 panels at most 109.6 ms, 8 109.3, 12 110.3)
-constexpr int PANEL_MAX_PIECES = 8;
 constexpr int PANEL_MIN_TILES = 512;    // contexts with fewer panel tiles go bin by bin
 // doubles per panel: f_mid, 1 / f_half, f_half, s at its ends, -, then per point f, the Hermite
 // weights hb1 .. he3 and sin, cos of pi f L (BinPre), and a pad to 16 bytes

@@ -25,6 +25,7 @@
 #include "../../include/pespace_amd.h"
 #include "response.hpp"
 #include "mathfn.hpp"
+#include "panel_cut.hpp"
 
 using namespace pes;
 
@@ -1588,9 +1589,9 @@ static void free_dev(void* p) {
   if (p) (void)hipFree(p);
 }
 
-// Panels (panel.hpp): each tile is cut at its node interval ends, and each part into equal panels
-// within the truncation bounds; a tile of more than PANEL_MAX_PIECES stays bin by bin (its panels
-// would hold too few bins to pay for their points).  bf, bj: frequency and node interval per bin.
+// Panels (panel.hpp) of every tile (panel_cut); a tile of more than PANEL_MAX_PIECES stays bin by bin
+// (its panels would hold too few bins to pay for their points).  bf, bj: frequency and node interval
+// per bin.
 static int build_panels(pes_context* ctx, const std::vector<double>& bf, const std::vector<int>& bj) {
   if (ctx->direct) return PES_OK;
   // a context for responses alone (no channel enters the likelihood: lnL = 0) does without
@@ -1602,31 +1603,13 @@ static int build_panels(pes_context* ctx, const std::vector<double>& bf, const s
     const int t0 = h.d.bin_offset / TILE;
     for (int t = t0; t < t0 + h.d.n_tiles; ++t) {
       const int bin0 = t * TILE, nb = std::min(TILE, h.d.n_bins - (t - t0) * TILE);
-      int parts[3 * PANEL_MAX_PIECES], np = 0;  // (first bin in the tile, bins, node interval)
-      for (int a = 0; a < nb && np >= 0;) {
-        int e = a + 1;
-        while (e < nb && bj[bin0 + e] == bj[bin0 + a]) ++e;
-        const double lo = bf[bin0 + a], hi = bf[bin0 + e - 1];
-        const double cuts = std::max((hi - lo) / ((hi + lo) * PANEL_EPS), 4.0 * PI * h.d.L * (hi - lo) / PANEL_SWING);
-        const int k = cuts < (double)(e - a) ? std::max(1, (int)std::ceil(cuts)) : e - a;
-        if (np + k > PANEL_MAX_PIECES) {
-          np = -1;
-          break;
-        }
-        for (int i = 0; i < k; ++i) {
-          const int b0 = a + (int)((long long)(e - a) * i / k), b1 = a + (int)((long long)(e - a) * (i + 1) / k);
-          parts[3 * np] = b0;
-          parts[3 * np + 1] = b1 - b0;
-          parts[3 * np + 2] = bj[bin0 + a];
-          ++np;
-        }
-        a = e;
-      }
-      if (np <= 0) continue;
+      PanelCut parts[PANEL_MAX_PIECES];
+      const int np = panel_cut(&bf[bin0], &bj[bin0], nb, h.d.L, parts);
+      if (np == 0) continue;
       tp[2 * (size_t)t] = (int)(pi.size() / 4);
       tp[2 * (size_t)t + 1] = np;
       for (int k = 0; k < np; ++k) {
-        const int b0 = parts[3 * k], n = parts[3 * k + 1], j = parts[3 * k + 2];
+        const int b0 = parts[k].first, n = parts[k].bins, j = parts[k].node;
         const double lo = bf[bin0 + b0], hi = bf[bin0 + b0 + n - 1];
         const double mid = 0.5 * (lo + hi), half = std::max(0.5 * (hi - lo), 1e-9 * mid);  // one bin: any width
         double d[PAN_D] = {mid, 1.0 / half, half};
