@@ -1286,7 +1286,7 @@ struct pes_context {
   // tiles that go bin by bin all the same, and per tile the last batch in which a row does
   PanelDev pan{};
   int *d_tile_pan = nullptr, *d_pan_i = nullptr, *d_bin_work = nullptr;
-  BinWork bin_work{};
+  BinWork bin_work{}, bin_work_noalloc{};  // of the context's scratch, and of pes_lnl_batch_noalloc
   double* d_pan_d = nullptr;
   double2* d_pan_rec = nullptr;
   unsigned long long* d_dbits = nullptr;  // [cap_P][off_words]
@@ -1649,14 +1649,19 @@ static int build_panels(pes_context* ctx, const std::vector<double>& bf, const s
   HIP_TRY(hipMalloc(&ctx->d_pan_d, pd.size() * sizeof(double)));
   HIP_TRY(hipMalloc(&ctx->d_pan_rec, (size_t)ctx->NB * PANEL_REC * sizeof(double2)));
   constexpr int STATE = 64;  // ints before the first array
-  HIP_TRY(hipMalloc(&ctx->d_bin_work, (STATE + 4 * (size_t)nt) * sizeof(int)));
+  const size_t per_bw = STATE + 3 * (size_t)nt;
+  HIP_TRY(hipMalloc(&ctx->d_bin_work, (2 * per_bw + nt) * sizeof(int)));
   HIP_TRY(hipMemcpy(ctx->d_tile_pan, tp.data(), tp.size() * sizeof(int), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(ctx->d_pan_i, pi.data(), pi.size() * sizeof(int), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(ctx->d_pan_d, pd.data(), pd.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemset(ctx->d_bin_work, 0, (STATE + 4 * (size_t)nt) * sizeof(int)));
-  int* w = ctx->d_bin_work + STATE;
-  // (tile_group is that of the batch's groups)
-  ctx->bin_work = {ctx->d_bin_work, w, w + nt, w + 2 * (size_t)nt, nullptr, w + 3 * (size_t)nt};
+  HIP_TRY(hipMemset(ctx->d_bin_work, 0, (2 * per_bw + nt) * sizeof(int)));
+  for (int i = 0; i < 2; ++i) {
+    int* w = ctx->d_bin_work + i * per_bw;
+    int* arr = w + STATE;
+    // (tile_group is that of the batch's groups)
+    (i == 0 ? ctx->bin_work : ctx->bin_work_noalloc) = {w, arr, arr + nt, arr + 2 * (size_t)nt, nullptr,
+                                                        ctx->d_bin_work + 2 * per_bw};
+  }
   for (int i = 0; i < (int)ctx->hdets.size(); ++i)
     hipLaunchKernelGGL(k_panel_rec, dim3(ctx->hdets[i].d.n_tiles), dim3(TILE), 0, nullptr, ctx->d_dets, i,
                        ctx->d_bin_f, ctx->d_bin_s, ctx->d_bin_j, ctx->d_bin_rec, ctx->du, ctx->d_pan_rec);
@@ -1961,6 +1966,7 @@ struct BatchScratch {
   unsigned long long* dbits;     // panels: per row the tiles that go bin by bin (null: all of them)
   double* fine;                  // per-tile sums of a small batch (null: items of tiles_per_group tiles)
   size_t cap_fine;               // doubles
+  BinWork bin_work;              // panels
 };
 
 static BatchScratch context_scratch(const pes_context* ctx) {
@@ -1970,7 +1976,7 @@ static BatchScratch context_scratch(const pes_context* ctx) {
           : nullptr;
   return {ctx->d_setup,   ctx->d_pconst,       ctx->d_nodes,    ctx->d_nodes_grad,
           ctx->d_partial, ctx->d_work_counter, ctx->d_off_bits, items, ctx->d_dbits,
-          ctx->d_fine,    ctx->cap_fine};
+          ctx->d_fine,    ctx->cap_fine,       ctx->bin_work};
 }
 
 static int check_batch_args(const pes_context* ctx, const double* d_params, int P) {
@@ -1987,7 +1993,7 @@ static int launch_setup_nodes(const pes_context* ctx, const BatchScratch& sc, co
                               bool direct, hipStream_t st) {
   const dim3 sg((P + SETUP_ROWS - 1) / SETUP_ROWS);
   hipLaunchKernelGGL(k_setup, sg, dim3(192), 0, st, d_params, P, ctx->modes, ctx->f_ref, sc.setup, sc.pconst,
-                     sc.work_counter, ctx->bin_work.state);
+                     sc.work_counter, sc.bin_work.state);
   HIP_TRY(hipGetLastError());
   const int NNS = ctx->n_nodes + 1;
   dim3 g((NNS + 127) / 128, P * ctx->modes.n);
@@ -2083,7 +2089,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   groups.tile0[n_ranges] = ctx->n_tiles;
   groups.per = ctx->tiles_per_group;
   groups.first = panels ? group_table(ctx).d_first : nullptr;
-  BinWork bin_work = ctx->bin_work;
+  BinWork bin_work = sc.bin_work;
   if (panels) bin_work.tile_group = group_table(ctx).d_tile_group;
   // a launch's groups in range r; fine: its tiles
   auto range_groups = [&](int r) -> RangeGroups {
@@ -2271,6 +2277,7 @@ extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, i
     sc.dbits = ctx->pan.tile_pan ? reinterpret_cast<unsigned long long*>(base + off[8]) : nullptr;
     sc.fine = nullptr;
     sc.cap_fine = 0;
+    sc.bin_work = ctx->bin_work_noalloc;
     const double* params = d_params + (size_t)p0 * PES_N_PARAMS;
     rc = launch_setup_nodes(ctx, sc, params, n, grad, ctx->direct_lnl(), st);
     if (rc == PES_OK)
