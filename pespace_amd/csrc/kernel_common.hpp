@@ -12,6 +12,7 @@ constexpr int chunk_rows() { return GRAD ? 48 : 160; }
 // default schedule: tiles per work item (8: the fastest in every timed schedule table of the
 // one-year network, 4-7% ahead of 32 on 512-row samples) ...
 constexpr int TILES_PER_GROUP = 8;
+constexpr int MAX_TILES_PER_GROUP = 4096;
 constexpr int BLOCKS_PER_CU = 4;     // ... and persistent blocks launched per CU
 constexpr int MAX_MODES = 6;         // modes per context (ModeList)
 // node rows per tile that the fused kernel stages in LDS (tiles spanning more read them from

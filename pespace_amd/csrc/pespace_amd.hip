@@ -1281,6 +1281,9 @@ struct pes_context {
   double *d_setup = nullptr, *d_pconst = nullptr, *d_nodes = nullptr, *d_nodes_grad = nullptr,
          *d_partial = nullptr;
   int* d_work_counter = nullptr;
+  // scratch of one row of pes_lnl_batch_noalloc, where it is accounted within the fixed array but needs
+  // more (noalloc_row)
+  char* d_noalloc_row = nullptr;
   unsigned long long* d_off_bits = nullptr;  // [cap_P][off_words] duty off-tile flags (duty contexts)
   // panels of the tiles that the panel kernel takes (none: pan.tile_pan is null); per row the
   // tiles that go bin by bin all the same, and per tile the last batch in which a row does
@@ -1550,9 +1553,11 @@ static int noalloc_base(int device, char** out) {
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// What a batch is accounted for against the array: the layout of a batch whose tile groups all
-// hold tiles_per_group tiles, without the panels' flags
-constexpr size_t N_SETUP_ACC = N_SU_USED - 7;  // without the precomputed powers
+// What a batch is accounted for against the array: scratch for tile groups of tiles_per_group tiles
+// each and a setup table of the model's own coefficients.  Panels take more (their flags, more
+// groups), as do the table's precomputed powers; contexts evaluated at every bin take less with the
+// gradient.  The account alone decides what is accepted
+constexpr size_t N_SETUP_ACC = SU_IETA;  // the first of the precomputed ones
 static size_t noalloc_account(const pes_context* ctx, int P, bool grad) {
   const size_t NNS = (size_t)ctx->n_nodes + 1, rows = (size_t)P, nm = (size_t)ctx->modes.n;
   TileRange r[MAX_TILE_RANGES];
@@ -1567,8 +1572,9 @@ static size_t noalloc_account(const pes_context* ctx, int P, bool grad) {
   if (ctx->any_duty) o += align256(rows * off_words_of(ctx) * sizeof(unsigned long long)) + align256(groups * rows);
   return o;
 }
-// byte offsets of the scratch buffers of P rows inside the array, and their total.  A batch that
-// is accounted within the array but needs more runs in parts (rows do not depend on their batch)
+// byte offsets of the scratch buffers of P rows inside the array, and their total.  A batch that is
+// accounted within the array but needs more runs in parts (rows do not depend on their batch), down to
+// single rows; where even one needs more, the context has room for it (noalloc_row)
 static size_t noalloc_layout(const pes_context* ctx, int P, bool grad, size_t off[9]) {
   const size_t NNS = (size_t)ctx->n_nodes + 1, rows = (size_t)P, nm = (size_t)ctx->modes.n;
   size_t o = 0;
@@ -1583,6 +1589,22 @@ static size_t noalloc_layout(const pes_context* ctx, int P, bool grad, size_t of
   off[7] = o; if (ctx->any_duty) o += align256((size_t)n_groups_of(ctx) * rows);  // work items: plain or duty
   off[8] = o; if (ctx->pan.tile_pan) o += align256(rows * off_words_of(ctx) * sizeof(unsigned long long));
   return o;
+}
+
+// Allocates d_noalloc_row where a row may be accepted (its account is least with the largest groups)
+// and need more than the array (its layout is largest with groups of one tile)
+static int noalloc_row(pes_context* ctx) {
+  const int set = ctx->tiles_per_group;
+  size_t most = 0, off[9];
+  for (int grad = 0; grad < 2; ++grad) {
+    ctx->tiles_per_group = MAX_TILES_PER_GROUP;
+    if (noalloc_account(ctx, 1, grad != 0) > (size_t)PES_NOALLOC_SCRATCH_BYTES) continue;
+    ctx->tiles_per_group = 1;
+    most = std::max(most, noalloc_layout(ctx, 1, grad != 0, off));
+  }
+  ctx->tiles_per_group = set;
+  if (most > (size_t)PES_NOALLOC_SCRATCH_BYTES) HIP_TRY(hipMalloc(&ctx->d_noalloc_row, most));
+  return PES_OK;
 }
 
 static void free_dev(void* p) {
@@ -1824,6 +1846,7 @@ extern "C" int pes_context_finalize(pes_context* ctx) {
   {
     int rc = build_panels(ctx, bf, bj);
     if (rc == PES_OK) rc = build_groups(ctx);
+    if (rc == PES_OK) rc = noalloc_row(ctx);
     if (rc != PES_OK) return rc;
   }
   HIP_TRY(hipMalloc(&ctx->d_work_counter, N_WORK_COUNTERS * sizeof(int)));  // one per fused-kernel launch
@@ -1862,6 +1885,7 @@ extern "C" void pes_context_destroy(pes_context* ctx) {
   free_dev(ctx->d_bin_work);
   free_dev(ctx->d_fine);
   free_dev(ctx->d_groups);
+  free_dev(ctx->d_noalloc_row);
   free_dev(ctx->d_partial);
   free_dev(ctx->d_live);
   for (auto e : ctx->ev_start) (void)hipEventDestroy(e);
@@ -2259,8 +2283,7 @@ extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, i
   size_t off[9];
   int part = P;
   while (part > 1 && noalloc_layout(ctx, part, grad, off) > (size_t)PES_NOALLOC_SCRATCH_BYTES) part = (part + 1) / 2;
-  if (noalloc_layout(ctx, part, grad, off) > (size_t)PES_NOALLOC_SCRATCH_BYTES)
-    return fail(PES_ERR_INVALID, "pes_lnl_batch_noalloc: one row needs more than the fixed scratch");
+  if (noalloc_layout(ctx, part, grad, off) > (size_t)PES_NOALLOC_SCRATCH_BYTES) base = ctx->d_noalloc_row;
   hipStream_t st = (hipStream_t)stream;
   for (int p0 = 0; p0 < P; p0 += part) {
     const int n = std::min(part, P - p0);
@@ -2570,7 +2593,7 @@ extern "C" int pes_whittle_lnl(const double* d_data, const double* d_resp, const
 
 extern "C" int pes_context_set_schedule(pes_context* ctx, int tiles_per_group, int blocks_per_cu) {
   if (!ctx) return fail(PES_ERR_INVALID, "ctx is NULL");
-  if (tiles_per_group < 1 || tiles_per_group > 4096 || blocks_per_cu < 1 || blocks_per_cu > 64)
+  if (tiles_per_group < 1 || tiles_per_group > MAX_TILES_PER_GROUP || blocks_per_cu < 1 || blocks_per_cu > 64)
     return fail(PES_ERR_INVALID, "schedule: tiles_per_group in [1, 4096], blocks_per_cu in [1, 64]");
   ctx->tiles_per_group = tiles_per_group;
   ctx->blocks_per_cu = blocks_per_cu;
