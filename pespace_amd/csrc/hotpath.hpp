@@ -181,6 +181,9 @@ constexpr bool kDuty = (KIND & 2) != 0;
 // adjoints go to the same places of the array that holds the node gradients otherwise
 template <int KIND>
 constexpr bool kDirect = (KIND & 4) != 0;
+// that array: read, but for the direct variant's adjoints
+template <int KIND, bool GRAD = true>
+using GradPtr = typename std::conditional<kDirect<KIND> && GRAD, double*, const double*>::type;
 
 struct ModeG {
   double A, t;      // amplitude, t_f + t_c
@@ -528,7 +531,7 @@ struct AdjAcc {
 // uslot: this lane's LDS slot of the mode's unit phasor, stored by the forward pass
 template <int PREC, int KIND>
 __device__ inline void mode_adjoint(const DetectorDev& det, const double* __restrict__ mf, int mid,
-                                    const double* __restrict__ n0, const double* __restrict__ g0, const BinPre& b,
+                                    const double* __restrict__ n0, GradPtr<KIND> __restrict__ g0, const BinPre& b,
                                     const RowC& rc, const Cx wl[6], const double* __restrict__ pc,
                                     AdjAcc& acc, double* __restrict__ uslot) {
   ModeG g;
@@ -639,10 +642,9 @@ __device__ inline void mode_adjoint(const DetectorDev& det, const double* __rest
   }
   acc.tc = fma(2.0 * b.pif, phib, acc.tc + tb);
   if constexpr (kDirect<KIND>) {
-    double* a = const_cast<double*>(g0);
-    a[0] = Ab;
-    a[TILE] = phib;
-    a[2 * TILE] = tb * b.he2;
+    g0[0] = Ab;
+    g0[TILE] = phib;
+    g0[2 * TILE] = tb * b.he2;
     return;
   }
   // intrinsic parameters through the node tables: weights of the eight node entries
@@ -789,7 +791,7 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
                                  const double* __restrict__ bin_f, const int* __restrict__ bin_j,
                                  const double* __restrict__ bin_s, const double* __restrict__ bin_rec,
                                  const double* __restrict__ tile_dd, const double* __restrict__ pconst,
-                                 const double* __restrict__ nodes, const double* __restrict__ nodes_grad, int NNS,
+                                 const double* __restrict__ nodes, GradPtr<KIND, GRAD> __restrict__ nodes_grad, int NNS,
                                  double du, const ModeList& modes, int lane, int wave, double* acc, int j0,
                                  int nj, double* stage_n, double* stage_g, int& buf,
                                  const unsigned long long* __restrict__ off_bits, int n_tiles, double* lane_lds,
@@ -879,7 +881,7 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
         }
       };
       const double* nb;  // node entries of this lane's bin, mode 0, and the per-mode strides
-      const double* gb;
+      GradPtr<KIND, GRAD> gb;
       size_t nstride, gstride;
       if constexpr (STAGED) {
         int qn = p + 1;  // next evaluated row
@@ -926,7 +928,7 @@ __device__ inline void tile_rows(const DetectorDev& det, int tile, double f0, in
         v -= wc * fma(rr, rr, ri * ri);
         wch[ch] = {2.0 * wc * rr, 2.0 * wc * ri};
       }
-      if (GRAD) {
+      if constexpr (GRAD) {
         Cx wX, wY, wZ, wT = {0.0, 0.0};
         if (det.orthogonal) {
           const double r2 = 0.70710678118654752440, r6 = 0.40824829046386301637;
@@ -1027,7 +1029,7 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
                                               const double* __restrict__ tile_f0, const double* __restrict__ tile_dd,
                                               RangeGroups grp, int n_grp, const double* __restrict__ pconst,
                                               const double* __restrict__ nodes,
-                                              const double* __restrict__ nodes_grad, int NNS, double du,
+                                              GradPtr<KD, GRAD> __restrict__ nodes_grad, int NNS, double du,
                                               ModeList modes, int P, int rows, const int* __restrict__ tile_jr,
                                               int group_offset,
                                               int* __restrict__ work_counter, double* __restrict__ partial,
