@@ -5,7 +5,9 @@
 // of a term is a multiple of the term: values and slopes come from the same powers.  The powers of y
 // are products of those of f, which are the same for all rows and tabulated per node or bin, and of
 // those of the mass in seconds, which are constants of the row: no cube root, logarithm or power is
-// taken per (row, frequency) outside a higher mode's merger.
+// taken per (row, frequency) outside a higher mode's merger.  One Newton step from y itself takes the
+// products' roundings out again (y_powers): without it A and Psi were 1.5 times further from
+// extended precision than with the functions taken per frequency (tests/test_host_nodes_error.py).
 // su: the row's setup table [5][N_SETUP].
 #pragma once
 
@@ -19,28 +21,41 @@ struct FreqPow {
 PES_HD FreqPow load_fpow(const double* t, size_t n, size_t i) {
   return {t[i], t[n + i], t[2 * n + i], t[3 * n + i], t[4 * n + i]};
 }
+PES_HD FreqPow freq_pow(double f) {
+  const double c = cbrt(f), ic = 1.0 / c;
+  return {f, c, ic, log(f), ic * ic * ic * sqrt(ic)};
+}
 
 struct NodeY {
   double x, y, r;          // M f, f22, d ln y / d ln x
   double c, ic, l, y76;    // y^(1/3), y^(-1/3), ln y, y^(-7/6)
 };
+// y^(1/3), y^(-1/3) and y^(-7/6) of y + yl from i = y^(-1/3) and p = y^(-7/6) to a few roundings: the
+// residual 1 - (y + yl) i^3, formed with the products' rounding errors, corrects all of them
+PES_HD void y_powers(double y, double yl, double i, double p, NodeY& o) {
+  const double i2 = i * i, e2 = fma(i, i, -i2);
+  const double i3 = i2 * i, e3 = fma(e2, i, fma(i2, i, -i3));
+  const double t = fma(-y, i3, 1.0) - fma(y, e3, yl * i3);
+  const double h = y * i2;
+  o.ic = fma(i, t * (1.0 / 3.0), i);
+  o.c = h + (fma(y, i2, -h) + fma(y, e2, fma(yl, i2, h * (t * (2.0 / 3.0)))));
+  const double s = p * y;  // y^(-1/6), corrected by its square
+  o.y76 = fma(i3, t, i3) * fma(0.5 * s * o.c, fma(-s, s, o.ic), s);
+}
 PES_HD int su_frd(int mode) {
   return mode == 1 ? SU_FRD21 : mode == 2 ? SU_FRD33 : mode == 3 ? SU_FRD32 : mode == 4 ? SU_FRD44
          : mode == 5 ? SU_FRD43 : SU_FRD;
 }
-// (2 / m)^(1/3), its inverse, ln(2 / m), (2 / m)^(-7/6), (2 pi / m)^(1/3) for m = 1, 2, 3, 4
+// (2 / m)^(-1/3), ln(2 / m), (2 / m)^(-7/6), (2 pi / m)^(1/3) for m = 1, 2, 3, 4
 struct ModePow {
-  double c, ic, l, p76, pi13;
+  double ic, l, p76, pi13;
 };
 PES_HD ModePow mode_pow(int m) {
   switch (m) {
-    case 1: return {1.2599210498948731648, 0.79370052598409973738, 0.69314718055994530942, 0.44544935907016965237,
-                    1.8452701486440284191};
-    case 2: return {1.0, 1.0, 0.0, 1.0, 1.4645918875615232630};
-    case 3: return {0.87358046473629886905, 1.1447142425533318678, -0.40546510810816438198, 1.6048697909004944263,
-                    1.2794388617850086711};
-    default: return {0.79370052598409973738, 1.2599210498948731648, -0.69314718055994530942, 2.2449240966187459629,
-                     1.1624473515096264756};
+    case 1: return {0.79370052598409973738, 0.69314718055994530942, 0.44544935907016965237, 1.8452701486440284191};
+    case 2: return {1.0, 0.0, 1.0, 1.4645918875615232630};
+    case 3: return {1.1447142425533318678, -0.40546510810816438198, 1.6048697909004944263, 1.2794388617850086711};
+    default: return {1.2599210498948731648, -0.69314718055994530942, 2.2449240966187459629, 1.1624473515096264756};
   }
 }
 PES_HD NodeY node_y(const double* su, int mode, const FreqPow& q) {
@@ -49,19 +64,19 @@ PES_HD NodeY node_y(const double* su, int mode, const FreqPow& q) {
   o.r = 1.0;
   const double m = (double)kModeM[mode], fi = 0.5 * m * HM_MAP_JOIN;
   if (mode == 0 || o.x < fi) {
+    double yl = fma(q.f, su[SU_MSEC], -o.x), i = q.ic * su[SU_IM13], p = q.f76 * su[SU_M76];
     o.y = o.x;
-    o.c = q.c * su[SU_M13];
-    o.ic = q.ic * su[SU_IM13];
     o.l = q.l + su[SU_LNM];
-    o.y76 = q.f76 * su[SU_M76];
     if (kModeM[mode] != 2) {
       const ModePow k = mode_pow(kModeM[mode]);
-      o.y *= 2.0 / m;
-      o.c *= k.c;
-      o.ic *= k.ic;
+      const double h = 2.0 / m;
+      o.y = o.x * h;
+      yl = fma(yl, h, fma(o.x, h, -o.y));
+      i *= k.ic;
+      p *= k.p76;
       o.l += k.l;
-      o.y76 *= k.p76;
     }
+    y_powers(o.y, yl, i, p, o);
     return o;
   }
   const double fr = su[su_frd(mode)], FRD = su[SU_FRD], rho = FRD / fr;
@@ -77,34 +92,36 @@ PES_HD NodeY node_y(const double* su, int mode, const FreqPow& q) {
   o.c = cbrt(o.y);
   o.ic = 1.0 / o.c;
   o.l = log(o.y);
-  o.y76 = o.ic * o.ic * o.ic * sqrt(o.ic);
+  o.y76 = sqrt(o.ic) / o.y;
   return o;
 }
 // v = cbrt(2 pi x / m) up to the join and saturating above it, and x dv/dx
-PES_HD void node_beta_v(const double* su, int mode, const FreqPow& q, double x, double& v, double& Dv) {
-  const double fi = 0.5 * (double)kModeM[mode] * HM_MAP_JOIN;
-  const double vr = q.c * su[SU_M13] * mode_pow(kModeM[mode]).pi13;
-  if (x < fi) {
-    v = vr;
-    Dv = vr * (1.0 / 3.0);
+PES_HD void node_beta_v(const double* su, int mode, const FreqPow& q, const NodeY& n, double& v, double& Dv) {
+  const double m = (double)kModeM[mode];
+  if (n.x < 0.5 * m * HM_MAP_JOIN) {  // 2 x / m = y
+    v = fma(n.c, 1.4645918875615231, n.c * 1.0150910436435383e-16);  // pi^(1/3), and what that is rounded by
+    Dv = v * (1.0 / 3.0);
   } else {
+    const double k = mode_pow(kModeM[mode]).pi13, i = q.ic * su[SU_IM13] / k, X = n.x * (2.0 * PI / m);
+    double vr = q.c * su[SU_M13] * k;
+    vr = fma(vr * (1.0 / 3.0), (X - vr * vr * vr) * (i * i * i), vr);  // the products' roundings, as in y_powers
     const double vi = cbrt(PI * HM_MAP_JOIN), e = exp(1.0 - vr / vi);
     v = vi * (2.0 - e);
     Dv = e * vr * (1.0 / 3.0);
   }
 }
-// beta = b1 v + b2 v^2 + b3 v^3
+// beta = k (b1 v + b2 v^2 + b3 v^3)
 struct NodeBeta {
-  double b1, b2, b3;
+  double k, b1, b2, b3;
 };
 PES_HD NodeBeta node_beta(const double* su, int mode) {
   const double d = su[SU_DELTA], eta = su[SU_ETA];
   switch (mode) {
-    case 1: return {sqrt(2.0) / 3.0 * d, -sqrt(2.0) / 2.0 * (su[SU_CHIA] + d * su[SU_CHIS]), 0.0};
-    case 2: return {sqrt(2.0 / 3.0) * 0.75 * sqrt(15.0 / 14.0) * d, 0.0, 0.0};
-    case 3: return {0.0, (1.0 / 3.0) * sqrt(5.0 / 7.0) * (1.0 - 3.0 * eta), 0.0};
-    case 4: return {0.0, sqrt(0.5) * (8.0 / 9.0) * sqrt(5.0 / 7.0) * (1.0 - 3.0 * eta), 0.0};
-    default: return {0.0, 0.0, sqrt(2.0 / 3.0) * (9.0 / (4.0 * sqrt(70.0))) * d * (1.0 - 2.0 * eta)};
+    case 1: return {sqrt(2.0) / 3.0, d, -1.5 * (su[SU_CHIA] + d * su[SU_CHIS]), 0.0};
+    case 2: return {sqrt(2.0 / 3.0) * 0.75 * sqrt(15.0 / 14.0), d, 0.0, 0.0};
+    case 3: return {(1.0 / 3.0) * sqrt(5.0 / 7.0), 0.0, 1.0 - 3.0 * eta, 0.0};
+    case 4: return {sqrt(0.5) * (8.0 / 9.0) * sqrt(5.0 / 7.0), 0.0, 1.0 - 3.0 * eta, 0.0};
+    default: return {sqrt(2.0 / 3.0) * (9.0 / (4.0 * sqrt(70.0))), 0.0, 0.0, d * (1.0 - 2.0 * eta)};
   }
 }
 // w, the taper over the end of the mode's range, and x dw/dx
@@ -135,9 +152,10 @@ PES_HD void node_red(const double* su, double y, double c, double& red, double& 
     red = exp(-d * g) * (F * k(SU_G1)) * den;
     Dred = -y * red * (g + 2.0 * d * den);
   } else {
-    const double d1 = k(SU_D1), d2 = k(SU_D2), d3 = k(SU_D3), d4 = k(SU_D4);
-    red = k(SU_D0) + y * (d1 + y * (d2 + y * (d3 + y * d4)));
-    Dred = y * (d1 + y * (2.0 * d2 + y * (3.0 * d3 + y * (4.0 * d4))));
+    // value and slope by one Horner scheme: the sums cancel, and the slope of what was computed errs less
+    const double d4 = k(SU_D4), p3 = fma(d4, y, k(SU_D3)), p2 = fma(p3, y, k(SU_D2)), p1 = fma(p2, y, k(SU_D1));
+    red = fma(p1, y, k(SU_D0));
+    Dred = y * fma(fma(fma(d4, y, p3), y, p2), y, p1);
   }
 }
 // phase phi(y) before the alignment, and G = y d phi / dy; l = log(y)
@@ -157,14 +175,15 @@ PES_HD void node_phi(const double* su, double y, double c, double ic, double l, 
     phi = ps * e - t;
     G = gs * e - g;
   } else if (y >= 0.5 * k(SU_FRD)) {
-    const double y34 = sqrt(y) * sqrt(sqrt(y)), iy = 1.0 / y, u = 1.0 / k(SU_FDM);
+    const double y34 = sqrt(y * sqrt(y)), iy = 1.0 / y, u = 1.0 / k(SU_FDM);
     const double z = (y - k(SU_AL5) * k(SU_FRD)) * u;
     const double c2 = k(SU_C2MRD) * y, b1 = k(SU_AL1) * y, b2 = k(SU_AL2) * iy, b3 = k(SU_AL3) * y34;
-    phi = (b1 - b2 + (4.0 / 3.0) * b3 + k(SU_AL4) * atan(z)) * e + k(SU_C1MRD) + c2;
+    phi = fma(fma(k(SU_AL1), y, fma(4.0 / 3.0, b3, -b2)) + k(SU_AL4) * atan(z), e, k(SU_C1MRD) + c2);
     G = (b1 + b2 + b3 + k(SU_AL4) * (y * u) / (1.0 + z * z)) * e + c2;
   } else {
     const double iy = 1.0 / y, b3 = k(SU_B3) * (iy * iy * iy), b1 = k(SU_B1) * y, c2 = k(SU_C2INT) * y;
-    phi = (b1 - (1.0 / 3.0) * b3 + k(SU_B2) * l) * e + k(SU_C1INT) + c2;
+    // (ln y anew: in the sum of logarithms those of f and M nearly cancel here)
+    phi = (b1 - (1.0 / 3.0) * b3 + k(SU_B2) * log(y)) * e + k(SU_C1INT) + c2;
     G = (b1 + b3 + k(SU_B2)) * e + c2;
   }
 }
@@ -177,9 +196,10 @@ PES_HD void node_values(const double* su, int mode, const FreqPow& q, double& A,
   double am = red * pre, Dam = (Dred - (7.0 / 6.0) * red) * pre * n.r;
   if (mode != 0) {
     double v, Dv;
-    node_beta_v(su, mode, q, n.x, v, Dv);
+    node_beta_v(su, mode, q, n, v, Dv);
     const NodeBeta b = node_beta(su, mode);
-    const double be = v * (b.b1 + v * (b.b2 + v * b.b3)), Dbe = Dv * (b.b1 + v * (2.0 * b.b2 + 3.0 * v * b.b3));
+    const double be = b.k * (v * (b.b1 + v * (b.b2 + v * b.b3)));
+    const double Dbe = b.k * (Dv * (b.b1 + v * (2.0 * b.b2 + 3.0 * v * b.b3)));
     Dam = Dam * be + am * Dbe;
     am *= be;
   }
@@ -242,7 +262,7 @@ PES_HD void node_adjoint(const double* su, int mode, const FreqPow& fq, double w
       add(SU_P6L, -c * (ap * L + ag * ((1.0 / 3.0) * L + 1.0)));
       add(SU_P7, -c2 * (ap + (2.0 / 3.0) * ag));
     } else if (y >= 0.5 * k(SU_FRD)) {
-      const double y34 = sqrt(y) * sqrt(sqrt(y)), iy = 1.0 / y, u = 1.0 / k(SU_FDM), FRD = k(SU_FRD);
+      const double y34 = sqrt(y * sqrt(y)), iy = 1.0 / y, u = 1.0 / k(SU_FDM), FRD = k(SU_FRD);
       const double z = (y - k(SU_AL5) * FRD) * u, n = 1.0 / (1.0 + z * z), q = y * u * n, at = atan(z);
       const double b1 = k(SU_AL1) * y, b2 = k(SU_AL2) * iy, b3 = k(SU_AL3) * y34, a4 = k(SU_AL4);
       const double c2 = k(SU_C2MRD) * y;
@@ -265,10 +285,11 @@ PES_HD void node_adjoint(const double* su, int mode, const FreqPow& fq, double w
       const double c2 = k(SU_C2INT) * y;
       G = (b1 + b3 + k(SU_B2)) * e + c2;
       DG = (b1 - 3.0 * b3) * e + c2;
-      aE += ap * (b1 - (1.0 / 3.0) * b3 + k(SU_B2) * l) + ag * (b1 + b3 + k(SU_B2));
+      const double ly = log(y);
+      aE += ap * (b1 - (1.0 / 3.0) * b3 + k(SU_B2) * ly) + ag * (b1 + b3 + k(SU_B2));
       add(SU_B1, e * y * as);
       add(SU_B3, e * iy3 * (ag - (1.0 / 3.0) * ap));
-      add(SU_B2, e * (ap * l + ag));
+      add(SU_B2, e * (ap * ly + ag));
       add(SU_C1INT, ap);
       add(SU_C2INT, y * as);
     }
@@ -287,11 +308,11 @@ PES_HD void node_adjoint(const double* su, int mode, const FreqPow& fq, double w
     const double aS = wA * w;  // adjoint of beta am
     if (mode != 0) {
       double v, Dv;
-      node_beta_v(su, mode, fq, x, v, Dv);
+      node_beta_v(su, mode, fq, nd, v, Dv);
       const NodeBeta b = node_beta(su, mode);
-      be = v * (b.b1 + v * (b.b2 + v * b.b3));
+      be = b.k * (v * (b.b1 + v * (b.b2 + v * b.b3)));
       const double ab = aS * am;
-      X += ab * Dv * (b.b1 + v * (2.0 * b.b2 + 3.0 * v * b.b3));
+      X += ab * b.k * Dv * (b.b1 + v * (2.0 * b.b2 + 3.0 * v * b.b3));
       const double d = k(SU_DELTA), eta = k(SU_ETA);
       if (mode == 1) {
         const double v2 = -sqrt(2.0) / 2.0 * v * v * ab;

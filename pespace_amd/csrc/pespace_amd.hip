@@ -202,11 +202,11 @@ __global__ __launch_bounds__(192) void k_setup(const double* __restrict__ params
 __global__ __launch_bounds__(128) void k_fpow(int n, double* __restrict__ t) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
-  const double f = t[j], c = cbrt(f), ic = 1.0 / c;
-  t[n + j] = c;
-  t[2 * (size_t)n + j] = ic;
-  t[3 * (size_t)n + j] = log(f);
-  t[4 * (size_t)n + j] = ic * ic * ic * sqrt(ic);
+  const FreqPow q = freq_pow(t[j]);
+  t[n + j] = q.c;
+  t[2 * (size_t)n + j] = q.ic;
+  t[3 * (size_t)n + j] = q.l;
+  t[4 * (size_t)n + j] = q.f76;
 }
 
 // ---- k_nodes ---------------------------------------------------------------------------
