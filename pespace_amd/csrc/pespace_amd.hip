@@ -198,11 +198,14 @@ __global__ __launch_bounds__(192) void k_setup(const double* __restrict__ params
   mf[MF_DFPR] = dFp.re; mf[MF_DFPI] = dFp.im; mf[MF_DFCR] = dFc.re; mf[MF_DFCI] = dFc.im;
 }
 
-// the powers of n frequencies (t[0 .. n - 1]) that node_eval.hpp takes, once per context
-__global__ __launch_bounds__(128) void k_fpow(int n, double* __restrict__ t) {
+// n frequencies (those given, or the nodes exp(u0 + j du)) and the powers of them that node_eval.hpp
+// takes, once per context
+__global__ __launch_bounds__(128) void k_fpow(int n, const double* __restrict__ given, double u0, double du,
+                                              double* __restrict__ t) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
-  const FreqPow q = freq_pow(t[j]);
+  const FreqPow q = freq_pow(given ? given[j] : exp(u0 + du * (double)j));
+  t[j] = q.f;
   t[n + j] = q.c;
   t[2 * (size_t)n + j] = q.ic;
   t[3 * (size_t)n + j] = q.l;
@@ -1265,7 +1268,7 @@ struct pes_context {
   double *d_bin_f = nullptr, *d_bin_s = nullptr;
   double* d_bin_rec = nullptr;  // per bin: (w, Re d, Im d) of the three channels and one pad, 80 B
   int* d_bin_j = nullptr;
-  double *d_tile_f0 = nullptr, *d_tile_dd = nullptr;  // first frequency and sum w |d|^2 per tile
+  double *d_tile_f0 = nullptr, *d_tile_dd = nullptr;  // first frequency and sum w |d|^2 per tile (one array)
   int* d_tile_jr = nullptr;  // per tile: first node index and number of node rows its bins use
   double* d_fpow = nullptr;  // [N_FPOW][n_nodes] the nodes' (direct mode: the bins') frequencies and their powers
   // scratch, grown on demand; while pinned (a captured HIP graph holds its pointers) it is
@@ -1688,7 +1691,6 @@ static int build_panels(pes_context* ctx, const std::vector<double>& bf, const s
     hipLaunchKernelGGL(k_panel_rec, dim3(ctx->hdets[i].d.n_tiles), dim3(TILE), 0, nullptr, ctx->d_dets, i,
                        ctx->d_bin_f, ctx->d_bin_s, ctx->d_bin_j, ctx->d_bin_rec, ctx->du, ctx->d_pan_rec);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipDeviceSynchronize());  // the record is read on the callers' streams
   ctx->tile_panels.resize(nt);
   ctx->tile_pan0.assign(nt + 1, 0);
   for (int t = 0; t < nt; ++t) {
@@ -1790,6 +1792,11 @@ extern "C" int pes_context_finalize(pes_context* ctx) {
   HIP_TRY(hipMalloc(&ctx->d_bin_j, NB * sizeof(int)));
   HIP_TRY(hipMalloc(&ctx->d_bin_rec, BIN_REC * (size_t)NB * sizeof(double)));
   HIP_TRY(hipMemcpy(ctx->d_bin_f, bf.data(), NB * sizeof(double), hipMemcpyHostToDevice));
+  // (runs beside the host's work and the copies that follow; waited for below)
+  HIP_TRY(hipMalloc(&ctx->d_fpow, (size_t)N_FPOW * ctx->n_nodes * sizeof(double)));
+  hipLaunchKernelGGL(k_fpow, dim3((ctx->n_nodes + 127) / 128), dim3(128), 0, nullptr, ctx->n_nodes,
+                     ctx->direct ? ctx->d_bin_f : nullptr, ctx->u0, ctx->du, ctx->d_fpow);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpy(ctx->d_bin_s, bs.data(), NB * sizeof(double), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(ctx->d_bin_j, bj.data(), NB * sizeof(int), hipMemcpyHostToDevice));
   {
@@ -1804,21 +1811,20 @@ extern "C" int pes_context_finalize(pes_context* ctx) {
   }
   {
     const int nt = ctx->n_tiles;
-    std::vector<double> tf0(nt), tdd(nt, 0.0);
+    std::vector<double> tf(2 * (size_t)nt);  // f0, dd
     for (int t = 0; t < nt; ++t) {
-      tf0[t] = bf[(size_t)t * TILE];
+      tf[t] = bf[(size_t)t * TILE];
       double s = 0.0;
       for (int ch = 0; ch < 3; ++ch)
         for (int k = 0; k < TILE; ++k) {
           const size_t i = (size_t)ch * NB + (size_t)t * TILE + k;
           s += bw[i] * (dre[i] * dre[i] + dim[i] * dim[i]);
         }
-      tdd[t] = s;
+      tf[nt + t] = s;
     }
-    HIP_TRY(hipMalloc(&ctx->d_tile_f0, nt * sizeof(double)));
-    HIP_TRY(hipMalloc(&ctx->d_tile_dd, nt * sizeof(double)));
-    HIP_TRY(hipMemcpy(ctx->d_tile_f0, tf0.data(), nt * sizeof(double), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(ctx->d_tile_dd, tdd.data(), nt * sizeof(double), hipMemcpyHostToDevice));
+    HIP_TRY(hipMalloc(&ctx->d_tile_f0, tf.size() * sizeof(double)));
+    HIP_TRY(hipMemcpy(ctx->d_tile_f0, tf.data(), tf.size() * sizeof(double), hipMemcpyHostToDevice));
+    ctx->d_tile_dd = ctx->d_tile_f0 + nt;
     // node rows j .. j+1 of every bin of a tile (node indices are non-decreasing with f)
     std::vector<int> tjr(2 * (size_t)nt);
     for (int t = 0; t < nt; ++t) {
@@ -1828,20 +1834,6 @@ extern "C" int pes_context_finalize(pes_context* ctx) {
     }
     HIP_TRY(hipMalloc(&ctx->d_tile_jr, 2 * (size_t)nt * sizeof(int)));
     HIP_TRY(hipMemcpy(ctx->d_tile_jr, tjr.data(), 2 * (size_t)nt * sizeof(int), hipMemcpyHostToDevice));
-  }
-  {
-    const int n = ctx->n_nodes;
-    HIP_TRY(hipMalloc(&ctx->d_fpow, (size_t)N_FPOW * n * sizeof(double)));
-    if (ctx->direct) {
-      HIP_TRY(hipMemcpy(ctx->d_fpow, ctx->d_bin_f, (size_t)n * sizeof(double), hipMemcpyDeviceToDevice));
-    } else {
-      std::vector<double> f(n);
-      for (int j = 0; j < n; ++j) f[j] = std::exp(ctx->u0 + ctx->du * (double)j);
-      HIP_TRY(hipMemcpy(ctx->d_fpow, f.data(), (size_t)n * sizeof(double), hipMemcpyHostToDevice));
-    }
-    hipLaunchKernelGGL(k_fpow, dim3((n + 127) / 128), dim3(128), 0, nullptr, n, ctx->d_fpow);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(nullptr));
   }
   {
     int rc = build_panels(ctx, bf, bj);
@@ -1855,6 +1847,7 @@ extern "C" int pes_context_finalize(pes_context* ctx) {
     const int rc = noalloc_base(ctx->device, &base);
     if (rc != PES_OK) return rc;
   }
+  HIP_TRY(hipStreamSynchronize(nullptr));  // k_fpow and k_panel_rec: their tables are read on the callers' streams
   ctx->finalized = true;
   return PES_OK;
 }
@@ -1870,7 +1863,6 @@ extern "C" void pes_context_destroy(pes_context* ctx) {
   free_dev(ctx->d_bin_rec);
   free_dev(ctx->d_tile_f0);
   free_dev(ctx->d_work_counter);
-  free_dev(ctx->d_tile_dd);
   free_dev(ctx->d_tile_jr);
   free_dev(ctx->d_setup);
   free_dev(ctx->d_pconst);
