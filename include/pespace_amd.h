@@ -267,6 +267,11 @@ int pes_profile_work(pes_context* ctx, double* bin_mode_rows, double* bin_rows);
 /* Number of bins of detector det (after finalize). */
 int pes_detector_bins(const pes_context* ctx, int det);
 
+/* Number of 256-bin tiles of detector det whose lnL is evaluated by panels (short polynomials of the
+ * response's smooth part; 0: every bin on its own), -1 for a bad argument.  No counterpart in the
+ * reference. */
+int pes_detector_panel_tiles(const pes_context* ctx, int det);
+
 #ifdef __cplusplus
 }
 #endif

@@ -49,6 +49,7 @@ SIGNATURES = [
     ("pes_profile_read", ctypes.c_int, [ctypes.c_void_p, c_int_p, c_double_p]),
     ("pes_profile_work", ctypes.c_int, [ctypes.c_void_p, c_double_p, c_double_p]),
     ("pes_detector_bins", ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
+    ("pes_detector_panel_tiles", ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     ("pes_links", ctypes.c_int,
      [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
     ("pes_links_from_waveform", ctypes.c_int,

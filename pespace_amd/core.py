@@ -264,6 +264,13 @@ class LikelihoodCore:
         self._build()
         return list(self._n_bins)
 
+    @property
+    def panel_tiles(self):
+        """Per detector, the number of 256-bin tiles whose lnL is evaluated by panels (0: every bin
+        on its own)."""
+        self._build()
+        return [lib().pes_detector_panel_tiles(self._ctx, i) for i in range(len(self._dets))]
+
     def response(self, det, params, precision="fp64"):
         """Complex (P, 3, N) TDI response of detector det."""
         self._build()

@@ -1890,6 +1890,12 @@ extern "C" int pes_detector_bins(const pes_context* ctx, int det) {
   return ctx->hdets[det].d.n_bins;
 }
 
+extern "C" int pes_detector_panel_tiles(const pes_context* ctx, int det) {
+  if (!ctx || !ctx->finalized || det < 0 || det >= (int)ctx->hdets.size()) return -1;
+  if (!ctx->pan.tile_pan) return 0;
+  const auto first = ctx->tile_panels.begin() + ctx->hdets[det].d.bin_offset / TILE;
+  return (int)std::count_if(first, first + ctx->hdets[det].d.n_tiles, [](int n) { return n > 0; });
+}
 
 // (re)allocate scratch for P rows; allocation happens only when P, the gradient flag or the
 // number of tile groups grows
