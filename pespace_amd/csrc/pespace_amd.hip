@@ -1197,11 +1197,11 @@ __global__ __launch_bounds__(TILE) void k_whittle_final(const double* __restrict
       const double *nodes_grad, int NNS, double du, ModeList modes, int P, int rows, const int *tile_jr,     \
       int group_offset, int *work_counter, double *partial,                                                  \
       const unsigned long long *off_bits, const unsigned char *items, const int *tile_pan,                   \
-      BinWork bw, int range, int list_base, const unsigned long long *dbits, int fine
+      BinWork bw, int range, int list_base, const unsigned long long *dbits, int fine, int want
 #define PES_LNL_NAMES                                                                                     \
   dets, n_det, n_tiles, bin_f, bin_j, bin_s, bin_rec, tile_f0, tile_dd, grp, n_grp, pconst,  \
       nodes, nodes_grad, NNS, du, modes, P, rows, tile_jr, group_offset, work_counter, partial, \
-      off_bits, items, tile_pan, bw, range, list_base, dbits, fine
+      off_bits, items, tile_pan, bw, range, list_base, dbits, fine, want
 
 }  // namespace
 
@@ -2048,6 +2048,7 @@ static int prepare(pes_context* ctx, const double* d_params, int P, bool grad, h
 // With panels the bin-by-bin kernel has little beyond the tiles without any (a year of LISA data:
 // 3 of 769 groups), so it is those that have to fill the chip: P = 512, 1.68 ms with 160 rows per
 // item, 0.57 with 8
+static int fine_items_per_slot(const pes_context* ctx, bool grad) { return grad && ctx->modes.n >= 3 ? 5 : 3; }
 static int rows_per_item(const pes_context* ctx, int P, bool grad, int grid, bool panels, bool fine) {
   const int max_rows = grad ? chunk_rows<true>() : chunk_rows<false>();
   if (ctx->rows_override > 0) return std::min(ctx->rows_override, max_rows);
@@ -2061,7 +2062,7 @@ static int rows_per_item(const pes_context* ctx, int P, bool grad, int grid, boo
     // 4 rows 149 -> 81 us (1 row an item), 16 rows 256 -> 121 (2), 64 rows 309 -> 284 (4); without
     // it 16 rows 102 -> 74 (2); one mode 300 rows 143 -> 122 (17)
     const long long slots = (long long)ctx->n_cu * (grad ? 2 : 3), work = (long long)P * groups;
-    const long long want = slots * (grad && ctx->modes.n >= 3 ? 5 : 3);
+    const long long want = slots * fine_items_per_slot(ctx, grad);
     const long long lo = !grad ? std::max(2, 4 / ctx->modes.n) : work > 3 * slots ? 2 : 1;
     return (int)std::max(lo, std::min((long long)max_rows, (work + want - 1) / want));
   }
@@ -2081,6 +2082,10 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   const bool fine = sc.fine && P < fine_rows(ctx) && fine_doubles(ctx, P, grad) <= sc.cap_fine;
   const int rows = rows_per_item(ctx, P, grad, grid, panels, fine);
   const int n_chunks = (P + rows - 1) / rows;
+  // items that the bin-by-bin kernel of a context with panels makes of a small batch that mostly goes its
+  // way (0: the rows are fixed)
+  const int want_items =
+      fine && ctx->rows_override == 0 ? ctx->n_cu * (grad ? 2 : 3) * fine_items_per_slot(ctx, grad) : 0;
   const int nout = grad ? 1 + PES_N_PARAMS : 1;
   // one launch per run of detectors with the same duty flag (two for a duty-cycled run, below):
   // the duty-cycled detectors' tiles run the DUTY instantiation, the others the plain one (whose
@@ -2182,12 +2187,13 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
       // orbit kind only
       const int kd = ranges[r].kind | (pass == 1 ? 2 : 0) | (direct ? 4 : 0);
       const unsigned char* items = ranges[r].duty ? items_buf : nullptr;
+      const int want = ranges[r].duty ? 0 : want_items;  // (a duty-cycled range's flags are per item)
       int* counter = sc.work_counter + (pass == 0 ? r : MAX_TILE_RANGES + r);
 #define PES_LNL_ARGS                                                                                         \
   ctx->d_dets, n_det, ctx->n_tiles, ctx->d_bin_f, ctx->d_bin_j, ctx->d_bin_s, ctx->d_bin_rec,                 \
       ctx->d_tile_f0, ctx->d_tile_dd, grp, n_grp, sc.pconst, sc.nodes, sc.nodes_grad, NNS, ctx->du,           \
       ctx->modes, P, rows, ctx->d_tile_jr, group_offset, counter, part_bin,                                   \
-      sc.off_bits, items, ctx->pan.tile_pan, bin_work, r, group_offset, sc.dbits, fine ? 1 : 0
+      sc.off_bits, items, ctx->pan.tile_pan, bin_work, r, group_offset, sc.dbits, fine ? 1 : 0, want
 #define PES_LNL_GRAD(PR, KD)                                                                                  \
   if (panels && !kDirect<KD>)                                                                                \
     hipLaunchKernelGGL((k_lnl<PR, true, KD, !kDirect<KD>>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS);          \
