@@ -20,6 +20,7 @@ uneven batches of 256, 3001 and 8192 rows from the wide prior, both modes
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
 import sys
@@ -62,6 +63,16 @@ WORKLOADS = {
 
 PEAK_FP64 = 78.6e12  # MI355X FP64 vector, FLOP/s
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_lnl_traffic.json")
+# the sources of the lnL kernels: the counters in TRAFFIC_FILE are those of one state of them
+KERNEL_SOURCES = ("hotpath.hpp", "kernel_common.hpp", "mathfn.hpp", "panel.hpp", "panel_cut.hpp", "response.hpp")
+
+
+def kernel_sources_sha256():
+    h = hashlib.sha256()
+    for name in KERNEL_SOURCES:
+        with open(os.path.join(ROOT, "pespace_amd", "csrc", name), "rb") as fh:
+            h.update(fh.read())
+    return h.hexdigest()
 
 
 def build_network(workload, seed=7, duty=True):
@@ -179,10 +190,12 @@ def traffic_of(workload, precision, grad):
     and their FP64 flops (add, mul = 1, FMA = 2), from the committed rocprofv3 counter summaries
     (FETCH_SIZE / WRITE_SIZE scaled by a plain copy; SQ_ACTIVE_INST_VALU over GRBM_GUI_ACTIVE;
     SQ_INSTS_VALU_{ADD,MUL,FMA}_F64) of a 4096-row step; None each for a workload they do not
-    cover."""
+    cover, and where the kernels' sources are not those that the counters were taken of."""
     try:
         with open(TRAFFIC_FILE) as fh:
             doc = json.load(fh)
+        if doc["kernel_sources_sha256"] != kernel_sources_sha256():
+            return None, None, None
         e = doc["runs"][f"{workload}/{precision}/{'grad' if grad else 'lnl'}"]
         return (e["fetch_kib"] * 1024 * doc["fetch_scale"] + e["write_kib"] * 1024 * doc["write_scale"],
                 e.get("valu_busy"), e.get("flops"))
@@ -454,7 +467,8 @@ def main():
                      "work": {"bin_mode_rows": h["bm"], "bin_rows": h["br"], "flops": flops},
                      "note": "FP64 flops issued by the lnL(+grad) kernels (panel and bin-by-bin launches) over "
                              "their HIP-event time; flops, traffic and valu_busy from the committed rocprofv3 "
-                             "counter summaries (profiles/) of this workload at 4096 particles, hbm_GB_per_s = "
+                             "counter summaries (profiles/) of this workload at 4096 particles (null where the kernels' "
+                             "sources have changed since), hbm_GB_per_s = "
                              "traffic over this run's kernel time; work: (bin, mode, row) and (bin, row) "
                              "triples at or below the cuts"},
     }

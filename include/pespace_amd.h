@@ -120,7 +120,10 @@ int pes_lnl_batch(pes_context* ctx, const double* d_params, int P, double* d_lnl
  * in a fixed array of PES_NOALLOC_SCRATCH_BYTES that every GPU holds once for the whole process;
  * pes_lnl_batch_noalloc_bytes(ctx, P, grad) gives what a batch is accounted for (0 for a bad
  * argument) and a batch accounted for more is rejected with PES_ERR_INVALID before anything is
- * launched; one whose buffers take more than its account runs in parts, with the same results.  Every
+ * launched.  The account is a bound of acceptance, not the memory used: panels take more (flags, more
+ * tile groups), contexts evaluated at every bin less.  A batch whose buffers take more than its account
+ * runs in parts, down to single rows, with the same results (a context of which even one row may not
+ * fit the array holds scratch for one).  Every
  * call on a GPU shares that GPU's array and leaves its contents behind (each call rewrites all it
  * reads): calls that overlap on one GPU race, so serialise them (one stream, or events).  The
  * context's profiling (pes_context_set_profiling) does not apply to this entry point.
@@ -229,20 +232,25 @@ int pes_context_pin_scratch(pes_context* ctx, int pinned);
 int pes_whittle_lnl(const double* d_data, const double* d_resp, const double* d_psd, int n_chan, int n, double df,
                     double* d_work, double* d_out, void* stream);
 
-/* Schedule of the fused kernel: work items of tiles_per_group 256-bin tiles x 48 rows (160 for
- * lnL without gradient), taken from a queue by blocks_per_cu x (number of CUs) persistent
- * blocks of 256 threads.  Defaults
- * 8 and 4; pespace_amd.core.LikelihoodCore.autotune picks them by timing.  Changing the
- * schedule, a larger batch or a first gradient call may reallocate scratch at the next call:
- * reserve and pin the scratch (below) before capturing a HIP graph.
+/* Schedule of the lnL kernels: work items of tiles_per_group 256-bin tiles x a number of rows, taken
+ * from a queue.  Defaults 8 tiles and 4 blocks; pespace_amd.core.LikelihoodCore.autotune picks them by
+ * timing.  What they act on: the bin-by-bin kernel takes items of 48 rows (160 for lnL without
+ * gradient; fewer on small grids and in small batches) in blocks_per_cu x (number of CUs) persistent
+ * blocks of 256 threads.  Long grids go by panels for the most part: a group is then also at most 12
+ * panels, so that more than 12 tiles_per_group is the same as 12, an item is 12 rows, and the panel
+ * kernel's own grid (two blocks per CU) does not depend on blocks_per_cu.  Batches too small to fill
+ * the chip run single tiles or panels whatever tiles_per_group is.  Results differ between schedules
+ * by the order of the partial sums only.  Changing the schedule takes effect at the next batch (a
+ * captured HIP graph keeps the schedule it was captured with) and, like a larger batch or a first
+ * gradient call, may reallocate scratch there: reserve and pin the scratch (above) before capturing.
  * No counterpart in the reference. */
 int pes_context_set_schedule(pes_context* ctx, int tiles_per_group, int blocks_per_cu);
 int pes_context_get_schedule(const pes_context* ctx, int* tiles_per_group, int* blocks_per_cu);
 
-/* Parameter rows per work item of the fused kernel (the rows a block evaluates over one tile
- * group): 0 (the default) picks them per batch (the kernel's chunk, 48 with the gradient and 160
- * without, fewer when the grid has too few tile groups); 1..160 fixes them (capped at the
- * kernel's chunk).  A tunable of the project's autotuner, beside the tile-group size and the
+/* Parameter rows per work item of the bin-by-bin kernel (the rows a block evaluates over one tile
+ * group; the panel kernel's items always hold 12): 0 (the default) picks them per batch (the kernel's
+ * chunk, 48 with the gradient and 160 without, fewer when the grid has too few tile groups or the
+ * batch is small); 1..160 fixes them (capped at the kernel's chunk).  A tunable of the project's autotuner, beside the tile-group size and the
  * blocks per CU; no counterpart in the reference. */
 int pes_context_set_rows_per_item(pes_context* ctx, int rows);
 int pes_context_get_rows_per_item(const pes_context* ctx, int* rows);

@@ -186,7 +186,10 @@ class LikelihoodCore:
     def set_schedule(self, tiles_per_group, blocks_per_cu, rows_per_item=None):
         """Work items of ``tiles_per_group`` 256-bin tiles x ``rows_per_item`` parameter rows
         (0: chosen per batch, 48 with the gradient and 160 without unless the grid or the
-        batch is small; None: unchanged; the panels' items always hold twelve rows), ``blocks_per_cu`` persistent blocks per CU."""
+        batch is small; None: unchanged), ``blocks_per_cu`` persistent blocks per CU.  On data
+        that goes by panels (``panel_tiles``) a group holds at most 12 tiles, the panels' items
+        hold twelve rows and their grid is fixed: rows and blocks act on the rest.  A captured HIP
+        graph keeps the schedule it was captured with."""
         self._build()
         check(lib().pes_context_set_schedule(self._ctx, int(tiles_per_group), int(blocks_per_cu)))
         if rows_per_item is not None:
@@ -214,7 +217,8 @@ class LikelihoodCore:
         The default candidates cover work items of 8-64 tiles and 2-8 persistent blocks per CU
         (the gradient kernel holds two blocks of four waves per CU, the lnL-only kernel three;
         blocks beyond those wait and find the work queue drained), with the rows per item chosen
-        per batch.
+        per batch.  On data that goes by panels, groups of more than 12 tiles are groups of 12:
+        those candidates differ by noise alone.
         """
         self._build()
         p = self._params(params)

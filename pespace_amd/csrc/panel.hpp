@@ -12,10 +12,10 @@
 // the rounding of the bin-by-bin evaluation: the five-point interpolation of a function that
 // turns by theta over half the panel, or is a power f^-p over a relative half-width eps, errs by
 // theta^5 / 1920 or (p)_5 eps^5 / 1920; the host cuts panels at eps <= 1.4e-3 and
-// 4 pi L (f_hi - f_lo) <= 3e-3 (PANEL_EPS, PANEL_SWING), and k_panel_class sends a (tile, row)
-// whose orbit angle turns by more than PANEL_SWING in a panel to the bin-by-bin kernel: ~3e-15 of
+// 4 pi L (f_hi - f_lo) <= 3e-3 (panel_cut.hpp), and k_panel_class sends a (tile, row) whose
+// orbit angle turns by more than PANEL_SWING in a panel to the bin-by-bin kernel: ~3e-15 of
 // the panel's largest |T| (interpolated against evaluated in FP64, three orbits, 1e-3 - 0.05 Hz).
-// lnL and gradient against the bin-by-bin kernel: 1e-16 and 3e-15 (2-norm over a batch).
+// lnL and gradient against the bin-by-bin kernel: 3e-16 and 2e-14 of the largest in a batch of 15 rows.
 //
 // The gradient needs no per-bin adjoint either: with g_c = conj(2 w r_c) P_c u_m, the sums over
 // the panel's bins M_{c,j} = sum g_c x^j (x in [-1, 1] the place in the panel) carry all of it.
@@ -27,7 +27,7 @@
 // ~300 and ~850 for the bin-by-bin kernel; the points' geometry and the moments' reduction add
 // about a fifth.  One-year network of LISA, Taiji and TianQin, six modes: 1024 rows with the
 // gradient 336 -> 111 ms, 2048 without 223 -> 95 ms; one mode on a year of LISA data, 512 rows, 4.2
-// -> 2.0 ms.  VALU busy 0.72 (two waves per SIMD: 256 registers); the rest is waits for LDS and L2.
+// -> 1.9 ms.  VALU busy 0.74 (two waves per SIMD: 256 registers); the rest is waits for LDS and L2.
 //
 // A wave takes one panel and NR rows (two for five or six modes, up to twelve for one) and needs
 // no barrier inside: lanes <-> (row, mode, point) for the geometry, then, two rows at a time,

@@ -1912,11 +1912,11 @@ static size_t partial_doubles(const pes_context* ctx, size_t cap) {
 }
 
 // Batches of fewer rows than this run one tile per work item (k_group_sums): those whose groups of
-// tiles_per_group tiles would give less than about one item to each wave (panels) or block of the
-// chip (16 rows of six modes on short data with the gradient: 64 items on 256 CUs, 1.24 -> 0.25 ms)
+// tiles_per_group tiles would give less than about one item to each wave (panels: twelve rows an item,
+// eight waves per CU) or block (eight rows, four per CU) of the chip (16 rows of six modes on short data with the gradient: 64 items on 256 CUs, 1.24 -> 0.25 ms)
 static int fine_rows(const pes_context* ctx) {
   const int groups = n_groups_of(ctx);
-  return ctx->pan.tile_pan ? 2048 * PANEL_ROWS / groups : 1024 * 8 / groups;
+  return (ctx->pan.tile_pan ? 8 * ctx->n_cu * PANEL_ROWS : 4 * ctx->n_cu * 8) / groups;
 }
 // their per-tile sums, and the duty flags of their work items, for every batch of up to cap rows
 static size_t fine_doubles(const pes_context* ctx, int cap, bool grad) {

@@ -74,11 +74,10 @@ struct ModeList {  // the modes of a context (ids into kModeM etc.), passed to k
 
 struct PanelDev {  // device arrays of a context's panels (panel.hpp)
   const int* tile_pan;     // [n_tiles][2]: first panel and number of panels (0: bin by bin)
-  const int* pan_i;        // [n][4]: node interval, first bin in its tile, bins, -
+  const int* pan_i;        // [n][4]: node interval, first bin in its tile, bins, tile
   const double* pan_d;     // [n][56]
-  const double2* rec;      // [n_tiles][8][256]
+  const double2* rec;      // [n_tiles][256 / 32][8][32] (panel_rec_at)
 };
-
 
 // What a batch leaves to the bin-by-bin kernel in a context with panels, filled by k_panel_class:
 // state[0] the batch's number, state[1 + r] the number of entries of tile range r in list; a tile
