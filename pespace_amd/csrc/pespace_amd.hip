@@ -2291,7 +2291,7 @@ extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, i
   hipStream_t st = (hipStream_t)stream;
   for (int p0 = 0; p0 < P; p0 += part) {
     const int n = std::min(part, P - p0);
-    noalloc_layout(ctx, n, grad, off);
+    const size_t used = noalloc_layout(ctx, n, grad, off);
     BatchScratch sc;
     sc.work_counter = reinterpret_cast<int*>(base + off[0]);
     sc.setup = reinterpret_cast<double*>(base + off[1]);
@@ -2302,8 +2302,10 @@ extern "C" int pes_lnl_batch_noalloc(pes_context* ctx, const double* d_params, i
     sc.off_bits = ctx->any_duty ? reinterpret_cast<unsigned long long*>(base + off[6]) : nullptr;
     sc.items = ctx->any_duty ? reinterpret_cast<unsigned char*>(base + off[7]) : nullptr;
     sc.dbits = ctx->pan.tile_pan ? reinterpret_cast<unsigned long long*>(base + off[8]) : nullptr;
-    sc.fine = nullptr;
-    sc.cap_fine = 0;
+    // a small batch's per-tile sums, where the array has room for them beside the rest
+    const bool room = used < (size_t)PES_NOALLOC_SCRATCH_BYTES;
+    sc.fine = room ? reinterpret_cast<double*>(base + used) : nullptr;
+    sc.cap_fine = room ? ((size_t)PES_NOALLOC_SCRATCH_BYTES - used) / sizeof(double) : 0;
     sc.bin_work = ctx->bin_work_noalloc;
     const double* params = d_params + (size_t)p0 * PES_N_PARAMS;
     rc = launch_setup_nodes(ctx, sc, params, n, grad, ctx->direct_lnl(), st);
