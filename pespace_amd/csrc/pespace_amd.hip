@@ -1911,12 +1911,16 @@ static size_t partial_doubles(const pes_context* ctx, size_t cap) {
   return n;
 }
 
-// Batches of fewer rows than this run one tile per work item (k_group_sums): those whose groups of
-// tiles_per_group tiles would give less than about one item to each wave (panels: twelve rows an item,
-// eight waves per CU) or block (eight rows, four per CU) of the chip (16 rows of six modes on short data with the gradient: 64 items on 256 CUs, 1.24 -> 0.25 ms)
+// Batches of fewer rows than this run one tile (panel) per work item (k_group_sums): without panels those
+// whose groups of tiles_per_group tiles would give less than about one item of eight rows to each block
+// of the chip (four per CU; 16 rows of six modes on short data with the gradient: 64 items on 256 CUs,
+// 1.24 -> 0.25 ms), with panels less than about four of twelve rows to each wave (eight per CU): fewer
+// leave waves idle behind the longest item (LISA and TianQin, 6e6 s, 22 mode, 96 rows: 0.76 -> 0.36 ms
+// and with the gradient 1.30 -> 0.65; all bins one by one 0.60 and 0.98; LISA alone, 5e6 s, 400 rows 0.60
+// -> 0.50; from there on both take the same time, 600 rows 0.73)
 static int fine_rows(const pes_context* ctx) {
   const int groups = n_groups_of(ctx);
-  return (ctx->pan.tile_pan ? 8 * ctx->n_cu * PANEL_ROWS : 4 * ctx->n_cu * 8) / groups;
+  return (ctx->pan.tile_pan ? 4 * 8 * ctx->n_cu * PANEL_ROWS : 4 * ctx->n_cu * 8) / groups;
 }
 // their per-tile sums, and the duty flags of their work items, for every batch of up to cap rows
 static size_t fine_doubles(const pes_context* ctx, int cap, bool grad) {

@@ -27,7 +27,7 @@ def _core(span, modes):
 
 
 @pytest.mark.parametrize("span", [4.0e6, 655360.0])
-@pytest.mark.parametrize("P", [5, 400])
+@pytest.mark.parametrize("P", [5, 1000])
 def test_replays_keep_their_groups(span, P):
     core = _core(span, ((2, 2), (3, 3)))
     center = inj_row(coalescence_time=0.7 * span)
@@ -79,7 +79,7 @@ def test_pinned_scratch_takes_a_schedule_with_fewer_groups(span):
     pinned sums of single tiles have no room for run in items of whole groups."""
     from pespace_amd._lib import PespaceError
     core = _core(span, ((2, 2), (3, 3)))
-    P = 400
+    P = 1000
     rows = particle_cloud(P, seed=60, rel=1e-3, center=inj_row(coalescence_time=0.7 * span))
     core.set_schedule(4, 4)
     core.reserve(P, grad=True)

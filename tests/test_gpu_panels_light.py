@@ -22,7 +22,7 @@ def test_light_systems_in_any_batch(modes):
     core = LikelihoodCore(modes=modes, n_nodes=1024, f_node_min=1e-4, f_node_max=0.05)
     add_to_core(core, d, labels)
     assert core.panel_tiles[0] >= 512
-    rows = particle_cloud(150, seed=95, rel=1e-4, center=inj_row(chirp_mass=30.0, coalescence_time=0.7 * T))
+    rows = particle_cloud(1000, seed=95, rel=1e-4, center=inj_row(chirp_mass=30.0, coalescence_time=0.7 * T))
     rows[40:60] = particle_cloud(20, seed=96, rel=1e-3, center=inj_row(coalescence_time=0.7 * T))
     lnl, g = (x.cpu().numpy() for x in core.lnl(rows, grad=True))
     l0 = core.lnl(rows).cpu().numpy()

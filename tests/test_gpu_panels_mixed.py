@@ -31,7 +31,7 @@ def test_run_of_detectors_without_panels(order):
                           f_node_max=INTERP[1])
     for d, labels in made:
         add_to_core(core, d, labels)
-    rows = particle_cloud(300, seed=33, rel=1e-3, center=inj_row(coalescence_time=0.7 * T))
+    rows = particle_cloud(1000, seed=33, rel=1e-3, center=inj_row(coalescence_time=0.7 * T))
     print(f"bins {core.n_bins}", flush=True)
     lnl, g = (x.cpu().numpy() for x in core.lnl(rows, grad=True))
     net = cb.Network([d for d, _ in made])
