@@ -1243,6 +1243,8 @@ struct GroupTable {
   const int *d_first = nullptr, *d_tile_group = nullptr;
 };
 
+constexpr int PANEL_MIN_BINS_FWD = 75;  // pes_context::panels
+
 struct pes_context {
   int device = 0;
   ModeList modes{};
@@ -1256,6 +1258,15 @@ struct pes_context {
   // evaluated at every bin, and no detector has a duty cycle (the classification of its tiles reads
   // the node tables).  2048 rows, 16384 bins, 22: lnL 1240 -> 780 us, with the gradient 4160 -> 2080
   bool direct_lnl() const { return direct && !any_duty; }
+  // lnL alone of one mode leaves the panel kernel's waves little to overlap, and a panel's points cost more
+  // than they save where it holds few bins: it goes by panels from PANEL_MIN_BINS_FWD bins per panel on
+  // (bins per panel; bin by bin / by panels, ms, 2000 rows near a source and from the prior: 58, 1.59 / 1.72
+  // and 3.64 / 4.01; 67, 1.62 / 1.48 and 3.15 / 3.66; 74, 1.89 / 1.92 and 4.71 / 5.35; 76, 2.13 / 1.79 and 4.21
+  // / 4.55; 97, 2.05 / 1.63 and 3.58 / 3.76; 103, 2.91 / 2.19 and 6.23 / 5.48; with the gradient panels win
+  // throughout).  The rule is the context's alone: a row's lnL is the same in every batch
+  bool panels(bool grad) const {
+    return pan.tile_pan && (grad || modes.n > 1 || pan_bins >= (long long)PANEL_MIN_BINS_FWD * tile_pan0.back());
+  }
   struct HostDet {
     DetectorDev d;
     std::vector<double> f, w, dre, dim;  // w, dre, dim: [3][n]
@@ -1297,6 +1308,7 @@ struct pes_context {
   double2* d_pan_rec = nullptr;
   unsigned long long* d_dbits = nullptr;  // [cap_P][off_words]
   int n_bin_tiles = 0;  // tiles without panels
+  long long pan_bins = 0;  // bins in panels
   std::vector<int> tile_panels;  // panels per tile
   std::vector<int> tile_pan0;    // panels before each tile, and their number
   // tile groups of a context with panels (build_groups), for each tiles_per_group
@@ -1458,7 +1470,8 @@ constexpr int GROUP_PANELS = 12, GROUP_BIN_TILE = 4;
 static const GroupTable& group_table(const pes_context* ctx) {
   return ctx->groups[std::min(ctx->tiles_per_group, GROUP_PANELS) - 1];
 }
-static int tile_ranges(const pes_context* ctx, TileRange* out) {
+// panels: the groups of a batch that goes by panels (at least as many as without)
+static int tile_ranges(const pes_context* ctx, TileRange* out, bool panels) {
   int n = 0;
   for (const auto& h : ctx->hdets) {
     const int t0 = h.d.bin_offset / TILE, t1 = t0 + h.d.n_tiles, duty = h.d.duty ? 1 : 0, kind = h.d.kind;
@@ -1470,7 +1483,7 @@ static int tile_ranges(const pes_context* ctx, TileRange* out) {
   }
   for (int r = 0, g = 0; r < n; ++r) {
     out[r].group_offset = g;
-    if (ctx->groups.empty())
+    if (!panels)
       g += (out[r].tile_end - out[r].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
     else
       while (group_table(ctx).first[g] < out[r].tile_end) ++g;
@@ -1481,7 +1494,7 @@ static int tile_ranges(const pes_context* ctx, TileRange* out) {
 static int build_groups(pes_context* ctx) {
   if (!ctx->pan.tile_pan) return PES_OK;
   TileRange r[MAX_TILE_RANGES];
-  const int n = tile_ranges(ctx, r), nt = ctx->n_tiles;
+  const int n = tile_ranges(ctx, r, false), nt = ctx->n_tiles;
   std::vector<GroupTable> tables(GROUP_PANELS);
   std::vector<int> up, tile_range(nt);
   for (int per = 1; per <= GROUP_PANELS; ++per) {
@@ -1523,9 +1536,10 @@ static int build_groups(pes_context* ctx) {
 // kernel forms the same count from n_tiles)
 static int off_words_of(const pes_context* ctx) { return (ctx->n_tiles + 63) / 64; }
 
+// the most groups of a batch
 static int n_groups_of(const pes_context* ctx) {
   TileRange r[MAX_TILE_RANGES];
-  const int n = tile_ranges(ctx, r);
+  const int n = tile_ranges(ctx, r, ctx->pan.tile_pan != nullptr);
   return r[n - 1].group_offset + r[n - 1].n_groups;
 }
 
@@ -1564,7 +1578,7 @@ constexpr size_t N_SETUP_ACC = SU_IETA;  // the first of the precomputed ones
 static size_t noalloc_account(const pes_context* ctx, int P, bool grad) {
   const size_t NNS = (size_t)ctx->n_nodes + 1, rows = (size_t)P, nm = (size_t)ctx->modes.n;
   TileRange r[MAX_TILE_RANGES];
-  const int n = tile_ranges(ctx, r);
+  const int n = tile_ranges(ctx, r, false);
   size_t groups = 0;
   for (int i = 0; i < n; ++i)
     groups += (r[i].tile_end - r[i].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
@@ -1656,6 +1670,7 @@ static int build_panels(pes_context* ctx, const std::vector<double>& bf, const s
           pt[8] = std::cos(PI * f * h.d.L);
         }
         pi.insert(pi.end(), {j, b0, n, t});
+        ctx->pan_bins += n;
         pd.insert(pd.end(), d, d + PAN_D);
       }
     }
@@ -1918,17 +1933,20 @@ static size_t partial_doubles(const pes_context* ctx, size_t cap) {
 // leave waves idle behind the longest item (LISA and TianQin, 6e6 s, 22 mode, 96 rows: 0.76 -> 0.36 ms
 // and with the gradient 1.30 -> 0.65; all bins one by one 0.60 and 0.98; LISA alone, 5e6 s, 400 rows 0.60
 // -> 0.50; from there on both take the same time, 600 rows 0.73)
-static int fine_rows(const pes_context* ctx) {
-  const int groups = n_groups_of(ctx);
-  return (ctx->pan.tile_pan ? 4 * 8 * ctx->n_cu * PANEL_ROWS : 4 * ctx->n_cu * 8) / groups;
+static int fine_rows(const pes_context* ctx, int groups, bool panels) {
+  return (panels ? 4 * 8 * ctx->n_cu * PANEL_ROWS : 4 * ctx->n_cu * 8) / groups;
 }
-// their per-tile sums, and the duty flags of their work items, for every batch of up to cap rows
-static size_t fine_doubles(const pes_context* ctx, int cap, bool grad) {
-  const size_t rows = (size_t)std::max(0, std::min(cap, fine_rows(ctx) - 1));
-  const size_t slots = (size_t)(TILE / 64) * ctx->n_tiles + (ctx->pan.tile_pan ? ctx->tile_pan0.back() : 0);
-  size_t n = slots * (grad ? 1 + PES_N_PARAMS : 1) * rows;
-  if (ctx->any_duty) n += ((size_t)ctx->n_tiles * rows + 7) / 8;
+// their per-tile sums, and the duty flags of their work items, of one batch ...
+static size_t fine_sums(const pes_context* ctx, int P, bool grad, bool panels) {
+  const size_t slots = (size_t)(TILE / 64) * ctx->n_tiles + (panels ? ctx->tile_pan0.back() : 0);
+  size_t n = slots * (grad ? 1 + PES_N_PARAMS : 1) * P;
+  if (ctx->any_duty) n += ((size_t)ctx->n_tiles * P + 7) / 8;
   return n;
+}
+// ... and of every batch of up to cap rows
+static size_t fine_doubles(const pes_context* ctx, int cap, bool grad) {
+  const bool panels = ctx->pan.tile_pan != nullptr;
+  return fine_sums(ctx, std::max(0, std::min(cap, fine_rows(ctx, n_groups_of(ctx), panels) - 1)), grad, panels);
 }
 
 static int ensure_scratch(pes_context* ctx, int P, bool grad) {
@@ -2053,11 +2071,11 @@ static int prepare(pes_context* ctx, const double* d_params, int P, bool grad, h
 // 3 of 769 groups), so it is those that have to fill the chip: P = 512, 1.68 ms with 160 rows per
 // item, 0.57 with 8
 static int fine_items_per_slot(const pes_context* ctx, bool grad) { return grad && ctx->modes.n >= 3 ? 5 : 3; }
-static int rows_per_item(const pes_context* ctx, int P, bool grad, int grid, bool panels, bool fine) {
+static int rows_per_item(const pes_context* ctx, int P, bool grad, int grid, int n_groups, bool panels, bool fine) {
   const int max_rows = grad ? chunk_rows<true>() : chunk_rows<false>();
   if (ctx->rows_override > 0) return std::min(ctx->rows_override, max_rows);
   const int per = fine ? 1 : std::min(ctx->tiles_per_group, GROUP_PANELS / GROUP_BIN_TILE);
-  const int groups = panels ? ctx->n_bin_tiles / per + 1 : (fine ? ctx->n_tiles : n_groups_of(ctx));
+  const int groups = panels ? ctx->n_bin_tiles / per + 1 : (fine ? ctx->n_tiles : n_groups);
   if (fine) {
     // about three items per resident block (two per CU with the gradient, three without), five where
     // a row is long (gradient of three modes or more): an item's rows follow one another, so a batch
@@ -2079,12 +2097,16 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
                              int precision, hipStream_t st, bool profile) {
   const bool grad = d_grad != nullptr;
   const int NNS = ctx->n_nodes + 1;
-  const int n_groups = n_groups_of(ctx);
   int grid = ctx->n_cu * ctx->blocks_per_cu;
-  const bool panels = sc.dbits != nullptr;
+  const bool panels = ctx->panels(grad);
+  unsigned long long* dbits = panels ? sc.dbits : nullptr;
   const bool direct = ctx->direct_lnl();
-  const bool fine = sc.fine && P < fine_rows(ctx) && fine_doubles(ctx, P, grad) <= sc.cap_fine;
-  const int rows = rows_per_item(ctx, P, grad, grid, panels, fine);
+  TileRange ranges[MAX_TILE_RANGES];
+  const int n_ranges = tile_ranges(ctx, ranges, panels);
+  const int n_groups = ranges[n_ranges - 1].group_offset + ranges[n_ranges - 1].n_groups;
+  const bool fine =
+      sc.fine && P < fine_rows(ctx, n_groups, panels) && fine_sums(ctx, P, grad, panels) <= sc.cap_fine;
+  const int rows = rows_per_item(ctx, P, grad, grid, n_groups, panels, fine);
   const int n_chunks = (P + rows - 1) / rows;
   // items that the bin-by-bin kernel of a context with panels makes of a small batch that mostly goes its
   // way (0: the rows are fixed)
@@ -2094,8 +2116,6 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   // one launch per run of detectors with the same duty flag (two for a duty-cycled run, below):
   // the duty-cycled detectors' tiles run the DUTY instantiation, the others the plain one (whose
   // register allocation is that of a kernel without the window code)
-  TileRange ranges[MAX_TILE_RANGES];
-  const int n_ranges = tile_ranges(ctx, ranges);
   double *part_pan = sc.partial, *part_bin = sc.partial;
   unsigned char* items_buf = sc.items;
   if (fine) {
@@ -2131,7 +2151,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     hipLaunchKernelGGL(k_panel_class, dim3(off_words, std::min(P, 65535)), dim3(64), 0, st, ctx->d_dets, n_det,
                        ctx->n_tiles, ctx->d_tile_f0, ctx->d_bin_f, sc.pconst, sc.nodes, NNS, ctx->du, ctx->modes, P,
                        off_words, ctx->any_duty ? sc.off_bits : nullptr, ctx->pan, bin_work, groups, fine ? 1 : 0,
-                       sc.dbits);
+                       dbits);
     HIP_TRY(hipGetLastError());
   }
   // a duty-cycled range's work items on the window's plateau (for every row and mode of the item)
@@ -2142,7 +2162,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     hipLaunchKernelGGL(k_duty_items, dim3(n_work), dim3(64), 0, st, ctx->d_dets, n_det, ctx->d_tile_f0,
                        ctx->d_tile_jr, sc.pconst, sc.nodes, NNS, ctx->u0, ctx->du, ctx->modes, P, rows, n_chunks,
                        range_groups(r), fine ? ranges[r].tile_begin : ranges[r].group_offset, ctx->direct ? 0 : 1,
-                       items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, sc.dbits);
+                       items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, dbits);
     HIP_TRY(hipGetLastError());
   }
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -2171,7 +2191,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
 #define PES_PANEL_ARGS                                                                                        \
   ctx->d_dets, n_det, ctx->n_tiles, ctx->d_tile_f0, ctx->d_tile_dd, grp.first, n_pg, sc.pconst, sc.nodes,            \
       sc.nodes_grad, NNS, ctx->du, ctx->modes, P, fine ? pan_begin : group_offset, counter,                   \
-      part_pan, off, sc.dbits, ctx->pan, pan_begin
+      part_pan, off, dbits, ctx->pan, pan_begin
 #define PES_PANEL(G, KD) \
   hipLaunchKernelGGL((k_lnl_panel<G, KD>), dim3(grid_p), dim3(TILE), 0, st, PES_PANEL_ARGS)
       if (grad) {
@@ -2197,7 +2217,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   ctx->d_dets, n_det, ctx->n_tiles, ctx->d_bin_f, ctx->d_bin_j, ctx->d_bin_s, ctx->d_bin_rec,                 \
       ctx->d_tile_f0, ctx->d_tile_dd, grp, n_grp, sc.pconst, sc.nodes, sc.nodes_grad, NNS, ctx->du,           \
       ctx->modes, P, rows, ctx->d_tile_jr, group_offset, counter, part_bin,                                   \
-      sc.off_bits, items, ctx->pan.tile_pan, bin_work, r, group_offset, sc.dbits, fine ? 1 : 0, want
+      sc.off_bits, items, ctx->pan.tile_pan, bin_work, r, group_offset, dbits, fine ? 1 : 0, want
 #define PES_LNL_GRAD(PR, KD)                                                                                  \
   if (panels && !kDirect<KD>)                                                                                \
     hipLaunchKernelGGL((k_lnl<PR, true, KD, !kDirect<KD>>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS);          \

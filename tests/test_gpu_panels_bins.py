@@ -59,3 +59,21 @@ def test_panels_match_bins(case):
           f"gradient {err_g.max():.1e}", flush=True)
     assert err_l.max() < 1e-13
     assert err_g.max() < 1e-11
+
+
+@pytest.mark.parametrize("modes", [("22",), ("22", "33")])
+@pytest.mark.parametrize("duty", [None, (1.0e6, 6.0e5, 2.0e5, 3.0e4)])
+def test_lnl_alone_of_short_panels(modes, duty):
+    """Where panels hold few bins lnL alone of one mode goes bin by bin and the gradient by panels (LISA
+    over 3.1e6 s; TianQin's panels are longer): the same lnL up to rounding, and each the same in every
+    batch, to the last bit."""
+    d, labels = make_detector(T=4.0e6 if duty else 3.1e6, dt=5.0, modes=tuple((int(m[0]), int(m[1])) for m in modes), interp=INTERP, seed=93,
+                              **(dict(TIANQIN, duty=duty) if duty else {}))
+    core = _core(d, labels, modes, 0, d.f.size)
+    assert core.panel_tiles[0] >= 512
+    rows = np.vstack([particle_cloud(900, seed=94, rel=1e-3, center=inj_row(coalescence_time=0.7 * T)),
+                      prior_rows(200, seed=95, tc_range=(0.0, T))])[np.random.default_rng(1).permutation(1100)]
+    lnl = core.lnl(rows).cpu().numpy()
+    np.testing.assert_allclose(core.lnl(rows, grad=True)[0].cpu().numpy(), lnl, rtol=1e-13)
+    for a, b in ((0, 1), (3, 8), (0, 90), (100, 330), (0, 700)):
+        np.testing.assert_array_equal(core.lnl(rows[a:b]).cpu().numpy(), lnl[a:b])
