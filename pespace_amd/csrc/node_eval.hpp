@@ -285,11 +285,10 @@ PES_HD void node_adjoint(const double* su, int mode, const FreqPow& fq, double w
       const double c2 = k(SU_C2INT) * y;
       G = (b1 + b3 + k(SU_B2)) * e + c2;
       DG = (b1 - 3.0 * b3) * e + c2;
-      const double ly = log(y);
-      aE += ap * (b1 - (1.0 / 3.0) * b3 + k(SU_B2) * ly) + ag * (b1 + b3 + k(SU_B2));
+      aE += ap * (b1 - (1.0 / 3.0) * b3 + k(SU_B2) * l) + ag * (b1 + b3 + k(SU_B2));
       add(SU_B1, e * y * as);
       add(SU_B3, e * iy3 * (ag - (1.0 / 3.0) * ap));
-      add(SU_B2, e * (ap * ly + ag));
+      add(SU_B2, e * (ap * l + ag));
       add(SU_C1INT, ap);
       add(SU_C2INT, y * as);
     }
