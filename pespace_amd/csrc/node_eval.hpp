@@ -30,15 +30,15 @@ struct NodeY {
   double x, y, r;          // M f, f22, d ln y / d ln x
   double c, ic, l, y76;    // y^(1/3), y^(-1/3), ln y, y^(-7/6)
 };
-// y^(1/3), y^(-1/3) and y^(-7/6) of y + yl from i = y^(-1/3) and p = y^(-7/6) to a few roundings: the
-// residual 1 - (y + yl) i^3, formed with the products' rounding errors, corrects all of them
-PES_HD void y_powers(double y, double yl, double i, double p, NodeY& o) {
+// y^(1/3), y^(-1/3) and y^(-7/6) of y from i = y^(-1/3) and p = y^(-7/6) to a few roundings: the residual
+// t = 1 - y i^3, formed with the products' rounding errors, corrects all of them
+PES_HD void y_powers(double y, double i, double p, NodeY& o) {
   const double i2 = i * i, e2 = fma(i, i, -i2);
   const double i3 = i2 * i, e3 = fma(e2, i, fma(i2, i, -i3));
-  const double t = fma(-y, i3, 1.0) - fma(y, e3, yl * i3);
+  const double t = fma(-y, e3, fma(-y, i3, 1.0)), t3 = t * (1.0 / 3.0);
   const double h = y * i2;
-  o.ic = fma(i, t * (1.0 / 3.0), i);
-  o.c = h + (fma(y, i2, -h) + fma(y, e2, fma(yl, i2, h * (t * (2.0 / 3.0)))));
+  o.ic = fma(i, t3, i);
+  o.c = h + (fma(y, i2, -h) + fma(y, e2, (2.0 * h) * t3));
   const double s = p * y;  // y^(-1/6), corrected by its square
   o.y76 = fma(i3, t, i3) * fma(0.5 * s * o.c, fma(-s, s, o.ic), s);
 }
@@ -64,19 +64,17 @@ PES_HD NodeY node_y(const double* su, int mode, const FreqPow& q) {
   o.r = 1.0;
   const double m = (double)kModeM[mode], fi = 0.5 * m * HM_MAP_JOIN;
   if (mode == 0 || o.x < fi) {
-    double yl = fma(q.f, su[SU_MSEC], -o.x), i = q.ic * su[SU_IM13], p = q.f76 * su[SU_M76];
+    double i = q.ic * su[SU_IM13], p = q.f76 * su[SU_M76];
     o.y = o.x;
     o.l = q.l + su[SU_LNM];
     if (kModeM[mode] != 2) {
       const ModePow k = mode_pow(kModeM[mode]);
-      const double h = 2.0 / m;
-      o.y = o.x * h;
-      yl = fma(yl, h, fma(o.x, h, -o.y));
+      o.y *= 2.0 / m;
       i *= k.ic;
       p *= k.p76;
       o.l += k.l;
     }
-    y_powers(o.y, yl, i, p, o);
+    y_powers(o.y, i, p, o);
     return o;
   }
   const double fr = su[su_frd(mode)], FRD = su[SU_FRD], rho = FRD / fr;
