@@ -1056,18 +1056,14 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
   // rows (1 <= rows <= CH) per work item, chosen by the host.  This launch covers the n_grp groups
   // of a tile range, whose partial sums go to groups group_offset + 0, 1, ...: one launch (and
   // counter) per tile range of one orbit kind and duty flag, two for a duty-cycled range
-  // with panels only the groups of the batch's list have work left here.  The host chose the rows for
-  // the tiles without panels; a small batch of which more goes bin by bin (light systems, whose orbit
-  // turns too fast for panels) takes as many rows per item as leave `want` items (a year of LISA
-  // data, 8 rows of 30 solar masses with the gradient: 0.95 -> 0.68 ms; all tiles bin by bin 0.86)
+  // with panels only the groups of the batch's list have work left here
   const int n_list = PAN ? bw.state[1 + range] : n_grp;
-  if constexpr (PAN)
-    if (want > 0) rows = max(rows, min(CH, (int)((long long)P * n_list / want)));
+  if constexpr (PAN) rows = listed_rows(rows, P, n_list, want, CH);
   const int n_chunks = (P + rows - 1) / rows;
   const int n_work = n_chunks * n_list;
   const int epoch = PAN ? bw.state[0] : 0;
   constexpr bool DUTY = kDuty<KD>;
-  // the duty pass of a range whose items all run in the plain one: k_duty_items counted none at
+  // the duty pass of a range whose items all run in the plain one: k_duty_items set no flag at
   // work_counter[MAX_TILE_RANGES] (every block leaves before its first barrier)
   if (DUTY && items && work_counter[MAX_TILE_RANGES] == 0) return;
   // work items are taken from a counter (zeroed by k_setup earlier on the same stream), so

@@ -561,10 +561,15 @@ __global__ __launch_bounds__(64) void k_duty_items(const DetectorDev* __restrict
                                                    const double* __restrict__ tile_f0, const int* __restrict__ tile_jr,
                                                    const double* __restrict__ pconst, const double* __restrict__ nodes,
                                                    int NNS, double u0, double du, ModeList modes, int P, int rows,
-                                                   int n_chunks, RangeGroups grp, int group_offset, int enable, unsigned char* __restrict__ items,
-                                                   int* __restrict__ n_duty_items, int words,
-                                                   const unsigned long long* __restrict__ dbits) {
+                                                   RangeGroups grp, int n_grp, int group_offset, int enable,
+                                                   unsigned char* __restrict__ items,
+                                                   int* __restrict__ any_duty_item, int words,
+                                                   const unsigned long long* __restrict__ dbits,
+                                                   const int* __restrict__ n_list, int want, int most) {
+  if (dbits) rows = listed_rows(rows, P, *n_list, want, most);  // as the fused kernel
+  const int n_chunks = (P + rows - 1) / rows;
   const int gl = blockIdx.x / n_chunks, c = blockIdx.x % n_chunks;
+  if (gl >= n_grp) return;
   const int t_first = grp.begin(gl), t_end = grp.end(gl);
   const int p0 = c * rows, p1 = min(P, p0 + rows);
   const int nt = t_end - t_first, np = p1 - p0;
@@ -588,7 +593,10 @@ __global__ __launch_bounds__(64) void k_duty_items(const DetectorDev* __restrict
   ok = __syncthreads_and(ok);
   if (threadIdx.x == 0) {
     items[(size_t)(group_offset + gl) * n_chunks + c] = ok ? 1 : 0;
-    if (!ok) atomicAdd(n_duty_items, 1);  // the range's duty pass ends at once when none need it
+    // the range's duty pass ends at once when none need it (a flag: counting the thousands of items of a
+    // small batch one by one took most of this kernel's 23 us)
+    if (!ok && __hip_atomic_load(any_duty_item, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+      __hip_atomic_store(any_duty_item, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -1236,10 +1244,10 @@ hipError_t pes::launch_lnl_fwd(int precision, int kd, int grid, hipStream_t st, 
 }
 #else
 // ================================= host side ================================================
-// The first tile of each tile group, and n_tiles, under one tiles_per_group; on the device those and
-// the group of each tile
+// The tile groups under one tiles_per_group: the first group of each tile range, and their number; on the
+// device the first tile of each group, and n_tiles, and the group of each tile
 struct GroupTable {
-  std::vector<int> first;
+  int group0[MAX_TILE_RANGES + 1];
   const int *d_first = nullptr, *d_tile_group = nullptr;
 };
 
@@ -1483,10 +1491,10 @@ static int tile_ranges(const pes_context* ctx, TileRange* out, bool panels) {
   }
   for (int r = 0, g = 0; r < n; ++r) {
     out[r].group_offset = g;
-    if (!panels)
-      g += (out[r].tile_end - out[r].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
+    if (panels)
+      g = group_table(ctx).group0[r + 1];
     else
-      while (group_table(ctx).first[g] < out[r].tile_end) ++g;
+      g += (out[r].tile_end - out[r].tile_begin + ctx->tiles_per_group - 1) / ctx->tiles_per_group;
     out[r].n_groups = g - out[r].group_offset;
   }
   return n;
@@ -1498,9 +1506,10 @@ static int build_groups(pes_context* ctx) {
   std::vector<GroupTable> tables(GROUP_PANELS);
   std::vector<int> up, tile_range(nt);
   for (int per = 1; per <= GROUP_PANELS; ++per) {
-    std::vector<int>& first = tables[per - 1].first;
+    std::vector<int> first;
     const size_t at = up.size();
     up.resize(at + nt);  // the group of each tile, then the groups' first tiles
+    tables[per - 1].group0[0] = 0;
     for (int i = 0; i < n; ++i) {
       int tiles = 0, cost = 0;
       for (int t = r[i].tile_begin; t < r[i].tile_end; ++t) {
@@ -1514,6 +1523,7 @@ static int build_groups(pes_context* ctx) {
         up[at + t] = (int)first.size() - 1;
         tile_range[t] = i;
       }
+      tables[per - 1].group0[i + 1] = (int)first.size();
     }
     first.push_back(nt);
     up.insert(up.end(), first.begin(), first.end());
@@ -1524,7 +1534,7 @@ static int build_groups(pes_context* ctx) {
   for (auto& t : tables) {
     t.d_tile_group = d;
     t.d_first = d + nt;
-    d = t.d_first + t.first.size();
+    d = t.d_first + t.group0[n] + 1;
   }
   ctx->groups = std::move(tables);
   int* to = ctx->d_bin_work + (ctx->bin_work.tile_range - ctx->d_bin_work);
@@ -2160,9 +2170,11 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
     if (!ranges[r].duty) continue;
     const int n_grp = fine ? ranges[r].tile_end - ranges[r].tile_begin : ranges[r].n_groups, n_work = n_grp * n_chunks;
     hipLaunchKernelGGL(k_duty_items, dim3(n_work), dim3(64), 0, st, ctx->d_dets, n_det, ctx->d_tile_f0,
-                       ctx->d_tile_jr, sc.pconst, sc.nodes, NNS, ctx->u0, ctx->du, ctx->modes, P, rows, n_chunks,
-                       range_groups(r), fine ? ranges[r].tile_begin : ranges[r].group_offset, ctx->direct ? 0 : 1,
-                       items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, dbits);
+                       ctx->d_tile_jr, sc.pconst, sc.nodes, NNS, ctx->u0, ctx->du, ctx->modes, P, rows,
+                       range_groups(r), n_grp, fine ? ranges[r].tile_begin : ranges[r].group_offset,
+                       ctx->direct ? 0 : 1, items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, dbits,
+                       panels ? bin_work.state + 1 + r : nullptr, want_items,
+                       grad ? chunk_rows<true>() : chunk_rows<false>());
     HIP_TRY(hipGetLastError());
   }
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -2211,13 +2223,12 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
       // orbit kind only
       const int kd = ranges[r].kind | (pass == 1 ? 2 : 0) | (direct ? 4 : 0);
       const unsigned char* items = ranges[r].duty ? items_buf : nullptr;
-      const int want = ranges[r].duty ? 0 : want_items;  // (a duty-cycled range's flags are per item)
       int* counter = sc.work_counter + (pass == 0 ? r : MAX_TILE_RANGES + r);
 #define PES_LNL_ARGS                                                                                         \
   ctx->d_dets, n_det, ctx->n_tiles, ctx->d_bin_f, ctx->d_bin_j, ctx->d_bin_s, ctx->d_bin_rec,                 \
       ctx->d_tile_f0, ctx->d_tile_dd, grp, n_grp, sc.pconst, sc.nodes, sc.nodes_grad, NNS, ctx->du,           \
       ctx->modes, P, rows, ctx->d_tile_jr, group_offset, counter, part_bin,                                   \
-      sc.off_bits, items, ctx->pan.tile_pan, bin_work, r, group_offset, dbits, fine ? 1 : 0, want
+      sc.off_bits, items, ctx->pan.tile_pan, bin_work, r, group_offset, dbits, fine ? 1 : 0, want_items
 #define PES_LNL_GRAD(PR, KD)                                                                                  \
   if (panels && !kDirect<KD>)                                                                                \
     hipLaunchKernelGGL((k_lnl<PR, true, KD, !kDirect<KD>>), dim3(grid_r), dim3(TILE), 0, st, PES_LNL_ARGS);          \
