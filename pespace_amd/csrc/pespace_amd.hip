@@ -555,8 +555,11 @@ __global__ __launch_bounds__(64) void k_duty_off(const DetectorDev* __restrict__
 // evaluates nothing there (the tile above its cuts, an invalid row).  Such items run in the plain
 // instantiation of the fused kernel, whose response and gradient equal the duty one's there; the
 // others in the duty instantiation.  The item index is that of the fused kernel (global group
-// g = group_offset + gl, chunk c: g n_chunks + c).  One block of 64 per item; enable = 0 (no node
-// intervals: direct evaluation at every bin) sends every item to the duty instantiation.
+// g = group_offset + gl, chunk c: g n_chunks + c).  One wave per item of more than 32 (tile, row)s;
+// of smaller ones (small batches, one tile and as little as one row each) a wave takes as many of
+// its group as it has lanes for: TianQin, 3e7 s, 120 rows of one row an item, 186 -> 10 us against a
+// wave for each.  n_blk blocks per group; enable = 0 (no node intervals: direct evaluation at every
+// bin) sends every item to the duty instantiation.
 __global__ __launch_bounds__(64) void k_duty_items(const DetectorDev* __restrict__ dets, int n_det,
                                                    const double* __restrict__ tile_f0, const int* __restrict__ tile_jr,
                                                    const double* __restrict__ pconst, const double* __restrict__ nodes,
@@ -565,37 +568,40 @@ __global__ __launch_bounds__(64) void k_duty_items(const DetectorDev* __restrict
                                                    unsigned char* __restrict__ items,
                                                    int* __restrict__ any_duty_item, int words,
                                                    const unsigned long long* __restrict__ dbits,
-                                                   const int* __restrict__ n_list, int want, int most) {
+                                                   const int* __restrict__ n_list, int want, int most, int n_blk) {
   if (dbits) rows = listed_rows(rows, P, *n_list, want, most);  // as the fused kernel
   const int n_chunks = (P + rows - 1) / rows;
-  const int gl = blockIdx.x / n_chunks, c = blockIdx.x % n_chunks;
+  const int gl = blockIdx.x / n_blk, lane = threadIdx.x;
   if (gl >= n_grp) return;
-  const int t_first = grp.begin(gl), t_end = grp.end(gl);
-  const int p0 = c * rows, p1 = min(P, p0 + rows);
-  const int nt = t_end - t_first, np = p1 - p0;
-  int ok = enable;
-  for (int k = threadIdx.x; ok && k < nt * np; k += blockDim.x) {
-    const int tile = t_first + k % nt, p = p0 + k / nt;
-    const double* pc = pconst + (size_t)p * PC_STRIDE;
-    const double f0 = tile_f0[tile];
-    if (pc[PC_VALID] == 0.0 || f0 > pc[PC_FCUT]) continue;
-    if (dbits && ((dbits[(size_t)p * words + (tile >> 6)] >> (tile & 63)) & 1ull) == 0) continue;  // in panels
-    const DetectorDev& det = dets[tile_detector(dets, n_det, tile)];
-    const int j0 = tile_jr[2 * tile], j1 = j0 + tile_jr[2 * tile + 1];
-    const double tc = pc[PC_TC];
-    for (int mi = 0; mi < modes.n && ok; ++mi) {
-      if (f0 > pc[PC_MODE + mi * PC_MODE_STRIDE + MF_CUT]) continue;
-      const double* nm = nodes + ((size_t)p * modes.n + mi) * NNS * 4;
-      for (int j = j0; j < j1 && ok; ++j)
-        ok = det.duty && interval_on(det, nm + (size_t)j * 4, exp(u0 + du * j), exp(u0 + du * (j + 1)), du, tc);
+  const int t_first = grp.begin(gl), nt = grp.end(gl) - t_first;
+  const int per = nt * rows, span = per <= 32 ? 64 / per : 1;  // items of a wave
+  const int sub = span > 1 ? lane / per : 0;
+  for (int c0 = (blockIdx.x % n_blk) * span; c0 < n_chunks; c0 += n_blk * span) {
+    const int c = c0 + sub, p0 = c * rows, np = min(P - p0, rows);
+    const bool mine = sub < span && c < n_chunks;
+    int ok = enable;
+    for (int k = span > 1 ? lane - sub * per : lane; mine && ok && k < nt * np; k += 64) {
+      const int tile = t_first + k % nt, p = p0 + k / nt;
+      const double* pc = pconst + (size_t)p * PC_STRIDE;
+      const double f0 = tile_f0[tile];
+      if (pc[PC_VALID] == 0.0 || f0 > pc[PC_FCUT]) continue;
+      if (dbits && ((dbits[(size_t)p * words + (tile >> 6)] >> (tile & 63)) & 1ull) == 0) continue;  // in panels
+      const DetectorDev& det = dets[tile_detector(dets, n_det, tile)];
+      const int j0 = tile_jr[2 * tile], j1 = j0 + tile_jr[2 * tile + 1];
+      const double tc = pc[PC_TC];
+      for (int mi = 0; mi < modes.n && ok; ++mi) {
+        if (f0 > pc[PC_MODE + mi * PC_MODE_STRIDE + MF_CUT]) continue;
+        const double* nm = nodes + ((size_t)p * modes.n + mi) * NNS * 4;
+        for (int j = j0; j < j1 && ok; ++j)
+          ok = det.duty && interval_on(det, nm + (size_t)j * 4, exp(u0 + du * j), exp(u0 + du * (j + 1)), du, tc);
+      }
     }
-  }
-  ok = __syncthreads_and(ok);
-  if (threadIdx.x == 0) {
-    items[(size_t)(group_offset + gl) * n_chunks + c] = ok ? 1 : 0;
+    const unsigned long long bad = __ballot(mine && !ok);
+    const unsigned long long item = span > 1 ? ((1ull << per) - 1) << (sub * per) : ~0ull;
+    if (mine && lane == sub * per) items[(size_t)(group_offset + gl) * n_chunks + c] = (bad & item) ? 0 : 1;
     // the range's duty pass ends at once when none need it (a flag: counting the thousands of items of a
     // small batch one by one took most of this kernel's 23 us)
-    if (!ok && __hip_atomic_load(any_duty_item, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    if (lane == 0 && bad != 0 && __hip_atomic_load(any_duty_item, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
       __hip_atomic_store(any_duty_item, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
@@ -1268,9 +1274,9 @@ struct pes_context {
   bool direct_lnl() const { return direct && !any_duty; }
   // lnL alone of one mode leaves the panel kernel's waves little to overlap, and a panel's points cost more
   // than they save where it holds few bins: it goes by panels from PANEL_MIN_BINS_FWD bins per panel on
-  // (bins per panel; bin by bin / by panels, ms, 2000 rows near a source and from the prior: 58, 1.59 / 1.72
-  // and 3.64 / 4.01; 67, 1.62 / 1.48 and 3.15 / 3.66; 74, 1.89 / 1.92 and 4.71 / 5.35; 76, 2.13 / 1.79 and 4.21
-  // / 4.55; 97, 2.05 / 1.63 and 3.58 / 3.76; 103, 2.91 / 2.19 and 6.23 / 5.48; with the gradient panels win
+  // (bins per panel; bin by bin / by panels, ms, 2000 rows near a source and from the prior: 58, 1.63 / 1.84
+  // and 3.62 / 3.71; 67, 1.69 / 1.60 and 3.29 / 3.37; 74, 2.03 / 2.06 and 4.75 / 4.83; 76, 2.20 / 1.98 and 4.22
+  // / 4.12; 97, 2.12 / 1.79 and 3.76 / 3.25; 103, 2.98 / 2.37 and 6.18 / 4.81; with the gradient panels win
   // throughout).  The rule is the context's alone: a row's lnL is the same in every batch
   bool panels(bool grad) const {
     return pan.tile_pan && (grad || modes.n > 1 || pan_bins >= (long long)PANEL_MIN_BINS_FWD * tile_pan0.back());
@@ -2168,13 +2174,14 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
   // run in the plain instantiation, the others in the duty one: two launches of the range
   for (int r = 0; r < n_ranges; ++r) {
     if (!ranges[r].duty) continue;
-    const int n_grp = fine ? ranges[r].tile_end - ranges[r].tile_begin : ranges[r].n_groups, n_work = n_grp * n_chunks;
-    hipLaunchKernelGGL(k_duty_items, dim3(n_work), dim3(64), 0, st, ctx->d_dets, n_det, ctx->d_tile_f0,
+    const int n_grp = fine ? ranges[r].tile_end - ranges[r].tile_begin : ranges[r].n_groups;
+    const int n_blk = fine ? std::min(n_chunks, (P + 31) / 32) : n_chunks;
+    hipLaunchKernelGGL(k_duty_items, dim3(n_grp * n_blk), dim3(64), 0, st, ctx->d_dets, n_det, ctx->d_tile_f0,
                        ctx->d_tile_jr, sc.pconst, sc.nodes, NNS, ctx->u0, ctx->du, ctx->modes, P, rows,
                        range_groups(r), n_grp, fine ? ranges[r].tile_begin : ranges[r].group_offset,
                        ctx->direct ? 0 : 1, items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, dbits,
                        panels ? bin_work.state + 1 + r : nullptr, want_items,
-                       grad ? chunk_rows<true>() : chunk_rows<false>());
+                       grad ? chunk_rows<true>() : chunk_rows<false>(), n_blk);
     HIP_TRY(hipGetLastError());
   }
   hipEvent_t e0 = nullptr, e1 = nullptr;
