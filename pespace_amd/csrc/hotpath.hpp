@@ -784,9 +784,11 @@ __device__ inline void stage_nodes_dma(const double* __restrict__ nodes, const d
 // finished the previous row, the last reader of the buffer the copy for the next row goes to.
 // Without STAGED each lane reads its node rows from global memory (tiles whose node range is
 // wider, e.g. the lowest frequencies of short data).
-// Which lanes' rows p < p1 of a tile with panels come bin by bin (k_panel_class)
+// Which lanes' rows p < p1 of a tile with panels come bin by bin (k_panel_class).  (A template, so that
+// host builds, which call no kernel, need no __ballot)
+template <typename Row>
 __device__ inline unsigned long long rows_listed(const unsigned long long* __restrict__ dbits, int n_tiles, int tile,
-                                                 int p, int p1) {
+                                                 Row p, int p1) {
   return __ballot(p < p1 && ((dbits[(size_t)p * ((n_tiles + 63) >> 6) + (tile >> 6)] >> (tile & 63)) & 1ull) != 0);
 }
 
@@ -1106,8 +1108,9 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
       const unsigned long long* db = nullptr;
       if constexpr (PAN) {
         // a tile with panels: the panel kernel has it, apart from the rows marked in dbits
-        db = tile_pan[2 * tile + 1] > 0 ? dbits : nullptr;
-        if (db && (bw.tile_any[tile] != epoch || tile_f0[tile] > chunk_cut)) continue;
+        const bool listed = dbits && tile_pan[2 * tile + 1] > 0;
+        if (listed && (bw.tile_any[tile] != epoch || tile_f0[tile] > chunk_cut)) continue;
+        db = listed && P > 1 ? dbits : nullptr;  // (the only row of a batch is the one marked)
         // ... none of this chunk's rows: its bins need not be prepared (TianQin, 6e6 s, duty-cycled, 600 rows
         // from the prior, lnL alone: this launch 786 -> 190 us, with the rows' flags read by votes)
         if (db) {
