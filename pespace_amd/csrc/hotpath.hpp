@@ -1072,7 +1072,7 @@ __global__ __launch_bounds__(TILE, GRAD ? 2 : 3) void k_lnl(const DetectorDev* _
   // counter) per tile range of one orbit kind and duty flag, two for a duty-cycled range
   // with panels only the groups of the batch's list have work left here
   const int n_list = PAN ? bw.state[1 + range] : n_grp;
-  if constexpr (PAN) rows = listed_rows(rows, P, n_list, want, CH);
+  if constexpr (PAN) rows = listed_rows(rows, P, n_list, want, modes.n);
   const int n_chunks = (P + rows - 1) / rows;
   const int n_work = n_chunks * n_list;
   const int epoch = PAN ? bw.state[0] : 0;

@@ -59,12 +59,15 @@ struct TileGroups {
 };
 
 // Rows per work item of the bin-by-bin kernel where panels leave it a list of n_list groups: the host's
-// `rows`, chosen for the tiles without panels, and more (at most `most`) where a small batch sends more
-// its way (light systems, whose orbit turns too fast for panels), so that about `want` items remain (0: the
-// host's).  A year of LISA data, 8 rows of 30 solar masses with the gradient: 0.95 -> 0.68 ms; all
-// tiles bin by bin 0.86
-__device__ inline int listed_rows(int rows, int P, int n_list, int want, int most) {
-  return want > 0 ? max(rows, min(most, (int)((long long)P * n_list / want))) : rows;
+// `rows`, chosen for the tiles without panels, and more where a small batch sends more its way (light
+// systems, whose orbit turns too fast for panels), so that about `want` items remain (0: the host's).  A year
+// of LISA data, 8 rows of 30 solar masses with the gradient: 0.95 -> 0.68 ms; all tiles bin by bin 0.86.
+// At most 24, 48 with one or two modes: the last items end together, and an item's rows share the tile's
+// preparation (lnL, ms, with 160, 48 and 24: LISA, 5e6 s, six modes, 300 rows from the prior 2.99, 2.63, 2.32;
+// TianQin, 6e6 s, duty-cycled, 22 mode, 400 rows 0.97, 0.86, 1.03; with the gradient 24 for 48 rows: 6.26 ->
+// 5.75 and 1.52 -> 1.64)
+__device__ inline int listed_rows(int rows, int P, int n_list, int want, int n_modes) {
+  return want > 0 ? max(rows, min(n_modes < 3 ? 48 : 24, (int)((long long)P * n_list / want))) : rows;
 }
 
 // detector owning tile `tile` (detectors are concatenated in tile order)

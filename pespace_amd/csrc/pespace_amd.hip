@@ -568,8 +568,8 @@ __global__ __launch_bounds__(64) void k_duty_items(const DetectorDev* __restrict
                                                    unsigned char* __restrict__ items,
                                                    int* __restrict__ any_duty_item, int words,
                                                    const unsigned long long* __restrict__ dbits,
-                                                   const int* __restrict__ n_list, int want, int most, int n_blk) {
-  if (dbits) rows = listed_rows(rows, P, *n_list, want, most);  // as the fused kernel
+                                                   const int* __restrict__ n_list, int want, int n_blk) {
+  if (dbits) rows = listed_rows(rows, P, *n_list, want, modes.n);  // as the fused kernel
   const int n_chunks = (P + rows - 1) / rows;
   const int gl = blockIdx.x / n_blk, lane = threadIdx.x;
   if (gl >= n_grp) return;
@@ -2180,8 +2180,7 @@ static int launch_lnl_reduce(pes_context* ctx, const BatchScratch& sc, int P, do
                        ctx->d_tile_jr, sc.pconst, sc.nodes, NNS, ctx->u0, ctx->du, ctx->modes, P, rows,
                        range_groups(r), n_grp, fine ? ranges[r].tile_begin : ranges[r].group_offset,
                        ctx->direct ? 0 : 1, items_buf, sc.work_counter + 2 * MAX_TILE_RANGES + r, off_words, dbits,
-                       panels ? bin_work.state + 1 + r : nullptr, want_items,
-                       grad ? chunk_rows<true>() : chunk_rows<false>(), n_blk);
+                       panels ? bin_work.state + 1 + r : nullptr, want_items, n_blk);
     HIP_TRY(hipGetLastError());
   }
   hipEvent_t e0 = nullptr, e1 = nullptr;
